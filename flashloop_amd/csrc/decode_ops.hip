@@ -12,11 +12,8 @@
 // Every rounding to bf16 happens where the torch modules round (Linear output, RMSNorm
 // output, each binary op of rotate-half RoPE, SiLU, the SwiGLU product, residual adds).
 //
-// GEMV work split: a workgroup of kGemvWaves waves owns kRows output rows and splits K
-// between its waves (each wave streams 64 contiguous 16-byte chunks of each row per
-// step); the waves reduce their partial dots in registers (DPP) and combine through LDS.
-// The grid has N / kRows workgroups (>= 512 for every matrix of the model), so every CU
-// has several row blocks of weights in flight.  Memory-bound: bytes = N * K * 2 + M * K.
+// The GEMVs are memory-bound (bytes = N * K * 2 + M * K * 2); gemv_mfma_kernel runs every K up
+// to 8192, gemv_kernel (VALU dots, one workgroup per 4 rows) the longer ones.
 #include "fl_common.h"
 
 namespace fl {
@@ -255,68 +252,6 @@ __global__ __launch_bounds__(kGemvThreads) void gemv_kernel(GemvArgs a) {
   gemv_finish<MT, EPI>(a, acc, red, mat, n0);
 }
 
-// The GEMV with every chunk a thread owns (S of them per row, K <= S * 2048) requested
-// at once as bounds-checked buffer loads: chunks past K and rows past M read as zero, so
-// no load sits under a branch (the compiler's wait after a branch join drains every
-// outstanding load).  Same accumulation order as gemv_kernel.
-template <int MT, int EPI, bool XF32, int S>
-__global__ __launch_bounds__(kGemvThreads) void gemv_flat_kernel(GemvArgs a) {
-  __shared__ float red[kGemvWaves][MT][kRows];
-  const uint16_t* rp[kRows];
-  int mat, n0;
-  block_rows<EPI>(a, blockIdx.x, rp, &mat, &n0);
-  constexpr int kStep = kGemvThreads;
-  constexpr uint32_t kXb = XF32 ? 4u : 2u;  // bytes per x element
-  const uint32_t q = threadIdx.x;
-  uint4 wv[S][kRows];
-#pragma unroll
-  for (int r = 0; r < kRows; ++r) {
-    const BufRes wr = buf_res(rp[r], static_cast<uint32_t>(a.K) * 2u);
-#pragma unroll
-    for (int s = 0; s < S; ++s) wv[s][r] = buf_load16(wr, 16u * (q + s * kStep));
-  }
-  uint4 xv[MT][S][XF32 ? 2 : 1];
-#pragma unroll
-  for (int m = 0; m < MT; ++m) {
-    const bool live = m < a.M;
-    const BufRes xr = buf_res(live ? static_cast<const char*>(a.x) + static_cast<int64_t>(m) * a.x_stride * kXb : nullptr,
-                              live ? static_cast<uint32_t>(a.K) * kXb : 0u);
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-      const uint32_t off = 8u * kXb * (q + s * kStep);
-      xv[m][s][0] = buf_load16(xr, off);
-      if (XF32) xv[m][s][XF32 ? 1 : 0] = buf_load16(xr, off + 16u);
-    }
-  }
-  float acc[MT][kRows];
-#pragma unroll
-  for (int m = 0; m < MT; ++m)
-#pragma unroll
-    for (int r = 0; r < kRows; ++r) acc[m][r] = 0.0f;
-#pragma unroll
-  for (int m = 0; m < MT; ++m)
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-      float x[8];
-      if (XF32) {
-        const uint4 u = xv[m][s][0], v = xv[m][s][XF32 ? 1 : 0];
-        const uint32_t w8[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = bf16_round(__uint_as_float(w8[e]));
-      } else {
-        unpack8(xv[m][s][0], x);
-      }
-#pragma unroll
-      for (int r = 0; r < kRows; ++r) {
-        float f[8];
-        unpack8(wv[s][r], f);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[m][r] = fmaf(x[e], f[e], acc[m][r]);
-      }
-    }
-  gemv_finish<MT, EPI>(a, acc, red, mat, n0);
-}
-
 // ---------------------------------------------------------------------------------
 // Residual / RMSNorm chain of one row (one workgroup per row).  Thread t owns the
 // 8-value chunks t, t + 256, ... of the row; every global load (x, r and the three
@@ -343,7 +278,8 @@ constexpr int kNormWaves = kNormThreads / kWave;
 
 // Block sums through two LDS buffers used in turn: reduction k writes buffer k & 1 and
 // every wave reads it before it reaches the barrier of reduction k + 1, so buffer k & 1 is
-// free again for reduction k + 2 -- one barrier per sum.
+// free again for reduction k + 2 -- one barrier per sum.  Waves past the first kNormWaves
+// of a larger workgroup take part in the barriers only.
 struct BlockSum {
   float (*red)[kNormWaves];
   int phase;
@@ -351,8 +287,8 @@ struct BlockSum {
     float* r = red[phase & 1];
     ++phase;
     v = wave_sum(v);
-    if ((threadIdx.x & 63) == 0) r[threadIdx.x >> 6] = v;
-    __syncthreads();
+    if ((threadIdx.x & 63) == 0 && threadIdx.x < kNormThreads) r[threadIdx.x >> 6] = v;
+    lds_barrier();  // (a global fence would wait for a caller's weight loads)
     float s = 0.0f;
 #pragma unroll
     for (int i = 0; i < kNormWaves; ++i) s += r[i];
@@ -469,64 +405,404 @@ __global__ __launch_bounds__(kNormThreads) void norm_chain_kernel(NormArgs a) {
   }
 }
 
-// GEMV whose input rows are the chain's output, computed in the prologue of every
-// workgroup (bit-identical to norm_chain_kernel: same chunk ownership, same reductions);
-// workgroup 0 writes h.  The weight chunks are requested before the chain so its loads
-// and reductions run under their latency.  K <= kChainMaxK (each thread's x chunks are the
-// chunks it normalises, so z stays in registers).
-constexpr int kChainSteps = 2;
-constexpr int kChainMaxK = kChainSteps * kGemvThreads * 8;
-static_assert(kGemvThreads == kNormThreads, "the chain prologue maps one GEMV thread to one chain thread");
+// ---------------------------------------------------------------------------------
+// The GEMV of a decode step on the matrix cores, with the chain of its input rows in the
+// prologue where there is one (bit-identical to norm_chain_kernel then this kernel: same
+// chunk ownership, same order of the sums).
+//
+// v_mfma_f32_16x16x32_bf16 takes 16 rows of W and 16 columns of x over 32 k.  A decode step
+// has 1 to 8 rows of x, so a tile is T rows of W by T rows of x (T = 8, or 4 for one row) and
+// the rest of the instruction's rows and columns holds further k of the same rows: row i and
+// column j are (row i % T, k-slice i / T) and (x row j % T, k-slice j / T).  The diagonal
+// T x T blocks of the product add up to the tile (the others mix slices and are not used), and
+// the lanes of one W row read 128 (T = 8) or 256 (T = 4) contiguous bytes per load.
+//
+// Bound by HBM and, for small matrices, by the launch's ramp: the VALU form it replaces cost
+// M * K fused multiply-adds per W row, M sequential chains per workgroup and one chain per 4
+// rows.  A unit of NT tiles (SwiGLU: gate and up rows; RoPE: rotary pairs) is one workgroup's
+// work, all its weights requested before its first product; its waves split K in steps of 512
+// and their partial tiles meet in LDS.  Eight rows take 8 waves, one wave per chain row; one
+// row takes 4 waves and 4-row tiles (twice the workgroups).  Measured, 2048 wide (q/k/v with
+// RoPE, o_proj, SwiGLU 5632, down, lm_head 49152), us before -> now: 8 rows 46.8 -> 11.3,
+// 12.1 -> 5.7, 75.2 -> 14.2, 15.6 -> 7.9, 287 -> 41 (4.9 TB/s); one row 9.2 -> 7.6, 4.8 -> 5.0,
+// 13.3 -> 11.4, 6.1 -> 6.7, 42.0 -> 36.5 (5.5 TB/s).  One row with 8 waves and 8-row tiles
+// took 9.1, 5.1, 11.9, 6.9 and 38.4.
+template <int MT>
+struct MmGeom {
+  static constexpr int kWaves = MT == 1 ? 4 : 8;
+  static constexpr int kThreads = kWaves * kWave;
+  static constexpr int kTile = MT == 1 ? 4 : 8;    // rows of W (and of x) per tile
+  static constexpr int kSlices = 16 / kTile;       // k-slices of 32 side by side in one MFMA
+  static constexpr int kWaveK = 32 * kSlices;      // k of one MFMA
+  static constexpr int kParts = kWaves * kSlices;  // partial tiles of a unit
+};
+constexpr int kMmStepK = 512;    // k of one step of all waves
+constexpr int kChainMaxK = 4096;
+constexpr int kMmMaxK = 8192;    // of the largest instantiation
 
-template <int MT, int EPI, int NC>
-__global__ __launch_bounds__(kGemvThreads) void gemv_chain_kernel(GemvArgs a, NormArgs c) {
-  __shared__ float red[kGemvWaves][MT][kRows];
-  __shared__ float nred[2][kNormWaves];
-  BlockSum bs{nred, 0};
-  const uint16_t* rp[kRows];
-  int mat, n0;
-  block_rows<EPI>(a, blockIdx.x, rp, &mat, &n0);
-  const int nq = a.K / 8;
-  constexpr int kStep = kGemvThreads;
-  const int q = threadIdx.x;
-  // row 0's chain inputs are requested before the weights: the wave's loads return in
-  // order, so the chain (two block reductions) then runs while the weights are in flight
-  ChainIn<NC> in0;
-  chain_load<NC>(c, 0, in0);
-  __builtin_amdgcn_sched_barrier(0);  // keep the issue order: chain inputs, then weights
-  uint4 wv[NC][kRows];  // weight chunks past K (buffer bounds) read as zero, no branch
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+
+// Two values rounded to bf16 and packed (v_cvt_pk_bf16_f32, nearest even, NaN kept NaN).
+__device__ __forceinline__ uint32_t bf16_pair(float lo, float hi) {
+  const f32x2_t f = {lo, hi};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2_t));
+}
+__device__ __forceinline__ uint4 bf16_pack8(const float* f) {
+  return make_uint4(bf16_pair(f[0], f[1]), bf16_pair(f[2], f[3]), bf16_pair(f[4], f[5]), bf16_pair(f[6], f[7]));
+}
+
+// Where a lane's tile rows of unit u lie: a buffer over the unit's rows and this lane's
+// byte offset in it, per tile.  Rows past the matrix repeat its last row (not stored).
+template <int NT>
+struct UnitRows {
+  BufRes res[NT];
+  uint32_t off[NT];
+};
+
+__device__ __forceinline__ BufRes rows_res(const uint16_t* w, int64_t row, int64_t rows, int K) {
+  const int64_t left = (rows - row) * K * 2;
+  return buf_res(w + row * K, static_cast<uint32_t>(left < 0x7FFFFFFF ? left : 0x7FFFFFFF));
+}
+
+template <int EPI, int MT>
+__host__ __device__ __forceinline__ int units_per_matrix(int n) {
+  constexpr int kTile = MmGeom<MT>::kTile;
+  return EPI == kEpiRope ? (n / 2 + kTile - 1) / kTile : (n + kTile - 1) / kTile;
+}
+
+// First k of this lane (its k-slice of its wave's MFMA).
+template <int MT>
+__device__ __forceinline__ int lane_k0() {
+  using G = MmGeom<MT>;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  return wave * G::kWaveK + ((lane & 15) / G::kTile) * 32 + (lane >> 4) * 8;
+}
+
+template <int EPI, int MT, int NT>
+__device__ __forceinline__ void unit_rows(const GemvArgs& a, int u, UnitRows<NT>& ur) {
+  constexpr int kTile = MmGeom<MT>::kTile;
+  const int i = threadIdx.x & (kTile - 1);
+  const uint32_t row_bytes = static_cast<uint32_t>(a.K) * 2u;
+  if (EPI == kEpiSwiGlu) {
+    const int n = kTile * u;
+    const uint32_t row = static_cast<uint32_t>(min(i, a.N - 1 - n));
 #pragma unroll
-  for (int r = 0; r < kRows; ++r) {
-    const BufRes wr = buf_res(rp[r], static_cast<uint32_t>(a.K) * 2u);
+    for (int t = 0; t < NT; ++t) {
+      ur.res[t] = rows_res(a.w[t], n, a.N, a.K);
+      ur.off[t] = row * row_bytes;
+    }
+  } else if (EPI == kEpiRope) {
+    const int per = units_per_matrix<EPI, MT>(a.N), half = a.head_dim / 2;
+    const int mat = u / per, p0 = (u - mat * per) * kTile;
+    const int p = min(p0 + i, a.N / 2 - 1);
+    const int n0 = (p0 / half) * a.head_dim + p0 % half;  // the unit's first row
+    const int n = (p / half) * a.head_dim + p % half;
+    const uint16_t* w = mat == 0 ? a.w[0] : (mat == 1 ? a.w[1] : a.w[2]);
 #pragma unroll
-    for (int s = 0; s < NC; ++s) wv[s][r] = buf_load16(wr, 16u * static_cast<uint32_t>(q + s * kStep));
-  }
-  float acc[MT][kRows];
+    for (int t = 0; t < NT; ++t) {
+      ur.res[t] = rows_res(w, n0, a.N, a.K);
+      ur.off[t] = static_cast<uint32_t>(n - n0 + t * half) * row_bytes;
+    }
+  } else {
+    const int n = NT * kTile * u;
 #pragma unroll
-  for (int m = 0; m < MT; ++m)
-#pragma unroll
-    for (int r = 0; r < kRows; ++r) acc[m][r] = 0.0f;
-#pragma unroll
-  for (int m = 0; m < MT; ++m) {
-    if (m < a.M) {
-      float z[NC][8];
-      if (m == 0)
-        chain_finish<NC>(c, 0, blockIdx.x == 0, in0, z, bs);
-      else
-        chain_row<NC>(c, static_cast<int64_t>(m) * c.stride, blockIdx.x == 0, z, bs);
-#pragma unroll
-      for (int s = 0; s < NC; ++s)
-        if (q + s * kStep < nq)
-#pragma unroll
-          for (int r = 0; r < kRows; ++r) {
-            float f[8];
-            unpack8(wv[s][r], f);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) acc[m][r] = fmaf(z[s][e], f[e], acc[m][r]);
-          }
+    for (int t = 0; t < NT; ++t) {
+      ur.res[t] = rows_res(a.w[0], n, a.N, a.K);
+      ur.off[t] = static_cast<uint32_t>(min(kTile * t + i, a.N - 1 - n)) * row_bytes;
     }
   }
-  gemv_finish<MT, EPI>(a, acc, red, mat, n0);
+}
+
+// This wave's k of the unit's tiles: step s covers kWaveK values from s * 512 + wave * kWaveK;
+// chunks past K lie outside the buffer and read as zero.
+template <int MT, int NT, int CS>
+__device__ __forceinline__ void load_unit(const UnitRows<NT>& ur, int K, uint4 (&w)[NT][CS]) {
+  const int k0 = lane_k0<MT>();
+#pragma unroll
+  for (int s = 0; s < CS; ++s) {
+    const int k = k0 + s * kMmStepK;
+    const uint32_t ko = k < K ? 2u * static_cast<uint32_t>(k) : 0x80000000u;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) w[t][s] = buf_load16(ur.res[t], ur.off[t] + ko);
+  }
+}
+
+// Output (m, i-th row of each tile) of unit u from the tiles' bf16-rounded dots v[t].
+template <int EPI, int MT, int NT>
+__device__ __forceinline__ void unit_store(const GemvArgs& a, int u, int m, int i, const float* v) {
+  constexpr int kTile = MmGeom<MT>::kTile;
+  if (EPI == kEpiSwiGlu) {
+    const int n = kTile * u + i;
+    if (n >= a.N) return;
+    const float g = v[0], up = v[NT - 1];
+    const float s = bf16_round(g / (1.0f + expf(-g)));  // F.silu on bf16 rounds, then the product
+    static_cast<uint16_t*>(a.y[0])[static_cast<int64_t>(m) * a.y_stride + n] = f32_to_bf16_rne(s * up);
+  } else if (EPI == kEpiRope) {  // rotate_half(x)[c] = -x[c + half], [c + half] = x[c]
+    const int per = units_per_matrix<EPI, MT>(a.N), half = a.head_dim / 2;
+    const int mat = u / per, p = (u - mat * per) * kTile + i;
+    if (p >= a.N / 2) return;
+    const int c = p % half;
+    const float lo = v[0], hi = v[NT - 1];
+    uint16_t* y = static_cast<uint16_t*>(mat == 0 ? a.y[0] : (mat == 1 ? a.y[1] : a.y[2])) +
+                  static_cast<int64_t>(m) * a.y_stride + (p / half) * a.head_dim + c;
+    if (mat == 2) {
+      y[0] = f32_to_bf16_rne(lo);
+      y[half] = f32_to_bf16_rne(hi);
+    } else {
+      const uint16_t* cs = a.cos + static_cast<int64_t>(m) * a.head_dim + c;
+      const uint16_t* sn = a.sin + static_cast<int64_t>(m) * a.head_dim + c;
+      y[0] = f32_to_bf16_rne(bf16_round(lo * bf16_to_f32(cs[0])) + bf16_round(-hi * bf16_to_f32(sn[0])));
+      y[half] = f32_to_bf16_rne(bf16_round(hi * bf16_to_f32(cs[half])) + bf16_round(lo * bf16_to_f32(sn[half])));
+    }
+  } else {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int n = (NT * u + t) * kTile + i;
+      if (n >= a.N) return;
+      const int64_t o = static_cast<int64_t>(m) * a.y_stride + n;
+      if (EPI == kEpiF32)
+        static_cast<float*>(a.y[0])[o] = v[t];
+      else if (EPI == kEpiAdd)
+        static_cast<uint16_t*>(a.y[0])[o] =
+            f32_to_bf16_rne(v[t] + bf16_to_f32(a.addend[static_cast<int64_t>(m) * a.addend_stride + n]));
+      else
+        static_cast<uint16_t*>(a.y[0])[o] = f32_to_bf16_rne(v[t]);
+    }
+  }
+}
+
+// One row's chain by one wave: lane l holds chunks l + 64 j, and the four partial sums of
+// a norm are those of norm_chain_kernel's four waves (thread 64 w + l: chunks 64 w + l and
+// 256 + 64 w + l), added in its order.
+template <int CH>
+struct WaveChainIn {
+  uint4 x[CH], r[CH], wa[CH], wb[CH];
+};
+
+template <int CH>
+__device__ __forceinline__ void wave_chain_load(const NormArgs& c, int64_t base, WaveChainIn<CH>& in) {
+  const uint32_t row = static_cast<uint32_t>(c.D) * 2u;
+  const BufRes r = buf_res(c.r + base, row);
+  const BufRes x = buf_res(c.x ? c.x + base : nullptr, c.x ? row : 0u);
+  const BufRes wa = buf_res(c.x ? c.wa : nullptr, c.x ? row : 0u);
+  const BufRes wb = buf_res(c.wb, c.wb ? row : 0u);
+  const uint32_t o = 16u * (threadIdx.x & 63u);
+#pragma unroll
+  for (int j = 0; j < CH; ++j) {
+    in.x[j] = buf_load16(x, o + 1024u * j);
+    in.r[j] = buf_load16(r, o + 1024u * j);
+    in.wa[j] = buf_load16(wa, o + 1024u * j);
+    in.wb[j] = buf_load16(wb, o + 1024u * j);
+  }
+}
+
+template <int CH>
+__device__ __forceinline__ void wave_rms(uint4 (&v)[CH], const uint4 (&w)[CH], int D, float eps) {
+  float ss[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int j = 0; j < CH; ++j) {
+    float f[8];
+    unpack8(v[j], f);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ss[j & 3] = fmaf(f[e], f[e], ss[j & 3]);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) ss[i] = wave_sum(ss[i]);
+  const float inv = rsqrtf((((ss[0] + ss[1]) + ss[2]) + ss[3]) / static_cast<float>(D) + eps);
+#pragma unroll
+  for (int j = 0; j < CH; ++j) {
+    float f[8], g[8];
+    unpack8(v[j], f);
+    unpack8(w[j], g);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = g[e] * (f[e] * inv);
+    v[j] = bf16_pack8(f);
+  }
+}
+
+// z (or h without n_b) of the row, as packed bf16, in in.r; h is written to h_out when asked
+template <int CH>
+__device__ __forceinline__ void wave_chain(const NormArgs& c, int64_t base, bool write_h, WaveChainIn<CH>& in) {
+  if (c.x != nullptr) {
+    wave_rms<CH>(in.x, in.wa, c.D, c.eps);
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+      float f[8], g[8];
+      unpack8(in.r[j], f);
+      unpack8(in.x[j], g);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) f[e] += g[e];
+      in.r[j] = bf16_pack8(f);
+    }
+  }
+  if (c.wf != nullptr) {  // the last chain of a loop only: loaded here, so that the others keep the registers
+    const BufRes res = buf_res(c.wf, static_cast<uint32_t>(c.D) * 2u);
+#pragma unroll
+    for (int j = 0; j < CH; ++j) in.x[j] = buf_load16(res, 16u * (threadIdx.x & 63u) + 1024u * j);
+    wave_rms<CH>(in.r, in.x, c.D, c.eps);
+  }
+  if (write_h && c.h_out != nullptr) {
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+      const int q = static_cast<int>(threadIdx.x & 63u) + 64 * j;
+      if (q < c.D / 8) reinterpret_cast<uint4*>(c.h_out + base)[q] = in.r[j];
+    }
+  }
+  if (c.wb != nullptr) wave_rms<CH>(in.r, in.wb, c.D, c.eps);
+}
+
+// This lane's x chunks (k as in load_unit) of row lane % 8, rounded to bf16 when x is f32;
+// zero past K (the weights there read as zero too) and in rows past M.
+template <int MT, int CS>
+__device__ __forceinline__ void load_x(const GemvArgs& a, bf16x8_t (&x)[CS]) {
+  const int k0 = lane_k0<MT>();
+  const int m = MT == 1 ? 0 : (threadIdx.x & 7);
+  const uint32_t es = a.x_f32 ? 4u : 2u;
+  const BufRes r = buf_res(a.x, (static_cast<uint32_t>(a.M - 1) * static_cast<uint32_t>(a.x_stride) + a.K) * es);
+  const uint32_t row = static_cast<uint32_t>(m) * static_cast<uint32_t>(a.x_stride) * es;
+  if (a.x_f32) {
+    uint4 lo[CS], hi[CS];
+#pragma unroll
+    for (int s = 0; s < CS; ++s) {
+      const int k = k0 + s * kMmStepK;
+      const uint32_t o = k < a.K && m < a.M ? row + 4u * static_cast<uint32_t>(k) : 0x80000000u;
+      lo[s] = buf_load16(r, o);
+      hi[s] = buf_load16(r, o + 16u);
+    }
+#pragma unroll
+    for (int s = 0; s < CS; ++s) {
+      const float f[8] = {__uint_as_float(lo[s].x), __uint_as_float(lo[s].y), __uint_as_float(lo[s].z),
+                          __uint_as_float(lo[s].w), __uint_as_float(hi[s].x), __uint_as_float(hi[s].y),
+                          __uint_as_float(hi[s].z), __uint_as_float(hi[s].w)};
+      x[s] = __builtin_bit_cast(bf16x8_t, bf16_pack8(f));
+    }
+  } else {
+#pragma unroll
+    for (int s = 0; s < CS; ++s) {
+      const int k = k0 + s * kMmStepK;
+      const uint32_t o = k < a.K && m < a.M ? row + 2u * static_cast<uint32_t>(k) : 0x80000000u;
+      x[s] = __builtin_bit_cast(bf16x8_t, buf_load16(r, o));
+    }
+  }
+}
+
+// KCAP: the largest K of the instantiation (a unit's weights are in registers).  MT: x rows
+// (1, or up to 8).  PP: grids of several units per workgroup, two units' weights in flight.
+template <int EPI, int MT, int KCAP, int NT, bool CHAIN, bool PP>
+__global__ __launch_bounds__(MmGeom<MT>::kThreads, 2) void gemv_mfma_kernel(GemvArgs a, NormArgs c, int units) {
+  using G = MmGeom<MT>;
+  constexpr int CS = KCAP / kMmStepK;  // steps of a wave over K
+  constexpr int kRow = KCAP + 8;       // x row in LDS, elements
+  __shared__ uint16_t xs[CHAIN ? MT * kRow : 8];
+  __shared__ float red[2][G::kParts][NT][MT][G::kTile];  // [unit parity][wave, k-slice][tile][x row][W row]
+  __shared__ float nred[2][kNormWaves];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+
+  uint4 w0[NT][CS], w1[PP ? NT : 1][PP ? CS : 1];
+  int u = blockIdx.x;
+  const auto load = [&](int unit, auto& w) __attribute__((always_inline)) {
+    UnitRows<NT> ur;
+    unit_rows<EPI, MT, NT>(a, min(unit, units - 1), ur);
+    load_unit<MT, NT, CS>(ur, a.K, w);
+  };
+  const auto load_first = [&]() __attribute__((always_inline)) {
+    load(u, w0);
+    if constexpr (PP) load(u + gridDim.x, w1);
+  };
+  bf16x8_t xr[CHAIN ? 1 : CS];
+  if constexpr (CHAIN && MT == 1) {
+    // one row: the workgroup holds it as norm_chain_kernel does
+    static_assert(G::kThreads == kNormThreads, "one GEMV thread per chain thread");
+    constexpr int NC = KCAP / (kNormThreads * 8);
+    ChainIn<NC> in;
+    float z[NC][8];
+    BlockSum bs{nred, 0};
+    chain_load<NC>(c, 0, in);
+    __builtin_amdgcn_sched_barrier(0);  // the chain's inputs return before the weights
+    load_first();
+    __builtin_amdgcn_sched_barrier(0);
+    chain_finish<NC>(c, 0, blockIdx.x == 0, in, z, bs);
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+      *reinterpret_cast<uint4*>(&xs[8 * (tid + i * kNormThreads)]) = bf16_pack8(z[i]);  // (zero past K)
+  } else if constexpr (CHAIN) {
+    constexpr int CH = KCAP / 512;
+    WaveChainIn<CH> in;  // wave w: row w (rows past M repeat the last: columns no output reads)
+    const int64_t base = static_cast<int64_t>(min(wave, a.M - 1)) * c.stride;
+    wave_chain_load<CH>(c, base, in);
+    __builtin_amdgcn_sched_barrier(0);
+    load_first();
+    __builtin_amdgcn_sched_barrier(0);
+    if (wave < a.M) {
+      wave_chain<CH>(c, base, blockIdx.x == 0, in);
+#pragma unroll
+      for (int j = 0; j < CH; ++j) *reinterpret_cast<uint4*>(&xs[wave * kRow + 8 * (lane + 64 * j)]) = in.r[j];
+    }
+  } else {
+    load_x<MT, CS>(a, xr);
+    load_first();
+  }
+  if constexpr (CHAIN) lds_barrier();
+
+  const uint16_t* xl = &xs[CHAIN ? (MT == 1 ? 0 : (lane & 7)) * kRow + lane_k0<MT>() : 0];
+  int par = 0;
+  const auto compute = [&](const auto& w, int unit) __attribute__((always_inline)) {
+    f32x4_t acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int s = 0; s < CS; ++s) {
+      bf16x8_t xv;
+      if constexpr (CHAIN)
+        xv = *reinterpret_cast<const bf16x8_t*>(xl + s * kMmStepK);
+      else
+        xv = xr[s];
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w[t][s]), xv, acc[t], 0, 0, 0);
+    }
+    // lane l holds rows 4 (l / 16) ..+3 of column l % 16: the diagonal blocks are kept
+    const int row = 4 * (lane >> 4), col = lane & 15;
+    if (row / G::kTile == col / G::kTile && col % G::kTile < MT)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        *reinterpret_cast<f32x4_t*>(&red[par][wave * G::kSlices + row / G::kTile][t][col % G::kTile][row % G::kTile]) = acc[t];
+    lds_barrier();
+    if (tid < MT * G::kTile) {
+      const int m = tid / G::kTile, i = tid % G::kTile;
+      if (m < a.M) {
+        float v[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          float sum = 0.0f;
+#pragma unroll
+          for (int p = 0; p < G::kParts; ++p) sum += red[par][p][t][m][i];
+          v[t] = bf16_round(sum);  // the Linear's bf16 output
+        }
+        unit_store<EPI, MT, NT>(a, unit, m, i, v);
+      }
+    }
+    par ^= 1;  // (a buffer is written again after the next unit's barrier)
+  };
+  const int step = gridDim.x;
+  while (true) {
+    compute(w0, u);
+    if constexpr (PP) {
+      if (u + step >= units) break;
+      load(u + 2 * step, w0);
+      compute(w1, u + step);
+      if (u + 2 * step >= units) break;
+      load(u + 3 * step, w1);
+      u += 2 * step;
+    } else {
+      u += step;
+      if (u >= units) break;
+      load(u, w0);
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------------
@@ -580,63 +856,69 @@ __global__ __launch_bounds__(kAppendThreads) void append_tail_kernel(AppendArgs 
   if (threadIdx.x == 0) a.tail_tokens[b] = pos + 1;
 }
 
-template <int MT, int EPI, bool XF32>
-void launch_gemv_x(const GemvArgs& a, int blocks, hipStream_t st) {
-  const int steps = (a.K + kGemvThreads * 8 - 1) / (kGemvThreads * 8);
-  const dim3 g(blocks), t(kGemvThreads);
-  switch (steps) {
-    case 1: hipLaunchKernelGGL((gemv_flat_kernel<MT, EPI, XF32, 1>), g, t, 0, st, a); break;
-    case 2: hipLaunchKernelGGL((gemv_flat_kernel<MT, EPI, XF32, 2>), g, t, 0, st, a); break;
-    case 3: hipLaunchKernelGGL((gemv_flat_kernel<MT, EPI, XF32, 3>), g, t, 0, st, a); break;
-    case 4: hipLaunchKernelGGL((gemv_flat_kernel<MT, EPI, XF32, 4>), g, t, 0, st, a); break;
-    default: hipLaunchKernelGGL((gemv_kernel<MT, EPI, XF32>), g, t, 0, st, a); break;  // K > 8192
+template <int EPI, int MT, int KCAP, int NT, bool CHAIN, bool PP>
+void launch_gemv_mfma(const GemvArgs& a, const NormArgs& c, int workgroups, hipStream_t st) {
+  const int per = units_per_matrix<EPI, MT>(a.N);
+  const int units = EPI == kEpiRope ? 3 * per : (EPI == kEpiSwiGlu ? per : (per + NT - 1) / NT);
+  int grid = units;
+  if (PP) {  // at most `workgroups`, each with the same number of units
+    const int rounds = (units + workgroups - 1) / workgroups;
+    grid = (units + rounds - 1) / rounds;
   }
+  hipLaunchKernelGGL((gemv_mfma_kernel<EPI, MT, KCAP, NT, CHAIN, PP>), dim3(grid), dim3(MmGeom<MT>::kThreads), 0, st, a, c, units);
 }
 
-template <int MT, int EPI>
-void launch_gemv_m(const GemvArgs& a, int blocks, hipStream_t st) {
-  if (MT > 2) {  // the flat form would hold MT x S x-chunks in registers
-    if (a.x_f32)
-      hipLaunchKernelGGL((gemv_kernel<MT, EPI, true>), dim3(blocks), dim3(kGemvThreads), 0, st, a);
+// Several units per workgroup (PP) where the prologue or the epilogue of one unit would not
+// hide behind the other workgroups of its CU.  Eight chained rows: the prologue is ~900 VALU
+// instructions per row, so one workgroup per CU runs it once (SwiGLU 5632 x 2048: 16.8 us with
+// a workgroup per unit, 14.1 with 235 of three units).  One row: only the many units of a
+// head-sized matrix gain (lm_head 49152 x 2048: 37.5 -> 36.3 us; SwiGLU lost, 11.4 -> 13.1).
+template <int EPI, int MT, bool CHAIN>
+void launch_gemv_k(const GemvArgs& a, const NormArgs& c, hipStream_t st) {
+  constexpr int kPair = EPI == kEpiSwiGlu || EPI == kEpiRope ? 2 : 1;
+  if (a.K <= 2048) {
+    if constexpr (CHAIN && MT == 8) {
+      return launch_gemv_mfma<EPI, MT, 2048, 2, CHAIN, true>(a, c, 256, st);
+    } else {
+      if (a.N >= 16384) return launch_gemv_mfma<EPI, MT, 2048, 2, CHAIN, true>(a, c, 1024, st);
+      launch_gemv_mfma<EPI, MT, 2048, kPair, CHAIN, false>(a, c, 0, st);
+    }
+  } else if (a.K <= 4096) {
+    launch_gemv_mfma<EPI, MT, 4096, kPair, CHAIN, false>(a, c, 0, st);
+  } else if constexpr (!CHAIN) {
+    if (a.K <= 6144)
+      launch_gemv_mfma<EPI, MT, 6144, kPair, false, false>(a, c, 0, st);
     else
-      hipLaunchKernelGGL((gemv_kernel<MT, EPI, false>), dim3(blocks), dim3(kGemvThreads), 0, st, a);
-  } else if (a.x_f32) {
-    launch_gemv_x<(MT > 2 ? 2 : MT), EPI, true>(a, blocks, st);
-  } else {
-    launch_gemv_x<(MT > 2 ? 2 : MT), EPI, false>(a, blocks, st);
+      launch_gemv_mfma<EPI, MT, kMmMaxK, kPair, false, false>(a, c, 0, st);
   }
 }
 
-template <int EPI>
-void launch_gemv(const GemvArgs& a, int blocks, hipStream_t st) {
+template <int EPI, bool XF32>
+void launch_gemv_long(const GemvArgs& a, hipStream_t st) {
+  const int blocks = EPI == kEpiSwiGlu ? a.N / 2 : (EPI == kEpiRope ? 3 * (a.N / kRows) : a.N / kRows);
+  const dim3 g(blocks), t(kGemvThreads);
   if (a.M <= 1)
-    launch_gemv_m<1, EPI>(a, blocks, st);
-  else if (a.M <= 2)
-    launch_gemv_m<2, EPI>(a, blocks, st);
-  else if (a.M <= 4)
-    launch_gemv_m<4, EPI>(a, blocks, st);
+    hipLaunchKernelGGL((gemv_kernel<1, EPI, XF32>), g, t, 0, st, a);
   else
-    launch_gemv_m<8, EPI>(a, blocks, st);
+    hipLaunchKernelGGL((gemv_kernel<8, EPI, XF32>), g, t, 0, st, a);
 }
 
-template <int EPI, int NC>
-void launch_gemv_chain_nc(const GemvArgs& a, const NormArgs& c, int blocks, hipStream_t st) {
-  if (a.M <= 1)
-    hipLaunchKernelGGL((gemv_chain_kernel<1, EPI, NC>), dim3(blocks), dim3(kGemvThreads), 0, st, a, c);
-  else if (a.M <= 2)
-    hipLaunchKernelGGL((gemv_chain_kernel<2, EPI, NC>), dim3(blocks), dim3(kGemvThreads), 0, st, a, c);
-  else if (a.M <= 4)
-    hipLaunchKernelGGL((gemv_chain_kernel<4, EPI, NC>), dim3(blocks), dim3(kGemvThreads), 0, st, a, c);
-  else
-    hipLaunchKernelGGL((gemv_chain_kernel<8, EPI, NC>), dim3(blocks), dim3(kGemvThreads), 0, st, a, c);
-}
-
-template <int EPI>
-void launch_gemv_chain(const GemvArgs& a, const NormArgs& c, int blocks, hipStream_t st) {
-  if (a.K <= kGemvThreads * 8)
-    launch_gemv_chain_nc<EPI, 1>(a, c, blocks, st);
-  else
-    launch_gemv_chain_nc<EPI, kChainSteps>(a, c, blocks, st);
+// K up to 8192 (a unit's weights in registers) runs on the matrix cores; longer rows, and
+// heads or x strides so wide that a unit's rows do not fit one buffer, on gemv_kernel.
+template <int EPI, bool CHAIN>
+void launch_gemv(const GemvArgs& a, const NormArgs& c, hipStream_t st) {
+  const bool wide = (EPI == kEpiRope && (static_cast<int64_t>(a.head_dim) + 16) * a.K * 2 > 0x7FFFFFFF) ||
+                    (a.M > 1 && a.x_stride > 0x7FFFFFFF / (4 * kMaxM));
+  if (CHAIN || (a.K <= kMmMaxK && !wide)) {
+    if (a.M <= 1)
+      launch_gemv_k<EPI, 1, CHAIN>(a, c, st);
+    else
+      launch_gemv_k<EPI, 8, CHAIN>(a, c, st);
+  } else if (a.x_f32) {
+    launch_gemv_long<EPI, true>(a, st);
+  } else {
+    launch_gemv_long<EPI, false>(a, st);
+  }
 }
 
 // Argument checks and GemvArgs shared by both GEMV entry points.
@@ -683,10 +965,6 @@ int32_t make_gemv_args(GemvArgs& a, const void* x, int32_t x_is_f32, int64_t x_s
   return FL_OK;
 }
 
-int gemv_blocks(int epilogue, int n) {
-  return epilogue == kEpiSwiGlu ? n / 2 : (epilogue == kEpiRope ? 3 * (n / kRows) : n / kRows);
-}
-
 }  // namespace
 }  // namespace fl
 
@@ -701,12 +979,13 @@ extern "C" int32_t fl_gemv_bf16(const void* x, int32_t x_is_f32, int64_t x_strid
                                     addend_stride, rope_cos, rope_sin, head_dim, "fl_gemv_bf16");
   if (rc != FL_OK) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
+  const NormArgs none{};
   switch (epilogue) {
-    case kEpiPlain: launch_gemv<kEpiPlain>(a, n / kRows, st); break;
-    case kEpiF32: launch_gemv<kEpiF32>(a, n / kRows, st); break;
-    case kEpiAdd: launch_gemv<kEpiAdd>(a, n / kRows, st); break;
-    case kEpiSwiGlu: launch_gemv<kEpiSwiGlu>(a, n / 2, st); break;
-    default: launch_gemv<kEpiRope>(a, 3 * (n / kRows), st); break;
+    case kEpiPlain: launch_gemv<kEpiPlain, false>(a, none, st); break;
+    case kEpiF32: launch_gemv<kEpiF32, false>(a, none, st); break;
+    case kEpiAdd: launch_gemv<kEpiAdd, false>(a, none, st); break;
+    case kEpiSwiGlu: launch_gemv<kEpiSwiGlu, false>(a, none, st); break;
+    default: launch_gemv<kEpiRope, false>(a, none, st); break;
   }
   FL_LAUNCH_CHECK("fl_gemv_bf16");
   return FL_OK;
@@ -734,13 +1013,12 @@ extern "C" int32_t fl_gemv_bf16_chain(int32_t m, int32_t k, float eps, const uin
   if (rc != FL_OK) return rc;
   const NormArgs c{k, eps, x, r, w_a, w_f, w_b, h_out, nullptr, stride};
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const int blocks = gemv_blocks(epilogue, n);
   switch (epilogue) {
-    case kEpiPlain: launch_gemv_chain<kEpiPlain>(a, c, blocks, st); break;
-    case kEpiF32: launch_gemv_chain<kEpiF32>(a, c, blocks, st); break;
-    case kEpiAdd: launch_gemv_chain<kEpiAdd>(a, c, blocks, st); break;
-    case kEpiSwiGlu: launch_gemv_chain<kEpiSwiGlu>(a, c, blocks, st); break;
-    default: launch_gemv_chain<kEpiRope>(a, c, blocks, st); break;
+    case kEpiPlain: launch_gemv<kEpiPlain, true>(a, c, st); break;
+    case kEpiF32: launch_gemv<kEpiF32, true>(a, c, st); break;
+    case kEpiAdd: launch_gemv<kEpiAdd, true>(a, c, st); break;
+    case kEpiSwiGlu: launch_gemv<kEpiSwiGlu, true>(a, c, st); break;
+    default: launch_gemv<kEpiRope, true>(a, c, st); break;
   }
   FL_LAUNCH_CHECK("fl_gemv_bf16_chain");
   return FL_OK;

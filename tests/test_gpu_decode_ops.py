@@ -177,3 +177,55 @@ def test_chained_step_equals_unchained_step():
         a = a_eng.decode(ids[:, i:i + 1]).logits
         b = b_eng.decode(ids[:, i:i + 1]).logits
         assert torch.equal(a, b), f"step {i}: max diff {(a - b).abs().max().item()}"
+
+
+def _dots(x, w):
+    """The Linear's output in float64 (rounded to bf16 once) and the bound of an fp32 sum of k
+    products: k * 2^-24 of the sum of their sizes."""
+    d = (x.double() @ w.double().t()).float().bfloat16().double()
+    return d, (x.double().abs() @ w.double().abs().t()) * x.shape[-1] * 2.0 ** -24
+
+
+def _near(got, want, slack, what, ulps=1.0):
+    """Within the bound of the sums plus ``ulps`` bf16 roundings (2^-8 relative each)."""
+    err = (got.double() - want).abs() - (slack + ulps * 2.0 ** -8 * want.abs() + 1e-30)
+    assert bool((err <= 0).all()), f"{what}: {err.max().item():.3e} beyond the bound"
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 4, 8), (1, 516, 200), (2, 12, 520), (5, 516, 2056), (8, 20, 2048), (8, 16388, 1024),
+                                   (1, 16388, 2040), (3, 36, 4104), (8, 260, 6152), (1, 260, 8192), (4, 8, 8200)])
+def test_gemv_at_tile_and_step_edges(m, n, k):
+    """Rows, N and K that end inside a tile, a 512-wide step or an instantiation."""
+    print(f"case: gemv edges m={m} n={n} k={k}", flush=True)
+    x, x32, add = _x(m, k, 60), _x(m, k, 61, torch.float32), _x(m, n, 62)
+    gate, up = _w(n, k, 63), _w(n, k, 64)
+    d, s = _dots(x, gate)
+    _near(kernels.gemv(x, [gate]), d, s, "plain")
+    _near(kernels.gemv(x, [gate], epilogue=kernels.EPI_F32), d, s, "f32")
+    df, sf = _dots(x32.bfloat16(), gate)
+    got = kernels.gemv(x32, [gate], epilogue=kernels.EPI_ADD, addend=add)
+    _near(got, df + add.double(), sf + 2.0 ** -8 * df.abs(), "add")
+    # |silu'| < 1.1: an error of the gate carries over, scaled by the up value
+    du, su = _dots(x, up)
+    silu = F.silu(d)
+    slack = 1.1 * (s + 2.0 ** -8 * d.abs()) * du.abs() + silu.abs() * (su + 2.0 ** -8 * du.abs())
+    _near(kernels.gemv(x, [gate, up], epilogue=kernels.EPI_SWIGLU), silu * du, slack, "swiglu", ulps=3.0)
+
+
+@pytest.mark.parametrize("m,heads,hd,k", [(1, 3, 24, 200), (8, 1, 8, 2048), (5, 3, 40, 4104), (8, 4, 128, 2056), (1, 2, 128, 8192)])
+def test_gemv_rope_at_head_edges(m, heads, hd, k):
+    """Rotary pairs that straddle heads inside a tile, and heads smaller than one."""
+    print(f"case: gemv rope edges m={m} heads={heads} hd={hd} k={k}", flush=True)
+    n = heads * hd
+    x, ws = _x(m, k, 70), [_w(n, k, 71 + i) for i in range(3)]
+    ang = torch.rand(m, hd // 2, device=DEV, generator=torch.Generator(device=DEV).manual_seed(74)) * 6.28
+    cos, sin = (torch.cat((f, f), dim=-1).bfloat16() for f in (ang.cos(), ang.sin()))
+    q, key, v = kernels.gemv(x, ws, epilogue=kernels.EPI_ROPE, rope=(cos, sin), head_dim=hd)
+    _near(v, *_dots(x, ws[2]), "v")
+    for got, w in ((q, ws[0]), (key, ws[1])):
+        d, s = (t.view(m, heads, hd) for t in _dots(x, w))
+        rot = torch.cat((-d[..., hd // 2:], d[..., :hd // 2]), dim=-1)
+        want = d * cos.double()[:, None] + rot * sin.double()[:, None]
+        # the dots' own roundings and each product's (2^-8 of its size, twice)
+        slack = s + s.roll(hd // 2, dims=-1) + 2.0 ** -7 * (d.abs() + rot.abs())
+        _near(got.view(m, heads, hd), want, slack, "rope")
