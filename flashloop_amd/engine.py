@@ -12,7 +12,9 @@ on this build's HIP kernels:
   selection (``fl_decode_topk``), loops 3-4 cached-mass sparse attention
   (``fl_decode_attn_sparse_delta[_fused]``).
 
-Model GEMMs, norms and SDPA of the dense prefill loops are torch (hipBLASLt).
+The prefill's contractions with the weights are library GEMMs (hipBLASLt); its attention
+(``fl_prefill_attention``), rotary embedding and K/V placement (``fl_rope_store``), norms and
+residuals (``fl_norm_chain``) and SwiGLU (``fl_swiglu``) are HIP kernels.
 """
 
 from __future__ import annotations
@@ -29,7 +31,7 @@ import torch.nn.functional as F
 from . import kernels
 from .cache import CrossLoopKVCache, CrossLoopKVLayer
 from .config import FlashLoopConfig, validate_ouro_model
-from .model import OuroConfig, OuroForCausalLM, apply_rope
+from .model import MLP, Attention, OuroConfig, OuroForCausalLM, RMSNorm, apply_rope
 
 
 @dataclass(frozen=True)
@@ -259,8 +261,88 @@ class FlashLoopEngine:
         v = attn.v_proj(x).view(bsz, rows, -1, attn.head_dim).transpose(1, 2)
         return q, k, v
 
+    def _prefill_weights(self, hidden: torch.Tensor):
+        """Per-layer weights of the HIP prefill path and its norm epsilon, or None when a module
+        is not a plain bf16 ``nn.Linear`` / ``RMSNorm`` on the device (a wrapped or hooked
+        module keeps the module path, which calls it)."""
+        def plain(m, kind) -> bool:
+            w = m.weight
+            return (type(m) is kind and not m._forward_hooks and not m._forward_pre_hooks
+                    and getattr(m, "bias", None) is None and w.dtype == torch.bfloat16 and w.is_cuda and w.is_contiguous())
+
+        d = hidden.shape[-1]
+        if hidden.dtype != torch.bfloat16 or d % 8 or d > 8192:
+            return None
+        eps = {self.backbone.norm.eps} if plain(self.backbone.norm, RMSNorm) else set()
+        layers = []
+        for layer in self.layers:
+            a, m = layer.self_attn, layer.mlp
+            lin = (a.q_proj, a.k_proj, a.v_proj, a.o_proj, m.gate_proj, m.up_proj, m.down_proj)
+            norms = (layer.input_layernorm, layer.input_layernorm_2, layer.post_attention_layernorm,
+                     layer.post_attention_layernorm_2)
+            if (type(a) is not Attention or type(m) is not MLP or m._forward_hooks or m._forward_pre_hooks
+                    or m.gate_proj.weight.shape[0] % 8
+                    or not all(plain(x, torch.nn.Linear) for x in lin) or not all(plain(x, RMSNorm) for x in norms)):
+                return None
+            eps.update(x.eps for x in norms)
+            layers.append(tuple(x.weight for x in (*lin, *norms)))
+        return (layers, float(eps.pop())) if len(eps) == 1 else None
+
+    def _layer_rows(self, weights, hid, z, rope, kv, positions, eps, w_next, w_final):
+        """One prefill layer over rows ``hid`` [n, hidden] whose input norm is ``z``: K/V rows into
+        ``kv`` ([H, T, 128] each, at ``positions`` or 0..n-1), attention up to each row's own
+        position, MLP.  Returns (rows after the layer, and ``w_final`` when given; their next
+        input norm, by ``w_next``)."""
+        wq, wk, wv, wo, gate, up, down, _, ln2, ln3, ln4 = weights
+        q, k, v = F.linear(z, wq), F.linear(z, wk), F.linear(z, wv)
+        kernels.rope_store(q, k, v, rope, kv[0], kv[1], positions)
+        heads = kv[0].shape[0]
+        o = kernels.prefill_attention(q.view(q.shape[0], heads, -1).transpose(0, 1), kv[0], kv[1],
+                                      self.layers[0].self_attn.scaling, positions)
+        hid, z = kernels.norm_chain(hid, x=F.linear(o, wo), w_a=ln2, w_b=ln3, eps=eps)
+        y = F.linear(kernels.swiglu(F.linear(z, gate), F.linear(z, up)), down)
+        return kernels.norm_chain(hid, x=y, w_a=ln4, w_f=w_final, w_b=w_next, eps=eps)
+
+    def _rows_loop(self, weights, rows, rope, kv, positions):
+        """Every layer over ``rows`` [n, hidden], then the final norm."""
+        layers, eps = weights
+        hid, (_, z) = rows, kernels.norm_chain(rows, w_b=layers[0][7], eps=eps, want_h=False)
+        for li, w in enumerate(layers):
+            last = li == len(layers) - 1
+            hid, z = self._layer_rows(w, hid, z, rope, kv[li], positions, eps, None if last else layers[li + 1][7],
+                                      self.backbone.norm.weight if last else None)
+        return hid
+
     def _dense_loop(self, hidden: torch.Tensor, cos, sin):
-        """``dense_prefill_loop`` (flashloop/prefill.py:275-304): every row, causal SDPA."""
+        """``dense_prefill_loop`` (flashloop/prefill.py:275-304): every row, causal attention."""
+        weights = self._prefill_weights(hidden)
+        if weights is None:
+            return self._dense_loop_modules(hidden, cos, sin)
+        _, t, d = hidden.shape
+        a = self.layers[0].self_attn
+        shape = (2, len(self.layers), 1, a.num_heads, t, a.head_dim)
+        keys, values = torch.empty(shape, dtype=hidden.dtype, device=hidden.device).unbind(0)
+        h = self._rows_loop(weights, hidden.reshape(t, d), (cos[0], sin[0]),
+                            [(k[0], v[0]) for k, v in zip(keys, values)], None)
+        return h.view(1, t, d), list(keys), list(values)
+
+    def _sparse_loop(self, hidden: torch.Tensor, positions: torch.Tensor, prev_keys, prev_values, cos, sin):
+        """``sparse_prefill_loop`` (flashloop/prefill.py:122-272): only the active rows are
+        recomputed; their K/V replace the previous loop's rows of a composite cache."""
+        weights = self._prefill_weights(hidden)
+        if weights is None:
+            return self._sparse_loop_modules(hidden, positions, prev_keys, prev_values, cos, sin)
+        keys = [k.clone() for k in prev_keys]
+        values = [v.clone() for v in prev_values]
+        active, _ = kernels.gather_rows(hidden, positions, dim=1)
+        rows = self._rows_loop(weights, active[0], (cos[0], sin[0]), [(k[0], v[0]) for k, v in zip(keys, values)],
+                               positions)
+        h = hidden.clone()
+        kernels.scatter_rows_(h, positions, rows[None], dim=1)
+        return h, keys, values
+
+    def _dense_loop_modules(self, hidden: torch.Tensor, cos, sin):
+        """``_dense_loop`` on the torch modules and SDPA."""
         t = hidden.shape[1]
         keys, values = [], []
         h = hidden
@@ -276,9 +358,8 @@ class FlashLoopEngine:
             values.append(v.contiguous())
         return self.backbone.norm(h), keys, values
 
-    def _sparse_loop(self, hidden: torch.Tensor, positions: torch.Tensor, prev_keys, prev_values, cos, sin):
-        """``sparse_prefill_loop`` (flashloop/prefill.py:122-272): only the active rows are
-        recomputed; their K/V replace the previous loop's rows of a composite cache."""
+    def _sparse_loop_modules(self, hidden: torch.Tensor, positions: torch.Tensor, prev_keys, prev_values, cos, sin):
+        """``_sparse_loop`` on the torch modules and SDPA."""
         t = hidden.shape[1]
         n = positions.numel()
         h = hidden.clone()

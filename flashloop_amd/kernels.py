@@ -501,3 +501,70 @@ def append_tail(view, keys, values, tail_active, tail_tokens: torch.Tensor) -> N
         C.cast(ptr_array([t.data_ptr() for t in tail_active]), _lib._PP), tail_tokens.data_ptr(), _stream(),
     )
     check(rc, "fl_append_tail")
+
+
+# ---------------------------------------------------------------------------- prefill ops
+def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scaling: float,
+                      positions: torch.Tensor | None = None) -> torch.Tensor:
+    """Causal attention of one sequence (``fl_prefill_attention``): ``q`` [H, n, 128], ``k`` /
+    ``v`` [H, T, 128] bf16 (any head and row strides that are multiples of 8 elements).  Query i
+    attends to the keys up to ``positions[i]`` (i32 [n]), or up to i without positions.
+    Returns [n, H * 128] bf16, the rows that o_proj takes."""
+    h, n, c = q.shape
+    t = k.shape[1]
+    if c != HEAD_DIM or tuple(k.shape) != (h, t, c) or k.shape != v.shape:
+        raise ValueError("q must be [H, n, 128] and k, v [H, T, 128]")
+    for x, name in ((q, "q"), (k, "k"), (v, "v")):
+        if not x.is_cuda:
+            raise RuntimeError(f"{name} must be a device tensor")
+        if x.dtype != torch.bfloat16 or x.stride(2) != 1:
+            raise ValueError(f"{name} must be bf16 with contiguous channels")
+    if positions is not None:
+        _require(positions, torch.int32, "positions")
+        if positions.numel() != n:
+            raise ValueError("positions needs one entry per query")
+    out = torch.empty(n, h * c, dtype=torch.bfloat16, device=q.device)
+    lib = load()
+    ws_bytes = lib.fl_prefill_attention_workspace(h, n, t)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
+    rc = lib.fl_prefill_attention(
+        q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0), k.stride(1), v.data_ptr(), v.stride(0),
+        v.stride(1), out.data_ptr(), c, h * c, h, n, t, _p(positions), float(scaling),
+        _p(ws), ws_bytes, _stream())
+    check(rc, "fl_prefill_attention")
+    return out
+
+
+def rope_store(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, rope: tuple[torch.Tensor, torch.Tensor],
+               k_dst: torch.Tensor, v_dst: torch.Tensor, positions: torch.Tensor | None = None) -> None:
+    """Rotary embedding of the projected rows ``q``, ``k`` [n, H*128] (``fl_rope_store``): q in
+    place, k and the plain v into rows ``positions`` (or 0..n-1) of ``k_dst`` / ``v_dst``
+    [H, T, 128].  ``rope``: cos and sin [T, 128] bf16 by position."""
+    h, t, c = k_dst.shape
+    n = q.shape[0]
+    for x, name in ((q, "q"), (k, "k"), (v, "v"), (k_dst, "k_dst"), (v_dst, "v_dst"), (rope[0], "rope cos"),
+                    (rope[1], "rope sin")):
+        _require(x, torch.bfloat16, name)
+    if c != HEAD_DIM or k_dst.shape != v_dst.shape or any(tuple(x.shape) != (n, h * c) for x in (q, k, v)):
+        raise ValueError("q, k and v must be [n, H*128] and the destinations [H, T, 128]")
+    if any(tuple(x.shape) != (t, c) for x in rope):
+        raise ValueError("rope tables must be [T, 128]")
+    if positions is not None:
+        _require(positions, torch.int32, "positions")
+        if positions.numel() != n:
+            raise ValueError("positions needs one entry per row")
+    rc = load().fl_rope_store(q.data_ptr(), k.data_ptr(), v.data_ptr(), h * c, q.data_ptr(), k_dst.data_ptr(),
+                              v_dst.data_ptr(), t * c, rope[0].data_ptr(), rope[1].data_ptr(), _p(positions), n, h, t,
+                              _stream())
+    check(rc, "fl_rope_store")
+
+
+def swiglu(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
+    """``F.silu(gate) * up`` of bf16 rows (``fl_swiglu``)."""
+    _require(gate, torch.bfloat16, "gate")
+    _require(up, torch.bfloat16, "up")
+    if gate.shape != up.shape:
+        raise ValueError("gate and up shapes differ")
+    out = torch.empty_like(gate)
+    check(load().fl_swiglu(gate.data_ptr(), up.data_ptr(), out.data_ptr(), gate.numel(), _stream()), "fl_swiglu")
+    return out

@@ -420,6 +420,40 @@ int32_t fl_gemv_bf16_chain(int32_t m, int32_t k, float eps, const uint16_t* x, c
                            int64_t addend_stride, const uint16_t* rope_cos, const uint16_t* rope_sin,
                            int32_t head_dim, void* stream);
 
+/*
+ * Prefill ops -- one sequence's prompt rows (flashloop/prefill.py:122-304).
+ *
+ * fl_prefill_attention: out[i, h, :] = sum_j softmax_j(scaling * q[i, h] . k[h, j]) v[h, j]
+ * over the keys j <= positions[i] (j <= i when positions is NULL) -- the causal SDPA of a dense
+ * loop, or the masked SDPA of a token-sparse loop's active rows.  bf16 tensors of 128
+ * channels; element (head h, row r) of a tensor starts h * head_stride + r * row_stride
+ * elements from its pointer (16-byte aligned, strides multiples of 8).  Scores, softmax
+ * and sums are fp32; probabilities are rounded to bf16 for the second product.  positions:
+ * i32 [queries] in device memory, each in [0, keys).  With a workspace (16-byte aligned, of
+ * fl_prefill_attention_workspace bytes; nullable) calls of few query blocks divide each
+ * block's keys over several workgroups and merge; a smaller one divides them less.
+ */
+size_t fl_prefill_attention_workspace(int32_t heads, int32_t queries, int32_t keys);
+int32_t fl_prefill_attention(const uint16_t* q, int64_t q_head_stride, int64_t q_row_stride,
+                             const uint16_t* k, int64_t k_head_stride, int64_t k_row_stride,
+                             const uint16_t* v, int64_t v_head_stride, int64_t v_row_stride,
+                             uint16_t* out, int64_t out_head_stride, int64_t out_row_stride,
+                             int32_t heads, int32_t queries, int32_t keys, const int32_t* positions,
+                             float scaling, void* workspace, size_t workspace_bytes, void* stream);
+/*
+ * fl_rope_store: rotary embedding (rotate-half, each binary op rounded to bf16) of n rows of
+ * q and k [n, heads * 128] (row stride `row_stride`) with the bf16 tables rope_cos/rope_sin
+ * [rows, 128]; q to q_out (same strides; may be q), k and the plain v to row positions[i] (i
+ * when positions is NULL) of k_dst / v_dst [heads, rows, 128] (head stride dst_head_stride).
+ * A position outside [0, rows) is skipped.
+ * fl_swiglu: out = bf16(bf16(silu(gate)) * up) over `count` (multiple of 8) bf16 values.
+ */
+int32_t fl_rope_store(const uint16_t* q, const uint16_t* k, const uint16_t* v, int64_t row_stride,
+                      uint16_t* q_out, uint16_t* k_dst, uint16_t* v_dst, int64_t dst_head_stride,
+                      const uint16_t* rope_cos, const uint16_t* rope_sin, const int32_t* positions,
+                      int32_t n, int32_t heads, int32_t rows, void* stream);
+int32_t fl_swiglu(const uint16_t* gate, const uint16_t* up, uint16_t* out, int64_t count, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,101 @@
+"""Prefill row ops (fl_prefill_attention, fl_rope_store, fl_swiglu) against plain torch."""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+
+from flashloop_amd import _lib, kernels  # noqa: E402
+from flashloop_amd.model import apply_rope  # noqa: E402
+
+DEV = "cuda"
+
+
+def _r(gen, *shape):
+    return torch.randn(*shape, generator=gen, device=DEV).to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("h,n,t", [(1, 1, 1), (2, 5, 5), (3, 64, 64), (2, 65, 65), (1, 129, 129), (2, 1000, 1000),  # dense
+                                   (2, 1, 70), (3, 128, 130), (2, 200, 1500), (16, 820, 4100)])  # active rows
+def test_prefill_attention(h, n, t):
+    """Query blocks, key tiles and key ranges that end early; with positions the rows of a
+    token-sparse loop, in order and shuffled.  Bound: every probability is rounded to bf16
+    (2^-9 relative) and so is the sum that divides (the same rounded values), the output
+    once more; the fp32 sums add far less."""
+    print(f"case: prefill attention h={h} n={n} t={t}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(80)
+    q = _r(g, n, h, 128).transpose(0, 1)  # the projections' row-major layout
+    k, v = _r(g, h, t, 128), _r(g, h, t, 128)
+    pos = None if n == t else torch.randperm(t, generator=g, device=DEV)[:n].sort().values.int()
+    if pos is not None:
+        pos[-1] = t - 1
+    for p in ([pos] if pos is None else [pos, pos.flip(0).contiguous()]):
+        at = torch.arange(n, device=DEV) if p is None else p.long()
+        s = torch.bmm(q.double(), k.double().transpose(1, 2).contiguous()) * 128 ** -0.5
+        w = s.masked_fill(torch.arange(t, device=DEV)[None, None] > at[None, :, None], -torch.inf).softmax(-1)
+        want = torch.bmm(w, v.double()).transpose(0, 1).reshape(n, h * 128)
+        size = torch.bmm(w, v.double().abs()).transpose(0, 1).reshape(n, h * 128)
+        got = kernels.prefill_attention(q, k, v, 128 ** -0.5, p)
+        err = (got.double() - want).abs() - (2.0 ** -8 * size + 2.0 ** -8 * want.abs() + 1e-6)
+        assert bool((err <= 0).all()), f"{err.max().item():.3e} beyond the bound"
+
+
+@pytest.mark.parametrize("ranges", [0, 1, 2, 5])
+def test_prefill_attention_with_less_workspace(ranges):
+    """A workspace of fewer key ranges than asked for (or none) divides the keys less."""
+    print(f"case: prefill attention ranges={ranges}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(81)
+    h, n, t = 2, 150, 4000
+    q, k, v = _r(g, h, n, 128), _r(g, h, t, 128), _r(g, h, t, 128)
+    pos = torch.randperm(t, generator=g, device=DEV)[:n].sort().values.int()
+    lib = _lib.load()
+    one = n * h * 130 * 4
+    assert lib.fl_prefill_attention_workspace(h, n, t) >= 6 * one
+    ws = torch.empty(max(1, ranges * one), dtype=torch.uint8, device=DEV)
+    guard = torch.full((64,), 7, dtype=torch.uint8, device=DEV)
+    out = torch.empty(n, h * 128, dtype=torch.bfloat16, device=DEV)
+    _lib.check(lib.fl_prefill_attention(
+        q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0), k.stride(1), v.data_ptr(), v.stride(0),
+        v.stride(1), out.data_ptr(), 128, h * 128, h, n, t, pos.data_ptr(), 128 ** -0.5, ws.data_ptr(), ranges * one,
+        torch.cuda.current_stream().cuda_stream), "fl_prefill_attention")
+    want = kernels.prefill_attention(q, k, v, 128 ** -0.5, pos).double()
+    # a range's probabilities are rounded to bf16 against its own maximum (another power of
+    # two times another fraction), so each side has test_prefill_attention's bound
+    s = torch.bmm(q.double(), k.double().transpose(1, 2).contiguous()) * 128 ** -0.5
+    w = s.masked_fill(torch.arange(t, device=DEV)[None, None] > pos.long()[None, :, None], -torch.inf).softmax(-1)
+    size = torch.bmm(w, v.double().abs()).transpose(0, 1).reshape(n, h * 128)
+    assert bool(((out.double() - want).abs() <= 2 * (2.0 ** -8 * size + 2.0 ** -8 * want.abs() + 1e-6)).all())
+    assert bool((guard == 7).all())
+
+
+@pytest.mark.parametrize("n,t", [(1, 1), (33, 33), (70, 400)])
+def test_rope_store_equals_the_modules(n, t):
+    print(f"case: rope store n={n} t={t}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(82)
+    h = 3
+    rows = [_r(g, n, h * 128) for _ in range(3)]
+    ang = torch.rand(t, 64, generator=g, device=DEV) * 6.28
+    cos, sin = (torch.cat((f, f), dim=-1).bfloat16() for f in (ang.cos(), ang.sin()))
+    pos = None if n == t else torch.randperm(t, generator=g, device=DEV)[:n].sort().values.int()
+    at = torch.arange(t, device=DEV) if pos is None else pos.long()
+    want = [x.view(n, h, 128).transpose(0, 1) for x in rows]
+    wq, wk = apply_rope(want[0][None], want[1][None], cos[at][None], sin[at][None])
+    base = _r(g, 2, h, t, 128)
+    kd, vd = base.clone().unbind(0)
+    q = rows[0].clone()
+    kernels.rope_store(q, rows[1], rows[2], (cos, sin), kd, vd, pos)
+    assert torch.equal(q.view(n, h, 128).transpose(0, 1), wq[0])
+    assert torch.equal(kd, base[0].index_copy(1, at, wk[0]))
+    assert torch.equal(vd, base[1].index_copy(1, at, want[2]))
+
+
+@pytest.mark.parametrize("n,d", [(1, 8), (3, 40), (257, 5632)])
+def test_swiglu_rows(n, d):
+    print(f"case: swiglu n={n} d={d}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(83)
+    gate, up = _r(g, n, d) * 4, _r(g, n, d)
+    want = F.silu(gate.double()) * up.double()
+    got = kernels.swiglu(gate, up).double()
+    # two bf16 roundings
+    assert bool(((got - want).abs() <= 2.0 ** -7 * want.abs() + 1e-30).all())
