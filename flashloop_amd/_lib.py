@@ -63,6 +63,10 @@ SIGNATURES = {
     "fl_last_error": (C.c_char_p, []),
     "fl_abi_version": (_I32, []),
     "fl_pack_kv_groups": (_I32, [_VIEW, _I32, _PP, _PP, _I64, _I32, _PP, _I64, _P, _I32, _PP, _PP, _P]),
+    "fl_count_active_rows": (_I32, [_PP, _I64, _I32, _I32, _P, _P, _P]),
+    "fl_cache_prepare": (_I32, [_VIEW, _PP, _PP, _I64, _PP, _I64, _PP, _P, _P, _P, _P, _P, _P, _P, _P]),
+    "fl_roll_begin": (_I32, [_VIEW, _P, _P, _P, _PP, _P, _P]),
+    "fl_roll_end": (_I32, [_VIEW, _P, _P, _P, _PP, _P, _P]),
     "fl_decode_attn_dense_workspace": (_SZ, [_VIEW]),
     "fl_decode_attn_dense": (_I32, [_VIEW, _I32, _P, _P, _P, _F32, _P, _P, _I64, _P, _SZ, _P]),
     "fl_decode_attn_dense_noalloc_max_bytes": (_SZ, []),

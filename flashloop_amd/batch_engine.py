@@ -127,6 +127,7 @@ class FlashLoopBatchEngine:
             mask4[b, :n] = r.mask4[0]
         extra = self.config.decode_capacity if decode_capacity is None else int(decode_capacity)
         cache = CrossLoopKVCache(num_layers=nl)
+        late = CrossLoopKVLayer.count_late_rows(mask3, mask4, lengths)
         for li in range(nl):
             keys, values = [], []
             for loop in range(4):
@@ -139,7 +140,7 @@ class FlashLoopBatchEngine:
                 keys.append(kb)
                 values.append(vb)
             cache.set_layer(li, CrossLoopKVLayer.from_prefill(keys, values, mask_loop3=mask3, mask_loop4=mask4,
-                                                              lengths=lengths, token_capacity=tmax + extra))
+                                                              lengths=lengths, token_capacity=tmax + extra, late_counts=late))
             del keys, values
         logits = torch.cat([r.logits for r in runs], dim=0)
         self._state = BatchState(cache, tuple(lengths), mask3, mask4, tuple(r.receipts for r in runs))

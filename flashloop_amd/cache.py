@@ -51,7 +51,9 @@ class CrossLoopKVLayer:
     residual_length = 64
     group_size = GROUP
 
-    def __init__(self, geometry: LayerGeometry, device) -> None:
+    def __init__(self, geometry: LayerGeometry, device, *, _clear: bool = True) -> None:
+        # _clear=False: the buffers are left to fl_cache_prepare and fl_pack_kv_groups, which
+        # between them write every byte (from_prefill)
         g = geometry
         if g.token_capacity % GROUP:
             raise ValueError("token_capacity must be a multiple of 64")
@@ -65,28 +67,30 @@ class CrossLoopKVLayer:
         rows = g.batch * g.heads
         dev = self.device
         # one 128-byte line per token and stream: K codes in bytes 0..63, V codes in 64..127
-        self.codes = [torch.zeros(rows, g.row_capacity[s], 2 * (HEAD_DIM // 2), dtype=torch.uint8, device=dev)
-                      for s in range(4)]
+        new = torch.zeros if _clear else torch.empty
+        self.codes = [new(rows, g.row_capacity[s], 2 * (HEAD_DIM // 2), dtype=torch.uint8, device=dev) for s in range(4)]
         self.key_codes = [c[..., : HEAD_DIM // 2] for c in self.codes]
         self.value_codes = [c[..., HEAD_DIM // 2 :] for c in self.codes]
-        self.key_meta = [torch.zeros(rows, g.token_capacity // GROUP, HEAD_DIM, 2, dtype=torch.float32, device=dev) for _ in range(4)]
-        self.value_meta = [torch.zeros(rows, g.row_capacity[s], 2, 2, dtype=torch.float32, device=dev) for s in range(4)]
+        self.key_meta = [new(rows, g.token_capacity // GROUP, HEAD_DIM, 2, dtype=torch.float32, device=dev) for _ in range(4)]
+        self.value_meta = [new(rows, g.row_capacity[s], 2, 2, dtype=torch.float32, device=dev) for s in range(4)]
         # the V metadata of all four streams again, one 64-byte record per logical token
         # ([half][stream][scale, min]) for the readers of selected tokens
-        self.value_meta_token = torch.zeros(rows, g.token_capacity, 2, 4, 2, dtype=torch.float32, device=dev)
+        self.value_meta_token = new(rows, g.token_capacity, 2, 4, 2, dtype=torch.float32, device=dev)
         # fp16 copy of the K metadata, streamed by the readers of selected tokens
-        self.key_meta_half = [torch.zeros(rows, g.token_capacity // GROUP, HEAD_DIM, 2, dtype=torch.float16, device=dev)
+        self.key_meta_half = [new(rows, g.token_capacity // GROUP, HEAD_DIM, 2, dtype=torch.float16, device=dev)
                               for _ in range(4)]
-        self.value_meta_half = [torch.zeros(rows, g.row_capacity[s], 2, 2, dtype=torch.float16, device=dev)
-                                for s in range(4)]
-        self.rank = [torch.full((g.batch, g.token_capacity), -1, dtype=torch.int32, device=dev) for _ in range(2)]
-        self.tail_key = [torch.zeros(rows, g.tail_capacity, HEAD_DIM, dtype=torch.bfloat16, device=dev) for _ in range(4)]
-        self.tail_value = [torch.zeros(rows, g.tail_capacity, HEAD_DIM, dtype=torch.bfloat16, device=dev) for _ in range(4)]
+        self.value_meta_half = [new(rows, g.row_capacity[s], 2, 2, dtype=torch.float16, device=dev) for s in range(4)]
+        self.rank = [new(g.batch, g.token_capacity, dtype=torch.int32, device=dev) for _ in range(2)]
+        if _clear:
+            for r in self.rank:
+                r.fill_(-1)
+        self.tail_key = [new(rows, g.tail_capacity, HEAD_DIM, dtype=torch.bfloat16, device=dev) for _ in range(4)]
+        self.tail_value = [new(rows, g.tail_capacity, HEAD_DIM, dtype=torch.bfloat16, device=dev) for _ in range(4)]
         # loop-3/4 activity of tail rows (flashloop/cache.py:_tail_active)
-        self.tail_active = [torch.zeros(g.batch, g.tail_capacity, dtype=torch.uint8, device=dev) for _ in range(2)]
-        self.packed_tokens = torch.zeros(g.batch, dtype=torch.int32, device=dev)
-        self.tail_tokens = torch.zeros(g.batch, dtype=torch.int32, device=dev)
-        self.late_rows = torch.zeros(2, g.batch, dtype=torch.int32, device=dev)  # rows used in streams 2/3
+        self.tail_active = [new(g.batch, g.tail_capacity, dtype=torch.uint8, device=dev) for _ in range(2)]
+        self.packed_tokens = new(g.batch, dtype=torch.int32, device=dev)
+        self.tail_tokens = new(g.batch, dtype=torch.int32, device=dev)
+        self.late_rows = new(2, g.batch, dtype=torch.int32, device=dev)  # rows used in streams 2/3
         # host mirrors (no device sync on the decode path)
         self.packed_host = [0] * g.batch
         self.tail_host = [0] * g.batch
@@ -177,6 +181,7 @@ class CrossLoopKVLayer:
         lengths: Sequence[int] | None = None,
         token_capacity: int | None = None,
         recon: bool = False,
+        late_counts: Sequence[Sequence[int]] | None = None,
     ) -> "CrossLoopKVLayer":
         """Pack a prefill's four loop K/V ``[B, H, T, 128]`` bf16 (``CrossLoopKVLayer.from_prefill``,
         flashloop/cache.py:752-817; codec of kv_quantization.py:531-650).
@@ -186,6 +191,8 @@ class CrossLoopKVLayer:
         ``token_capacity``: packed-prefix capacity (room for decode rollover).
         With ``recon=True`` the reconstructed prefixes R_r are returned as
         ``layer.recon_keys/recon_values`` (bf16 ``[B*H, T, 128]``) for audits.
+        ``late_counts``: what ``count_late_rows`` returned for these masks and lengths, for a
+        caller that packs several layers with the same masks (rows beyond a count are dropped).
         """
         if len(keys) != 4 or len(values) != 4:
             raise ValueError("exactly four loop K/V tensors are required")
@@ -199,67 +206,69 @@ class CrossLoopKVLayer:
         if len(lengths) != b or any(x <= 0 or x > t for x in lengths):
             raise ValueError("lengths must give 1..T tokens per sequence")
         dev = keys[0].device
-        masks = []
-        for m in (mask_loop3, mask_loop4):
-            if m is None:
-                masks.append(torch.ones(b, t, dtype=torch.bool, device=dev))
-            else:
-                if tuple(m.shape) != (b, t):
-                    raise ValueError("prefill masks must have shape [B, T]")
-                masks.append(m.to(device=dev, dtype=torch.bool))
-        if not bool(torch.all(~masks[1] | masks[0]).item()):
-            raise ValueError("Loop-4 overrides must be nested in Loop-3 overrides")
+        masks = cls._mask_bytes(mask_loop3, mask_loop4, b, t, dev)
+        if late_counts is None:
+            late = cls._late_counts(masks, lengths)
+        else:
+            late = [[int(x) for x in c] for c in late_counts]
+            if len(late) != 2 or any(len(c) != b or min(c) < 0 for c in late):
+                raise ValueError("late_counts must give a count per sequence for loops 3 and 4")
         tp = [packed_prefix_tokens(x) for x in lengths]
         tp_max = max(tp)
         cap = _round_up(max(token_capacity or 0, tp_max, GROUP), GROUP)
-        # loop-3/4 compact rows of the packed prefix: rank = running count of active rows
-        pos = torch.arange(t, device=dev)
-        tp_t = torch.tensor(tp, device=dev)
-        prefix = pos[None, :] < tp_t[:, None]
-        late_counts = []
-        ranks = []
-        for m in masks:
-            act = m & prefix
-            r = torch.cumsum(act.to(torch.int32), dim=1) - 1
-            r = torch.where(act, r, torch.full_like(r, -1)).to(torch.int32)
-            ranks.append(r)
-            late_counts.append([int(x) for x in act.sum(dim=1).tolist()])
         growth = cap - min(tp)  # every future decode token is active in every loop
-        row_cap = (cap, cap, max(max(late_counts[0]) + growth, 1), max(max(late_counts[1]) + growth, 1))
-        layer = cls(LayerGeometry(b, h, cap, 2 * GROUP, row_cap), dev)
-        for s in range(2):
-            layer.rank[s][:, : min(t, cap)] = ranks[s][:, : min(t, cap)]
-            layer.late_rows_host[s] = late_counts[s]
-            layer.late_rows[s] = torch.tensor(late_counts[s], dtype=torch.int32, device=dev)
+        row_cap = (cap, cap, max(max(late[0]) + growth, 1), max(max(late[1]) + growth, 1))
+        layer = cls(LayerGeometry(b, h, cap, 2 * GROUP, row_cap), dev, _clear=False)
+        layer.late_rows_host = late
         layer.packed_host = list(tp)
         layer.tail_host = [x - p for x, p in zip(lengths, tp)]
-        layer.packed_tokens.copy_(torch.tensor(tp, dtype=torch.int32))
-        layer.tail_tokens.copy_(torch.tensor(layer.tail_host, dtype=torch.int32))
+        src_k, src_v = [x.contiguous() for x in keys], [x.contiguous() for x in values]
+        group0 = torch.empty(b, dtype=torch.int32, device=dev)
+        # lengths, loop-3/4 compact rows (rank = running count of active rows), BF16 tails
+        # (flashloop/cache.py:806-812) and the unused capacity, then the packed prefix
+        kernels.cache_prepare(layer.view(), src_k, src_v, masks, layer.tail_active, tp, layer.tail_host, late,
+                              layer.packed_tokens, layer.tail_tokens, layer.late_rows, group0)
         if tp_max:
-            src_k = [x.reshape(b * h, t, c) for x in keys]
-            src_v = [x.reshape(b * h, t, c) for x in values]
-            mk = [m.to(torch.uint8).contiguous() for m in masks]
             rk = rv = None
             if recon:
                 rk = [torch.zeros(b * h, t, c, dtype=torch.bfloat16, device=dev) for _ in range(4)]
                 rv = [torch.zeros(b * h, t, c, dtype=torch.bfloat16, device=dev) for _ in range(4)]
             kernels.pack_kv_groups(
-                layer.view(), 4, [x.contiguous() for x in src_k], [x.contiguous() for x in src_v],
-                src_bh_stride=t, src_row_offset=0,
-                dst_group0=torch.zeros(b, dtype=torch.int32, device=dev), n_groups=tp_max // GROUP,
-                masks=mk, mask_stride=t, recon_keys=rk, recon_values=rv,
+                layer.view(), 4, src_k, src_v, src_bh_stride=t, src_row_offset=0, dst_group0=group0,
+                n_groups=tp_max // GROUP, masks=masks, mask_stride=t, recon_keys=rk, recon_values=rv,
             )
             if recon:
                 layer.recon_keys, layer.recon_values = rk, rv
-        # BF16 tails (flashloop/cache.py:806-812)
-        for bi, (p, n) in enumerate(zip(tp, lengths)):
-            rows = slice(bi * h, (bi + 1) * h)
-            for r in range(4):
-                layer.tail_key[r][rows, : n - p] = keys[r][bi, :, p:n]
-                layer.tail_value[r][rows, : n - p] = values[r][bi, :, p:n]
-            for s in range(2):
-                layer.tail_active[s][bi, : n - p] = masks[s][bi, p:n].to(torch.uint8)
         return layer
+
+    @staticmethod
+    def _mask_bytes(mask_loop3, mask_loop4, b: int, t: int, dev):
+        """The prefill masks as contiguous u8 [B, T] on the device (None: every row)."""
+        masks = []
+        for m in (mask_loop3, mask_loop4):
+            if m is not None and tuple(m.shape) != (b, t):
+                raise ValueError("prefill masks must have shape [B, T]")
+            masks.append(None if m is None else m.to(device=dev, dtype=torch.bool).contiguous().view(torch.uint8))
+        return masks
+
+    @staticmethod
+    def _late_counts(masks, lengths: Sequence[int]) -> list[list[int]]:
+        tp = [packed_prefix_tokens(x) for x in lengths]
+        if masks[0] is None and masks[1] is None:
+            return [list(tp), list(tp)]
+        counts, nested = kernels.count_active_rows(masks, tp)
+        if not nested:
+            raise ValueError("Loop-4 overrides must be nested in Loop-3 overrides")
+        return counts
+
+    @classmethod
+    def count_late_rows(cls, mask_loop3: torch.Tensor, mask_loop4: torch.Tensor,
+                        lengths: Sequence[int] | None = None) -> list[list[int]]:
+        """Packed-prefix rows of each sequence that loops 3 and 4 keep under these prefill masks
+        (``[B, T]`` bool on the device), read back once: ``late_counts`` of ``from_prefill``."""
+        b, t = mask_loop3.shape
+        masks = cls._mask_bytes(mask_loop3, mask_loop4, b, t, mask_loop3.device)
+        return cls._late_counts(masks, [t] * b if lengths is None else [int(x) for x in lengths])
 
     # ------------------------------------------------------------------ readers
     def logits_capacity(self) -> int:
@@ -409,11 +418,10 @@ class CrossLoopKVLayer:
     def _roll_groups(self) -> None:
         """``_roll_one_group`` (flashloop/cache.py:1778-1838) for every sequence whose tail
         holds residual+group rows: pack tail rows [0, 64) as prefix group Tp/64, then shift
-        the tail down by 64.  O(group): the prefix is never re-read.  Every step is a device
-        op on device counts (no host read-back), unless the loop-3/4 row capacity could be
-        exhausted, which is then checked exactly."""
-        b, h = self.batch, self.heads
-        dev = self.device
+        the tail down by 64.  O(group): the prefix is never re-read.  Three launches on device
+        counts (no host read-back), unless the loop-3/4 row capacity could be exhausted,
+        which is then checked exactly."""
+        b = self.batch
         roll = [x >= self.residual_length + GROUP for x in self.tail_host]
         for i in range(b):
             if roll[i] and self.packed_host[i] + GROUP > self.geometry.token_capacity:
@@ -427,44 +435,16 @@ class CrossLoopKVLayer:
                     act_n = int(self.tail_active[s][i, :GROUP].sum().item())
                     if self.late_rows_host[s][i] + act_n > cap:  # exact (reads back)
                         raise RuntimeError("loop-3/4 row capacity exhausted")
-        # rank maps of the new group's rows (active rows continue the compact numbering)
-        for s in range(2):
-            for i in range(b):
-                if not roll[i]:
-                    continue
-                act = self.tail_active[s][i, :GROUP].bool()
-                r = torch.cumsum(act.to(torch.int32), 0) - 1 + self.late_rows[s, i]
-                p = self.packed_host[i]
-                self.rank[s][i, p : p + GROUP] = torch.where(act, r, torch.full_like(r, -1))
-                self.late_rows[s, i] += act.sum(dtype=torch.int32)
-                self._late_pending[s][i] += GROUP
-                self._late_stale = True
-        dst = torch.full((b,), -1, dtype=torch.int32, device=dev)
+        # the device rolls the sequences its own lengths say are full: those of the mirrors
+        kernels.roll_group(self.view(), self.tail_key, self.tail_value, self.tail_active, self.packed_tokens,
+                           self.tail_tokens, self.late_rows)
         for i in range(b):
             if roll[i]:
-                dst[i] = self.packed_host[i] // GROUP
-        kernels.pack_kv_groups(
-            self.view(), 4, self.tail_key, self.tail_value, src_bh_stride=self.geometry.tail_capacity,
-            src_row_offset=0, dst_group0=dst, n_groups=1, masks=self.tail_active,
-            mask_stride=self.geometry.tail_capacity,
-        )
-        for i in range(b):
-            if not roll[i]:
-                continue
-            rows = slice(i * h, (i + 1) * h)
-            n = self.tail_host[i] - GROUP
-            # rows [GROUP, GROUP + n) -> [0, n): disjoint ranges (no copy first) when n <= GROUP
-            def shift(src):
-                return src if n <= GROUP else src.clone()
-            for tensor in (*self.tail_key, *self.tail_value):
-                tensor[rows, :n] = shift(tensor[rows, GROUP : GROUP + n])
-            for act in self.tail_active:
-                act[i, :n] = shift(act[i, GROUP : GROUP + n])
-                act[i, n:] = 0
-            self.packed_host[i] += GROUP
-            self.tail_host[i] = n
-            self.packed_tokens[i] += GROUP
-            self.tail_tokens[i] -= GROUP
+                self.packed_host[i] += GROUP
+                self.tail_host[i] -= GROUP
+                for s in range(2):
+                    self._late_pending[s][i] += GROUP
+                self._late_stale = True
 
     # ------------------------------------------------------------------ serialization
     # On-disk format (FORMAT_NAME, FORMAT_VERSION): one safetensors file whose tensors are

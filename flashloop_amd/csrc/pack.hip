@@ -357,8 +357,9 @@ __device__ __forceinline__ void value_loop(const PackArgs& a, int b, int bh, int
   if (__builtin_expect(__any(needs_exact_div(q)), 0)) encode_row(std::true_type{});
   else encode_row(std::false_type{});
   const int row = token_row<R>(a, tin);
+  const int64_t rec =
+      ((static_cast<int64_t>(bh) * v.token_capacity + g * kGroup + i) * 2 + half) * 4 + R;  // per-token record entry
   if (row >= 0) {
-    const int t = g * kGroup + i;
     const int64_t rowi = static_cast<int64_t>(bh) * v.row_capacity[R] + row;
     *reinterpret_cast<uint4*>(v.value_codes[R] + rowi * kCodeStride + 16 * quarter) =
         make_uint4(words[0], words[1], words[2], words[3]);
@@ -366,9 +367,10 @@ __device__ __forceinline__ void value_loop(const PackArgs& a, int b, int bh, int
       *reinterpret_cast<float2*>(v.value_meta[R] + (rowi * 2 + half) * 2) = make_float2(q.scale, q.minimum);
       *reinterpret_cast<uint32_t*>(v.value_meta_half[R] + (rowi * 2 + half) * 2) =
           static_cast<uint32_t>(f32_to_f16(q.scale)) | (static_cast<uint32_t>(f32_to_f16(q.minimum)) << 16);
-      const int64_t rec = ((static_cast<int64_t>(bh) * v.token_capacity + t) * 2 + half) * 4 + R;
       *reinterpret_cast<float2*>(v.value_meta_token + rec * 2) = make_float2(q.scale, q.minimum);
     }
+  } else if (R >= 2 && (quarter & 1) == 0) {  // not stored: the record says so with zeros
+    *reinterpret_cast<float2*>(v.value_meta_token + rec * 2) = make_float2(0.0f, 0.0f);
   }
   if (a.rv[R] != nullptr) {
     uint4* dst = reinterpret_cast<uint4*>(a.rv[R] + row_off);

@@ -445,10 +445,11 @@ class FlashLoopEngine:
         loops = self._prefill_loops(input_ids, stage, all_logits=all_logits)
         cap = t + (self.config.decode_capacity if decode_capacity is None else int(decode_capacity))
         cache = CrossLoopKVCache(num_layers=len(self.layers))
+        late = CrossLoopKVLayer.count_late_rows(loops.mask3, loops.mask4)
         for li in range(len(self.layers)):
             cache.set_layer(li, CrossLoopKVLayer.from_prefill(
                 [k[li] for k in loops.keys], [v[li] for v in loops.values],
-                mask_loop3=loops.mask3, mask_loop4=loops.mask4, token_capacity=cap))
+                mask_loop3=loops.mask3, mask_loop4=loops.mask4, token_capacity=cap, late_counts=late))
         stage("physical_cache_finalized")
         self._state = EngineState(cache, t, loops.mask3, loops.mask4, loops.receipts)
         self._runner.reset()  # a new cache: captured pointers are stale

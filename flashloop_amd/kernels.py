@@ -60,6 +60,56 @@ def pack_kv_groups(view, loops, src_keys, src_values, *, src_bh_stride, src_row_
     check(rc, "fl_pack_kv_groups")
 
 
+def _ptrs(tensors):
+    return C.cast(ptr_array([_p(t) or 0 for t in tensors]), _lib._PP)
+
+
+def _ints(values):
+    return (C.c_int32 * len(values))(*values)
+
+
+def count_active_rows(masks, packed) -> tuple[list[list[int]], bool]:
+    """Tokens below each sequence's packed prefix that loops 3/4 keep (``masks``: two u8 [B, T]
+    device tensors or None for every token), and whether the masks are nested
+    (``fl_count_active_rows``).  Reads the counts back (one synchronisation)."""
+    some = next(m for m in masks if m is not None)
+    b, t = some.shape
+    for m in masks:
+        if m is not None:
+            _require(m, torch.uint8, "mask")
+    counts = torch.zeros(2 * b + 1, dtype=torch.int32, device=some.device)
+    check(load().fl_count_active_rows(_ptrs(masks), t, b, t, _ints(packed), counts.data_ptr(), _stream()),
+          "fl_count_active_rows")
+    got = counts.tolist()
+    return [got[:b], got[b:2 * b]], got[2 * b] == 0
+
+
+def cache_prepare(view, src_keys, src_values, masks, tail_active, packed, tail, late, packed_tokens, tail_tokens,
+                  late_rows, dst_group0) -> None:
+    """Lengths, rank maps, BF16 tails and unused capacity of a new layer (``fl_cache_prepare``);
+    sources bf16 [B, H, T, 128], masks u8 [B, T] or None, ``packed``/``tail``/``late`` host lists."""
+    t = src_keys[0].shape[2]
+    check(load().fl_cache_prepare(
+        C.byref(view), _ptrs(src_keys), _ptrs(src_values), t, _ptrs(masks), t, _ptrs(tail_active), _ints(packed),
+        _ints(tail), _ints([*late[0], *late[1]]), packed_tokens.data_ptr(), tail_tokens.data_ptr(), late_rows.data_ptr(),
+        dst_group0.data_ptr(), _stream()), "fl_cache_prepare")
+
+
+def roll_group(view, tail_keys, tail_values, tail_active, packed_tokens, tail_tokens, late_rows) -> None:
+    """Roll one 64-token group out of every full tail: rank rows, packing, tail shift and
+    lengths, decided by the device lengths (``fl_roll_begin``, ``fl_pack_kv_groups``,
+    ``fl_roll_end``)."""
+    lib = load()
+    scratch = torch.empty(2 * view.batch, dtype=torch.int32, device=packed_tokens.device)
+    args = (C.byref(view), packed_tokens.data_ptr(), tail_tokens.data_ptr(), late_rows.data_ptr(), _ptrs(tail_active),
+            scratch.data_ptr(), _stream())
+    check(lib.fl_roll_begin(*args), "fl_roll_begin")
+    cap = view.tail_capacity
+    pack_kv_groups(view, 4, tail_keys, tail_values, src_bh_stride=cap, src_row_offset=0, dst_group0=scratch, n_groups=1,
+                   masks=tail_active, mask_stride=cap)
+    check(lib.fl_roll_end(*args), "fl_roll_end")
+
+
 # ---------------------------------------------------------------------------- J2
 class Workspace:
     """Grow-only device scratch reused across calls ordered on one stream (the reference

@@ -59,7 +59,7 @@ extern "C" {
  *   value_meta_token f32 [B*H, token_capacity, 2, 4, 2]  the same V (scale, min) again,
  *                      per logical token: [half][stream] in one 64-byte record, so that a
  *                      reader of selected tokens fetches one line for every stream's
- *                      V metadata (entries of streams 2/3 at inactive tokens are unused)
+ *                      V metadata (entries of streams 2/3 at inactive tokens are zero)
  *   key_meta_half[s] f16 [B*H, token_capacity/64, 128, 2]  key_meta[s] rounded to fp16
  *                      (nearest even, overflow to +-inf, as torch's .to(torch.float16))
  *   value_meta_half[s] f16 [B*H, row_capacity[s], 2, 2]  value_meta[s] rounded likewise
@@ -129,6 +129,41 @@ int32_t fl_pack_kv_groups(const fl_cache_view* view, int32_t loops,
                           const int32_t* dst_group0, int32_t n_groups,
                           uint16_t* const* recon_keys, uint16_t* const* recon_values,
                           void* stream);
+
+/*
+ * Set-up of a packed cache around fl_pack_kv_groups (CrossLoopKVLayer.from_prefill and
+ * _roll_one_group, flashloop/cache.py:752-817, 1778-1838).
+ *
+ * fl_count_active_rows: counts[s * batch + b] (i32, device) = tokens t < packed[b] (host
+ * array) with masks[s][b, t] set (u8 [batch, mask_stride]; a null mask sets every token),
+ * and counts[2 * batch] |= 1 if masks[1] sets a token of the first `tokens` that masks[0]
+ * does not (the caller zeroes that word).
+ * fl_cache_prepare: fills the parts of a newly allocated layer that fl_pack_kv_groups does not
+ * write.  Host arrays: packed, tail [B], late [2, B] (rows kept by streams 2/3).  Writes the
+ * device lengths packed_tokens, tail_tokens [B], late_rows [2, B], zeros dst_group0 [B], the
+ * rank maps (running count of the active tokens of masks[s] below packed[b]; -1 elsewhere),
+ * each loop's BF16 tail (source rows packed[b] .. + tail[b], then zeros) with its activity
+ * tail_active[s] (u8 [B, tail_capacity]), and zeros in the capacity past the packed prefix
+ * and past the kept rows.  Sources as for fl_pack_kv_groups.
+ * fl_roll_begin / fl_roll_end: around the packing of one group from the tails
+ * (fl_pack_kv_groups with src_row_offset 0, n_groups 1, dst_group0 = scratch).  A sequence
+ * rolls when its tail holds at least 128 rows and the prefix has room: begin writes its
+ * group (-1 for the others) to scratch[b], the group's rank rows and the advanced late_rows;
+ * end moves tail rows [64, tail) to the front with their activity (zeros past them) and
+ * sets the lengths.  scratch: i32 [2, B] device memory, unchanged between the two calls.
+ */
+int32_t fl_count_active_rows(const uint8_t* const* masks, int64_t mask_stride, int32_t batch, int32_t tokens,
+                             const int32_t* packed, int32_t* counts, void* stream);
+int32_t fl_cache_prepare(const fl_cache_view* view, const uint16_t* const* src_keys,
+                         const uint16_t* const* src_values, int64_t src_bh_stride,
+                         const uint8_t* const* masks, int64_t mask_stride, uint8_t* const* tail_active,
+                         const int32_t* packed, const int32_t* tail, const int32_t* late,
+                         int32_t* packed_tokens, int32_t* tail_tokens, int32_t* late_rows,
+                         int32_t* dst_group0, void* stream);
+int32_t fl_roll_begin(const fl_cache_view* view, int32_t* packed_tokens, int32_t* tail_tokens,
+                      int32_t* late_rows, uint8_t* const* tail_active, int32_t* scratch, void* stream);
+int32_t fl_roll_end(const fl_cache_view* view, int32_t* packed_tokens, int32_t* tail_tokens,
+                    int32_t* late_rows, uint8_t* const* tail_active, int32_t* scratch, void* stream);
 
 /*
  * J2 -- fused dense decode reader: dequantize, rebuild loop `loop`, q.K^T, online
