@@ -335,8 +335,8 @@ class CrossLoopKVLayer:
         ``flashloop/selection.py:78-79`` does."""
         cap = kernels.decode_capacity(self.token_count + 1, fraction)
         idx, valid, mass, w, counts = kernels.decode_topk(
-            logits.reshape(self.rows, -1), self.key_counts(), fraction, cap, rows_per_count=self.heads,
-            validate=validate,
+            logits.reshape(self.rows, -1), self.packed_tokens, fraction, cap, rows_per_count=self.heads,
+            validate=validate, more_keys=self.tail_tokens, plus_keys=1,
         )
         shape = (self.batch, self.heads, cap)
         return idx.view(shape), valid.view(shape), mass.view(self.batch, self.heads, 1, 1), w.view(shape), counts

@@ -8,12 +8,15 @@
 //    (flashloop/selection.py:26-69).
 //
 // One workgroup of 1024 threads per row.  Scores are mapped to order-preserving
-// unsigned keys.  Decode rows of up to 35K keys are held in registers and selected in
-// one read (decode_topk_resident_kernel).  Longer rows and the prefill token selection
-// re-read the row (it stays in L2): four 8-bit histogram passes (LDS atomics) find the
+// unsigned keys.  Decode rows of up to 36K keys are held in registers and selected in
+// one read (decode_topk_resident_kernel); longer rows, or selections, are divided over
+// several workgroups (fl_decode_topk_long).  Long rows without a workspace and the prefill
+// token selection re-read the row (it stays in L2): four 8-bit histogram passes (LDS atomics) find the
 // k-th largest key K* and how many keys equal to K* to take, then a final pass walks the
 // row in index order, takes every key > K* and the first `need` keys == K*
 // (ballot/popcount ranks), and writes the selected indices in ascending order.
+#include <algorithm>
+
 #include "dense_layout.h"
 #include "internal.h"
 
@@ -239,15 +242,11 @@ struct AllCand {
   __device__ bool operator()(int) const { return true; }
 };
 
-__global__ __launch_bounds__(kTopkThreads) void decode_topk_kernel(const float* scores, int64_t stride,
-                                                                   const int32_t* n_keys, int rows_per_count,
-                                                                   double fraction, int cap, int32_t* indices,
-                                                                   uint8_t* valid, float* mass, float* weights,
-                                                                   int32_t* counts, int32_t* nonfinite) {
-  __shared__ TopkShared sh;
-  const int r = blockIdx.x;
+// Top-k of row r (its first n scores) by one workgroup that re-reads the row from memory.
+__device__ __forceinline__ void topk_global_row(TopkShared& sh, int r, int n, const float* scores, int64_t stride,
+                                                double fraction, int cap, int32_t* indices, uint8_t* valid, float* mass,
+                                                float* weights, int32_t* counts, int32_t* nonfinite) {
   const float* x = scores + static_cast<int64_t>(r) * stride;
-  const int n = min(n_keys[r / rows_per_count], static_cast<int>(min<int64_t>(stride, 0x7fffffff)));
   int32_t* oi = indices + static_cast<int64_t>(r) * cap;
   uint8_t* ov = valid + static_cast<int64_t>(r) * cap;
   float* ow = weights + static_cast<int64_t>(r) * cap;
@@ -332,6 +331,17 @@ __global__ __launch_bounds__(kTopkThreads) void decode_topk_kernel(const float* 
     if (counts) counts[r] = k;
     if (nonfinite) nonfinite[r] = static_cast<int32_t>(sh.nonfin);
   }
+}
+
+__global__ __launch_bounds__(kTopkThreads) void decode_topk_kernel(const float* scores, int64_t stride,
+                                                                   const int32_t* n_keys, int rows_per_count,
+                                                                   double fraction, int cap, int32_t* indices,
+                                                                   uint8_t* valid, float* mass, float* weights,
+                                                                   int32_t* counts, int32_t* nonfinite) {
+  __shared__ TopkShared sh;
+  const int r = blockIdx.x;
+  const int n = min(n_keys[r / rows_per_count], static_cast<int>(min<int64_t>(stride, 0x7fffffff)));
+  topk_global_row(sh, r, n, scores, stride, fraction, cap, indices, valid, mass, weights, counts, nonfinite);
 }
 
 // Register-resident variant for rows of at most kResKeys keys and k <= kSelLds: thread t
@@ -924,6 +934,458 @@ __global__ __launch_bounds__(kTopkThreads) void select_merge_kernel(TopkArgs A, 
   reader::dense_merge_row(L.m, blockIdx.x - rows, ws, ws, W, v, out, out, 1);
 }
 
+// ---------------------------------------------------------------------------------
+// Rows beyond the register-resident kernel: each row over ceil(stride / 4096) workgroups, a
+// slice of 4096 keys each (four per thread), in six launches.  One workgroup per row left all
+// but `rows` CUs idle and re-read and re-exponentiated the row seven times: 16 rows of 70,001
+// keys took 200 us.  The keys, the normaliser's order and the ranking are those of the
+// resident kernel, so the selection is the same bit for bit:
+//   1. extremes: each slice's maximum, minimum and non-finite scores;
+//   2. normaliser: workgroup w sums the e of threads 64 w .. 64 w + 63 of the resident
+//      kernel's slot order over the whole row, and folds them as its wave w does;
+//   3. histogram: each slice's keys over the row's 1024 key-linear bins;
+//   4. candidates: the boundary bin B*, each slice's count of keys above it, and the keys of
+//      B* in a list of the row;
+//   5. compact: the candidates are ranked, which gives the k-th key; each slice writes its
+//      selected keys at its offset, in index order;
+//   6. finish: mass and normalised weights.  A row whose boundary bin overflows the list (many
+//      equal keys, or a row without finite weights, ranked by score in one bin) is done by
+//      one workgroup as before (topk_global_row).
+constexpr int kSliceKeys = kQuadChunk;
+constexpr int kSplitCand = 1024;
+
+struct SplitArgs {
+  const float* scores;
+  int64_t stride;
+  const int32_t* n_keys;
+  const int32_t* more_keys;
+  int plus_keys;
+  int rows_per_count;
+  double fraction;
+  int cap, slices;
+  int32_t* indices;
+  uint8_t* valid;
+  float* mass;
+  float* weights;
+  int32_t* counts;
+  int32_t* nonfinite;
+  uint32_t* ws;
+};
+
+int split_slices(int64_t stride) { return static_cast<int>((stride + kSliceKeys - 1) / kSliceKeys); }
+// 32-bit words of one row's workspace
+__host__ __device__ inline size_t split_words(int slices) {
+  const size_t w = 6 * static_cast<size_t>(slices) + kTopkWaves + kBins + 4 + 2 * kSplitCand;
+  return (w + 3) / 4 * 4;
+}
+
+struct SplitRow {
+  uint4* part;         // [slices]: max, min (float bits), max |x| bits, non-finite count
+  uint32_t* hist;      // [kBins]
+  uint32_t* ncand;     // [4] (one used)
+  uint32_t* cand_key;  // [kSplitCand]
+  uint32_t* cand_idx;  // [kSplitCand]
+  float* wsum;         // [kTopkWaves]
+  uint32_t* above;     // [slices]: keys above B*
+  float* pmass;        // [slices]
+  const float* x;
+  int n, k;
+};
+
+__device__ __forceinline__ SplitRow split_row(const SplitArgs& a, int r) {
+  SplitRow s;
+  uint32_t* p = a.ws + static_cast<size_t>(r) * split_words(a.slices);
+  s.part = reinterpret_cast<uint4*>(p);
+  p += 4 * a.slices;
+  s.hist = p;
+  p += kBins;
+  s.ncand = p;
+  p += 4;
+  s.cand_key = p;
+  p += kSplitCand;
+  s.cand_idx = p;
+  p += kSplitCand;
+  s.wsum = reinterpret_cast<float*>(p);
+  p += kTopkWaves;
+  s.above = p;
+  p += a.slices;
+  s.pmass = reinterpret_cast<float*>(p);
+  s.x = a.scores + static_cast<int64_t>(r) * a.stride;
+  const int i = r / a.rows_per_count;
+  const int64_t keys = static_cast<int64_t>(a.n_keys[i]) + (a.more_keys ? a.more_keys[i] : 0) + a.plus_keys;
+  s.n = static_cast<int>(max<int64_t>(0, min<int64_t>(keys, a.stride)));
+  s.k = 0;
+  if (s.n > 0) {
+    const double want = ceil(static_cast<double>(s.n) * a.fraction);
+    s.k = min(min(static_cast<int>(want < 1.0 ? 1.0 : want), s.n), a.cap);
+  }
+  return s;
+}
+
+// This thread's four keys of the slice, -inf past n.
+__device__ __forceinline__ void slice_scores(const SplitRow& s, int base, float (&x)[4]) {
+  if (base + 4 <= s.n && (reinterpret_cast<uintptr_t>(s.x) & 15u) == 0) {
+    const float4 v = *reinterpret_cast<const float4*>(s.x + base);
+    x[0] = v.x;
+    x[1] = v.y;
+    x[2] = v.z;
+    x[3] = v.w;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = base + e < s.n ? s.x[base + e] : -INFINITY;
+  }
+}
+
+// What a row's ranking needs, from its slices' extremes (every wave computes it alike).
+struct SplitScale {
+  float M;
+  bool weighted;  // false: a NaN, a +inf or only -inf
+  float invZ;
+  uint32_t kmin, shift, nonfinite;
+};
+
+__device__ __forceinline__ SplitScale split_scale(const SplitRow& s, bool with_z) {
+  const int lane = threadIdx.x & 63, slices = (s.n + kSliceKeys - 1) / kSliceKeys;
+  float mx = -INFINITY, mn = INFINITY;
+  uint32_t amax = 0, nf = 0;
+  for (int i = lane; i < slices; i += kWave) {
+    const uint4 p = s.part[i];
+    mx = fmaxf(mx, __uint_as_float(p.x));
+    mn = fminf(mn, __uint_as_float(p.y));
+    amax = max(amax, p.z);
+    nf += p.w;
+  }
+#pragma unroll
+  for (int off = kWave / 2; off >= 1; off >>= 1) {
+    mx = fmaxf(mx, __shfl_xor(mx, off, kWave));
+    mn = fminf(mn, __shfl_xor(mn, off, kWave));
+    amax = max(amax, static_cast<uint32_t>(__shfl_xor(static_cast<int>(amax), off, kWave)));
+    nf += static_cast<uint32_t>(__shfl_xor(static_cast<int>(nf), off, kWave));
+  }
+  SplitScale c{mx, amax <= 0x7F800000u && mx > -INFINITY && mx < INFINITY, 0.0f, kScoreKeyFloor, 31u, nf};
+  if (with_z && c.weighted) {
+    float Z = s.wsum[0];
+#pragma unroll
+    for (int i = 1; i < kTopkWaves; ++i) Z += s.wsum[i];
+    c.invZ = 1.0f / Z;
+    c.kmin = weight_key(softmax_exp(mn - mx), c.invZ);
+    const uint32_t span = max(__float_as_uint(c.invZ) + 1u, c.kmin) - c.kmin;
+    c.shift = span < static_cast<uint32_t>(kBins) ? 0u : 32u - static_cast<uint32_t>(__clz(span)) - 10u;
+  }
+  return c;
+}
+
+// Ranking key of score x (0 past the row's end), and its bin.
+__device__ __forceinline__ uint32_t split_key(const SplitScale& c, float x, bool in) {
+  if (!in) return 0u;
+  return c.weighted ? weight_key(softmax_exp(x - c.M), c.invZ) : score_key(x);
+}
+__device__ __forceinline__ int split_bin(const SplitScale& c, uint32_t key) {
+  const uint32_t top = c.weighted ? kBins - 1 : 0u;
+  return static_cast<int>(min(static_cast<uint32_t>(max(static_cast<int>(key - c.kmin), 0)) >> c.shift, top));
+}
+
+__global__ __launch_bounds__(kTopkThreads) void split_extremes_kernel(SplitArgs a) {
+  __shared__ uint4 red[kTopkWaves];
+  const SplitRow s = split_row(a, blockIdx.y);
+  const int slice = blockIdx.x, tid = threadIdx.x, base = slice * kSliceKeys + 4 * tid;
+  if (slice == 0) {
+    s.hist[tid] = 0;
+    if (tid == 0) s.ncand[0] = 0;
+  }
+  if (slice * kSliceKeys >= s.n) return;
+  float x[4];
+  slice_scores(s, base, x);
+  float mx = -INFINITY, mn = INFINITY;
+  uint32_t amax = 0, nf = 0;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const bool in = base + e < s.n;
+    mx = fmaxf(mx, x[e]);
+    mn = fminf(mn, in ? x[e] : INFINITY);
+    amax = max(amax, in ? __float_as_uint(x[e]) & 0x7FFFFFFFu : 0u);
+    nf += in && non_finite(x[e]) ? 1u : 0u;
+  }
+#pragma unroll
+  for (int off = kWave / 2; off >= 1; off >>= 1) {
+    mx = fmaxf(mx, __shfl_xor(mx, off, kWave));
+    mn = fminf(mn, __shfl_xor(mn, off, kWave));
+    amax = max(amax, static_cast<uint32_t>(__shfl_xor(static_cast<int>(amax), off, kWave)));
+    nf += static_cast<uint32_t>(__shfl_xor(static_cast<int>(nf), off, kWave));
+  }
+  if ((tid & 63) == 0) red[tid >> 6] = make_uint4(__float_as_uint(mx), __float_as_uint(mn), amax, nf);
+  __syncthreads();
+  if (tid == 0) {
+    for (int w = 1; w < kTopkWaves; ++w) {
+      mx = fmaxf(mx, __uint_as_float(red[w].x));
+      mn = fminf(mn, __uint_as_float(red[w].y));
+      amax = max(amax, red[w].z);
+      nf += red[w].w;
+    }
+    s.part[slice] = make_uint4(__float_as_uint(mx), __float_as_uint(mn), amax, nf);
+  }
+}
+
+// Workgroup w: the 64 threads 64 w + t of the resident kernel.  Its 16 waves take the e of the
+// quad chunks in turn (wave g chunk base + g, lane t), then wave 0 adds them in chunk order.
+__global__ __launch_bounds__(kTopkThreads) void split_normaliser_kernel(SplitArgs a) {
+  __shared__ float4 ex[kTopkWaves][kWave];
+  const SplitRow s = split_row(a, blockIdx.y);
+  const int w = blockIdx.x, lane = threadIdx.x & 63, g = threadIdx.x >> 6;
+  if (s.n == 0) return;
+  const SplitScale c = split_scale(s, false);
+  if (!c.weighted) return;
+  float z = 0.0f;
+  const int chunks = (s.n + kQuadChunk - 1) / kQuadChunk;
+  for (int q0 = 0; q0 < chunks; q0 += kTopkWaves) {
+    float e[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    const int base = (q0 + g) * kQuadChunk + 4 * (64 * w + lane);
+    if (base < s.n) {
+      float x[4];
+      slice_scores(s, base, x);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) e[i] = base + i < s.n ? softmax_exp(x[i] - c.M) : 0.0f;
+    }
+    __syncthreads();
+    ex[g][lane] = make_float4(e[0], e[1], e[2], e[3]);
+    __syncthreads();
+    if (g == 0) {
+      const int m = min(kTopkWaves, chunks - q0);
+      for (int q = 0; q < m; ++q) {  // (past the end the e are +0: they add nothing)
+        const float4 v = ex[q][lane];
+        z += v.x;
+        z += v.y;
+        z += v.z;
+        z += v.w;
+      }
+    }
+  }
+  if (g == 0) {
+    z = wave_sum_fixed(z);
+    if (lane == 0) s.wsum[w] = z;
+  }
+}
+
+__global__ __launch_bounds__(kTopkThreads) void split_histogram_kernel(SplitArgs a) {
+  __shared__ uint32_t hist[kBins];
+  const SplitRow s = split_row(a, blockIdx.y);
+  const int slice = blockIdx.x, tid = threadIdx.x, base = slice * kSliceKeys + 4 * tid;
+  if (slice * kSliceKeys >= s.n) return;
+  hist[tid] = 0;
+  float x[4];
+  slice_scores(s, base, x);
+  const SplitScale c = split_scale(s, true);
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint32_t key = split_key(c, x[e], base + e < s.n);
+    if (key != 0u) atomicAdd(&hist[split_bin(c, key)], 1u);
+  }
+  __syncthreads();
+  if (hist[tid] != 0u) atomicAdd(&s.hist[tid], hist[tid]);
+}
+
+// The boundary bin (all threads): B*, and the number of keys in higher bins.
+__device__ __forceinline__ void split_boundary(const SplitRow& s, uint32_t* cnt, uint32_t* found, int* bstar, int* above) {
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int bin = kBins - 1 - tid;  // descending scan
+  const uint32_t h = s.hist[bin];
+  uint32_t incl = h;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const uint32_t u = __shfl_up(incl, o, kWave);
+    if (lane >= o) incl += u;
+  }
+  if (lane == 63) cnt[w] = incl;
+  __syncthreads();
+  uint32_t before = 0;
+  for (int q = 0; q < w; ++q) before += cnt[q];
+  const uint32_t up = before + incl - h;
+  if (up < static_cast<uint32_t>(s.k) && up + h >= static_cast<uint32_t>(s.k)) {
+    found[0] = static_cast<uint32_t>(bin);
+    found[1] = up;
+  }
+  __syncthreads();
+  *bstar = static_cast<int>(found[0]);
+  *above = static_cast<int>(found[1]);
+}
+
+__global__ __launch_bounds__(kTopkThreads) void split_candidates_kernel(SplitArgs a) {
+  __shared__ uint32_t cnt[kTopkWaves], found[2], total, ncand, first;
+  __shared__ uint32_t ck[kSplitCand], ci[kSplitCand];
+  const SplitRow s = split_row(a, blockIdx.y);
+  const int slice = blockIdx.x, tid = threadIdx.x, base = slice * kSliceKeys + 4 * tid;
+  if (slice * kSliceKeys >= s.n) return;
+  float x[4];
+  slice_scores(s, base, x);
+  const SplitScale c = split_scale(s, true);
+  if (tid == 0) total = ncand = 0;
+  int bstar, above;
+  split_boundary(s, cnt, found, &bstar, &above);  // (its barriers order the counters' reset)
+  const int lane = tid & 63;
+  const uint64_t lt_mask = (1ull << lane) - 1ull;
+  uint32_t mine = 0;  // the wave's keys above B*
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint32_t key = split_key(c, x[e], base + e < s.n);
+    const int b = key != 0u ? split_bin(c, key) : -1;
+    mine += static_cast<uint32_t>(__popcll(ballot64(b > bstar)));
+    const uint64_t in_b = ballot64(b == bstar);
+    if (in_b == 0ull) continue;
+    uint32_t at = 0;
+    if (lane == 0) at = atomicAdd(&ncand, static_cast<uint32_t>(__popcll(in_b)));
+    at = __shfl(at, 0, kWave) + static_cast<uint32_t>(__popcll(in_b & lt_mask));
+    if (b == bstar && at < kSplitCand) {
+      ck[at] = key;
+      ci[at] = static_cast<uint32_t>(base + e);
+    }
+  }
+  if (lane == 0 && mine) atomicAdd(&total, mine);
+  __syncthreads();
+  if (tid == 0) {
+    s.above[slice] = total;
+    first = ncand ? atomicAdd(&s.ncand[0], ncand) : 0u;
+  }
+  __syncthreads();
+  for (uint32_t i = tid; i < min(ncand, static_cast<uint32_t>(kSplitCand)); i += kTopkThreads)
+    if (first + i < kSplitCand) {
+      s.cand_key[first + i] = ck[i];
+      s.cand_idx[first + i] = ci[i];
+    }
+}
+
+__global__ __launch_bounds__(kTopkThreads) void split_compact_kernel(SplitArgs a) {
+  __shared__ uint32_t cnt[kTopkWaves], found[2], kth[2], offset;
+  __shared__ uint32_t ck[kSplitCand], ci[kSplitCand], rk[kSplitCand];
+  __shared__ float red[kTopkWaves];
+  const int r = blockIdx.y;
+  const SplitRow s = split_row(a, r);
+  const int slice = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int base = slice * kSliceKeys + 4 * tid;
+  int32_t* oi = a.indices + static_cast<int64_t>(r) * a.cap;
+  uint8_t* ov = a.valid + static_cast<int64_t>(r) * a.cap;
+  float* ow = a.weights + static_cast<int64_t>(r) * a.cap;
+  for (int j = s.k + slice * kTopkThreads + tid; j < a.cap; j += a.slices * kTopkThreads) {
+    oi[j] = 0;
+    ov[j] = 0;
+    ow[j] = 0.0f;
+  }
+  const uint32_t m = slice * kSliceKeys < s.n ? s.ncand[0] : kSplitCand + 1u;
+  if (m > kSplitCand) return;  // an empty slice, or a row that the last launch does alone
+  float x[4];
+  slice_scores(s, base, x);
+  const SplitScale c = split_scale(s, true);
+  if (tid < static_cast<int>(m)) {
+    ck[tid] = s.cand_key[tid];
+    ci[tid] = s.cand_idx[tid];
+    rk[tid] = 0;
+  }
+  if (tid == 0) offset = 0;
+  int bstar, above;
+  split_boundary(s, cnt, found, &bstar, &above);
+  const int need = s.k - above;  // keys of B* that are selected, >= 1
+  // the candidates' ranks in (key desc, index asc) order: the m x m comparisons over all waves,
+  // wave w comparing the 64 candidates of block w % nb with part w / nb of the list
+  const int nb = (static_cast<int>(m) + kWave - 1) / kWave, parts = kTopkWaves / nb;
+  const int cand = (w % nb) * kWave + lane, part = w / nb;
+  if (part < parts && cand < static_cast<int>(m)) {
+    const int each = (static_cast<int>(m) + parts - 1) / parts;
+    const int u1 = min(static_cast<int>(m), (part + 1) * each);
+    const uint32_t mk = ck[cand], mi = ci[cand];
+    uint32_t rank = 0;
+#pragma unroll 4
+    for (int u = part * each; u < u1; ++u) rank += (ck[u] > mk || (ck[u] == mk && ci[u] < mi)) ? 1u : 0u;
+    if (rank) atomicAdd(&rk[cand], rank);
+  }
+  __syncthreads();
+  bool lower = false;  // a selected candidate of an earlier slice
+  if (tid < static_cast<int>(m)) {
+    const int rank = static_cast<int>(rk[tid]);
+    if (rank == need - 1) {
+      kth[0] = ck[tid];
+      kth[1] = ci[tid];
+    }
+    lower = rank < need && ci[tid] < static_cast<uint32_t>(slice * kSliceKeys);
+  }
+  uint32_t before = static_cast<uint32_t>(__popcll(ballot64(lower)));
+  if (w == 0) {
+    uint32_t up = 0;
+    for (int i = lane; i < slice; i += kWave) up += s.above[i];
+#pragma unroll
+    for (int off = kWave / 2; off >= 1; off >>= 1) up += static_cast<uint32_t>(__shfl_xor(static_cast<int>(up), off, kWave));
+    before += up;
+  }
+  if (lane == 0 && before) atomicAdd(&offset, before);
+  __syncthreads();
+  // selected keys of the slice, in index order from the slice's offset
+  bool sel[4];
+  uint32_t key[4];
+  uint32_t mine = 0;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    key[e] = split_key(c, x[e], base + e < s.n);
+    sel[e] = key[e] > kth[0] || (key[e] == kth[0] && static_cast<uint32_t>(base + e) <= kth[1]);
+    mine += sel[e] ? 1u : 0u;
+  }
+  uint32_t incl = mine;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const uint32_t u = __shfl_up(incl, o, kWave);
+    if (lane >= o) incl += u;
+  }
+  if (lane == 63) cnt[w] = incl;  // (cnt was last read before the barrier above)
+  __syncthreads();
+  uint32_t pos = offset + incl - mine;
+  for (int q = 0; q < w; ++q) pos += cnt[q];
+  float msum = 0.0f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (sel[e]) {
+      const float wt = c.weighted ? key_weight(key[e]) : NAN;
+      if (pos < static_cast<uint32_t>(s.k)) {
+        oi[pos] = base + e;
+        ov[pos] = 1;
+        ow[pos] = wt;
+        msum += wt;
+      }
+      ++pos;
+    }
+  msum = wave_sum(msum);
+  if (lane == 0) red[w] = msum;
+  __syncthreads();
+  if (tid == 0) {
+    float t = 0.0f;
+    for (int i = 0; i < kTopkWaves; ++i) t += red[i];
+    s.pmass[slice] = t;
+  }
+}
+
+__global__ __launch_bounds__(kTopkThreads) void split_finish_kernel(SplitArgs a) {
+  __shared__ TopkShared sh;
+  const int r = blockIdx.y;
+  const SplitRow s = split_row(a, r);
+  const int slice = blockIdx.x, tid = threadIdx.x;
+  if (s.n > 0 && s.ncand[0] > kSplitCand) {
+    if (slice == 0)
+      topk_global_row(sh, r, s.n, a.scores, a.stride, a.fraction, a.cap, a.indices, a.valid, a.mass, a.weights, a.counts,
+                      a.nonfinite);
+    return;
+  }
+  const int slices = (s.n + kSliceKeys - 1) / kSliceKeys;
+  float S = 0.0f;
+  for (int i = 0; i < slices; ++i) S += s.pmass[i];
+  float* ow = a.weights + static_cast<int64_t>(r) * a.cap;
+  for (int j = slice * kTopkThreads + tid; j < s.k; j += a.slices * kTopkThreads) ow[j] = ow[j] / S;
+  if (slice == 0 && tid < kWave) {
+    const SplitScale c = split_scale(s, false);
+    if (tid == 0) {
+      a.mass[r] = S;
+      if (a.counts) a.counts[r] = s.k;
+      if (a.nonfinite) a.nonfinite[r] = static_cast<int32_t>(s.n > 0 ? c.nonfinite : 0u);
+    }
+  }
+}
+
 struct EligibleCand {
   const uint8_t* elig;
   int last;  // excluded index (forced), or -1
@@ -1069,6 +1531,48 @@ extern "C" int32_t fl_decode_topk(const float* scores, int64_t scores_stride, in
     hipLaunchKernelGGL(decode_topk_kernel, grid, block, 0, st, scores, scores_stride, n_keys, rows_per_count,
                        fraction, capacity, indices, valid, mass, weights, counts, nonfinite);
   FL_LAUNCH_CHECK("fl_decode_topk");
+  return FL_OK;
+}
+
+extern "C" size_t fl_decode_topk_workspace(int32_t rows, int64_t scores_stride, double fraction) {
+  using namespace fl;
+  if (rows <= 0 || scores_stride <= 0 || select_merge_fits(scores_stride, fraction)) return 0;
+  return static_cast<size_t>(rows) * split_words(split_slices(scores_stride)) * sizeof(uint32_t);
+}
+
+extern "C" int32_t fl_decode_topk_long(const float* scores, int64_t scores_stride, int32_t rows, const int32_t* n_keys,
+                                       const int32_t* more_keys, int32_t plus_keys, int32_t rows_per_count,
+                                       double fraction, int32_t capacity, int32_t* indices, uint8_t* valid,
+                                       float* mass, float* weights, int32_t* counts, int32_t* nonfinite,
+                                       void* workspace, size_t workspace_bytes, void* stream) {
+  using namespace fl;
+  clear_error();
+  FL_REQUIRE(scores && n_keys && indices && valid && mass && weights && workspace, "fl_decode_topk_long: null pointer");
+  FL_REQUIRE(rows >= 0 && rows_per_count > 0 && capacity > 0, "fl_decode_topk_long: bad rows/rows_per_count/capacity");
+  FL_REQUIRE(fraction > 0.0 && fraction <= 1.0, "fl_decode_topk_long: fraction must be in (0, 1]");
+  FL_REQUIRE(scores_stride > 0 && scores_stride <= 0x7FFFFFFF, "fl_decode_topk_long: bad stride");
+  FL_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 16 == 0, "fl_decode_topk_long: workspace must be 16-byte aligned");
+  const int slices = split_slices(scores_stride);
+  FL_REQUIRE(workspace_bytes >= static_cast<size_t>(std::max(rows, 1)) * split_words(slices) * sizeof(uint32_t),
+             "fl_decode_topk_long: workspace too small");
+  FL_REQUIRE(rows <= 65535, "fl_decode_topk_long: at most 65535 rows");
+  if (rows == 0) return FL_OK;
+  const SplitArgs a{scores, scores_stride, n_keys, more_keys, plus_keys, rows_per_count, fraction, capacity, slices,
+                    indices, valid, mass, weights, counts, nonfinite, static_cast<uint32_t*>(workspace)};
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const dim3 grid(slices, rows), block(kTopkThreads);
+  hipLaunchKernelGGL(split_extremes_kernel, grid, block, 0, st, a);
+  FL_LAUNCH_CHECK("fl_decode_topk_long(extremes)");
+  hipLaunchKernelGGL(split_normaliser_kernel, dim3(kTopkWaves, rows), block, 0, st, a);
+  FL_LAUNCH_CHECK("fl_decode_topk_long(normaliser)");
+  hipLaunchKernelGGL(split_histogram_kernel, grid, block, 0, st, a);
+  FL_LAUNCH_CHECK("fl_decode_topk_long(histogram)");
+  hipLaunchKernelGGL(split_candidates_kernel, grid, block, 0, st, a);
+  FL_LAUNCH_CHECK("fl_decode_topk_long(candidates)");
+  hipLaunchKernelGGL(split_compact_kernel, grid, block, 0, st, a);
+  FL_LAUNCH_CHECK("fl_decode_topk_long(compact)");
+  hipLaunchKernelGGL(split_finish_kernel, grid, block, 0, st, a);
+  FL_LAUNCH_CHECK("fl_decode_topk_long(finish)");
   return FL_OK;
 }
 

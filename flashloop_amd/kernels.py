@@ -220,9 +220,11 @@ def decode_capacity(keys: int, fraction: float) -> int:
 
 
 def decode_topk(logits: torch.Tensor, n_keys: torch.Tensor, fraction: float, capacity: int,
-                rows_per_count: int = 1, validate: bool = False, nonfinite: torch.Tensor | None = None):
+                rows_per_count: int = 1, validate: bool = False, nonfinite: torch.Tensor | None = None,
+                more_keys: torch.Tensor | None = None, plus_keys: int = 0):
     """Top-k of each logits row by fp32 softmax weight (ties to the lower index) ->
-    (indices i32, valid u8, mass f32, weights f32, counts i32).
+    (indices i32, valid u8, mass f32, weights f32, counts i32).  A row holds
+    ``n_keys (+ more_keys) + plus_keys`` scores.
 
     ``nonfinite`` (optional i32 [rows]) receives each row's count of NaN/inf scores.
     ``validate=True`` waits for the kernel and raises ``ValueError`` when a row holds one
@@ -243,11 +245,28 @@ def decode_topk(logits: torch.Tensor, n_keys: torch.Tensor, fraction: float, cap
         _require(nonfinite, torch.int32, "nonfinite")
         if nonfinite.numel() < rows:
             raise ValueError("nonfinite needs one entry per row")
-    rc = load().fl_decode_topk(logits.data_ptr(), logits.stride(0), rows, n_keys.data_ptr(), rows_per_count,
-                               float(fraction), capacity, idx.data_ptr(), valid.data_ptr(), mass.data_ptr(),
-                               w.data_ptr(), counts.data_ptr(), nonfinite.data_ptr() if nonfinite is not None else None,
-                               _stream())
-    check(rc, "fl_decode_topk")
+    if more_keys is not None:
+        _require(more_keys, torch.int32, "more_keys")
+        if more_keys.numel() != n_keys.numel():
+            raise ValueError("more_keys needs the entries of n_keys")
+    lib = load()
+    ws_bytes = lib.fl_decode_topk_workspace(rows, logits.stride(0), float(fraction))
+    if ws_bytes and rows <= 65535:  # a row over several workgroups
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        rc = lib.fl_decode_topk_long(logits.data_ptr(), logits.stride(0), rows, n_keys.data_ptr(), _p(more_keys),
+                                     int(plus_keys), rows_per_count, float(fraction), capacity, idx.data_ptr(),
+                                     valid.data_ptr(), mass.data_ptr(), w.data_ptr(), counts.data_ptr(), _p(nonfinite),
+                                     ws.data_ptr(), ws_bytes, _stream())
+        check(rc, "fl_decode_topk_long")
+    else:
+        if more_keys is not None:
+            n_keys = n_keys + more_keys
+        if plus_keys:
+            n_keys = n_keys + int(plus_keys)
+        rc = lib.fl_decode_topk(logits.data_ptr(), logits.stride(0), rows, n_keys.data_ptr(), rows_per_count,
+                                float(fraction), capacity, idx.data_ptr(), valid.data_ptr(), mass.data_ptr(),
+                                w.data_ptr(), counts.data_ptr(), _p(nonfinite), _stream())
+        check(rc, "fl_decode_topk")
     if validate:
         bad = int((nonfinite[:rows] != 0).sum().item())
         if bad:

@@ -267,6 +267,21 @@ int32_t fl_decode_topk(const float* scores, int64_t scores_stride, int32_t rows,
                        float* weights, int32_t* counts, int32_t* nonfinite, void* stream);
 
 /*
+ * fl_decode_topk for rows (or selections) beyond the register-resident kernel: the same
+ * selection, each row divided over several workgroups.  A row's key count is
+ * n_keys[i] + more_keys[i] (nullable) + plus_keys, i = r / rows_per_count.  Workspace
+ * (16-byte aligned): fl_decode_topk_workspace bytes, 0 where fl_decode_topk itself is the
+ * faster call (logits rows of up to 36864 keys with up to 8192 selected).
+ */
+size_t fl_decode_topk_workspace(int32_t rows, int64_t scores_stride, double fraction);
+int32_t fl_decode_topk_long(const float* scores, int64_t scores_stride, int32_t rows,
+                            const int32_t* n_keys, const int32_t* more_keys, int32_t plus_keys,
+                            int32_t rows_per_count, double fraction, int32_t capacity,
+                            int32_t* indices, uint8_t* valid, float* mass, float* weights,
+                            int32_t* counts, int32_t* nonfinite, void* workspace,
+                            size_t workspace_bytes, void* stream);
+
+/*
  * J2 + J3 -- the loop-2 dense read and its key selection in two launches instead of
  * three: fl_decode_attn_dense(view, loop, ..., logits required) followed by
  * fl_decode_topk on the logits rows with n = packed_tokens[b] + tail_tokens[b] + 1 keys

@@ -1,0 +1,65 @@
+"""fl_decode_topk_long (a row over several workgroups) against fl_decode_topk (one workgroup
+per row): the same keys, counts and non-finite counts bit for bit; the masses sum in
+another order (at most k fp32 additions of positive terms: k * 2^-24 relative)."""
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from flashloop_amd import _lib, kernels  # noqa: E402
+
+DEV = "cuda"
+
+
+def _rows(kind, rows, stride, gen):
+    x = torch.randn(rows, stride, generator=gen, device=DEV)
+    if kind == "peaked":
+        x *= 40.0
+    elif kind == "tied":
+        x = (x * 4.0).round() / 4.0
+    elif kind == "equal":
+        x = torch.full_like(x, 0.25)
+    elif kind == "mixed":  # NaN, infinities, only -inf and signed zeros, among ordinary rows
+        x[0, stride // 3] = float("nan")
+        x[1, 7] = float("inf")
+        x[2] = float("-inf")
+        x[3, ::2] = float("-inf")
+        x[4] = torch.where(torch.arange(stride, device=DEV) % 2 == 0, 0.0, -0.0)
+    return x
+
+
+@pytest.mark.parametrize("kind", ["normal", "peaked", "tied", "equal", "mixed"])
+@pytest.mark.parametrize("stride,fraction", [(36865, 0.1), (40961, 0.001), (70144, 0.1), (4096, 1.0), (12289, 0.9)])
+def test_long_rows_equal_one_workgroup_per_row(kind, stride, fraction):
+    print(f"case: long top-k {kind} stride={stride} fraction={fraction}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(95)
+    rows = 7
+    x = _rows(kind, rows, stride, gen)
+    n = torch.tensor([stride, stride - 1, stride, stride - 4096, min(stride, 4097), 5, 0], dtype=torch.int32, device=DEV)
+    cap = kernels.decode_capacity(stride, fraction)
+    lib = _lib.load()
+    st = torch.cuda.current_stream().cuda_stream
+
+    def outputs():
+        return [torch.full((rows, cap), 77, dtype=torch.int32, device=DEV), torch.full((rows, cap), 77, dtype=torch.uint8, device=DEV),
+                torch.zeros(rows, device=DEV), torch.full((rows, cap), 77.0, device=DEV),
+                torch.zeros(rows, dtype=torch.int32, device=DEV), torch.zeros(rows, dtype=torch.int32, device=DEV)]
+
+    want, got = outputs(), outputs()
+    _lib.check(lib.fl_decode_topk(x.data_ptr(), stride, rows, n.data_ptr(), 1, fraction, cap, *(t.data_ptr() for t in want), st),
+               "fl_decode_topk")
+    # the workspace function answers 0 for rows that the other call takes; the slices do not mind
+    nbytes = rows * 4 * (6 * (-(-stride // 4096)) + 16 + 1024 + 4 + 2048 + 4)
+    assert lib.fl_decode_topk_workspace(rows, stride, fraction) <= nbytes
+    ws = torch.full((nbytes,), 0xA5, dtype=torch.uint8, device=DEV)
+    part = torch.full_like(n, 3)
+    _lib.check(lib.fl_decode_topk_long(x.data_ptr(), stride, rows, (n - 4).data_ptr(), part.data_ptr(), 1, 1, fraction, cap,
+                                       *(t.data_ptr() for t in got), ws.data_ptr(), nbytes, st), "fl_decode_topk_long")
+    for name, a, b in zip(("indices", "valid", "counts", "nonfinite"), (got[0], got[1], got[4], got[5]), (want[0], want[1], want[4], want[5])):
+        assert torch.equal(a, b), f"{name} differ in rows {(a != b).reshape(rows, -1).any(1).nonzero().flatten().tolist()}"
+    for a, b in ((got[2], want[2]), (got[3], want[3])):
+        a, b = a.double().cpu().numpy(), b.double().cpu().numpy()
+        assert np.array_equal(np.isnan(a), np.isnan(b))
+        assert np.all(np.isnan(b) | (np.abs(a - b) <= 2 * cap * 2.0 ** -24 * np.abs(b)))
