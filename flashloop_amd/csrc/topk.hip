@@ -1392,13 +1392,26 @@ struct EligibleCand {
   __device__ bool operator()(int i) const { return i != last && (elig == nullptr || elig[i] != 0); }
 };
 
+// A flag that is written, not only set (the callers with a forced last token, or without an
+// eligibility mask): workgroup 0 looks at every row's last token.
+__device__ __forceinline__ void tokens_flag(const uint8_t* eligible, int tokens, int32_t* flag) {
+  if (blockIdx.x != 0 || threadIdx.x >= kWave) return;
+  bool bad = false;
+  if (eligible != nullptr)
+    for (int b = threadIdx.x; b < static_cast<int>(gridDim.x); b += kWave)
+      bad |= eligible[static_cast<int64_t>(b) * tokens + tokens - 1] == 0;
+  const uint64_t any = ballot64(bad);
+  if (threadIdx.x == 0) *flag = any != 0ull;
+}
+
 __global__ __launch_bounds__(kTopkThreads) void select_tokens_kernel(const float* scores, int tokens, double fraction,
                                                                      const uint8_t* eligible, int force_last,
                                                                      uint8_t* mask, int32_t* positions,
-                                                                     int32_t* counts, int32_t* error_flag) {
+                                                                     int32_t* counts, int32_t* error_flag, int own) {
   __shared__ TopkShared sh;
   __shared__ int n_elig_sh;
   const int b = blockIdx.x;
+  if (own) tokens_flag(eligible, tokens, error_flag);
   const float* x = scores + static_cast<int64_t>(b) * tokens;
   const uint8_t* el = eligible ? eligible + static_cast<int64_t>(b) * tokens : nullptr;
   uint8_t* om = mask + static_cast<int64_t>(b) * tokens;
@@ -1418,7 +1431,7 @@ __global__ __launch_bounds__(kTopkThreads) void select_tokens_kernel(const float
   const int n_elig = n_elig_sh;
   if (n_elig == 0 || (forced && el != nullptr && el[last] == 0)) {
     if (threadIdx.x == 0) {
-      if (error_flag) atomicExch(error_flag, 1);
+      if (error_flag && !own) atomicExch(error_flag, 1);
       if (counts) counts[b] = 0;
     }
     return;
@@ -1466,6 +1479,159 @@ __global__ __launch_bounds__(kTopkThreads) void select_tokens_kernel(const float
     }
   }
   if (threadIdx.x == 0 && counts) counts[b] = selected + (forced ? 1 : 0);
+}
+
+
+// The same selection for rows of at most 1024 * PER tokens: thread t holds tokens t * PER .. of the
+// row in registers, so the radix passes (three digits of 11, 11 and 10 bits) read LDS only, and
+// two prefix sums over the threads give the ranks of the equal keys and the positions in index
+// order.  The one-workgroup kernel above re-reads the row in each pass and walks it twice with
+// three barriers per 1024 tokens: 8192 tokens 31 us, here 13.
+template <int PER>
+__global__ __launch_bounds__(kTopkThreads) void select_tokens_resident_kernel(const float* scores, int tokens,
+                                                                              double fraction, const uint8_t* eligible,
+                                                                              int force_last, uint8_t* mask,
+                                                                              int32_t* positions, int32_t* counts,
+                                                                              int32_t* error_flag, int own) {
+  constexpr int kDigits = 2048;
+  __shared__ uint32_t hist[kDigits];
+  __shared__ uint32_t cnt[kTopkWaves], found[2];
+  const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6, last = tokens - 1;
+  if (own) tokens_flag(eligible, tokens, error_flag);
+  const float* x = scores + static_cast<int64_t>(b) * tokens;
+  const uint8_t* el = eligible ? eligible + static_cast<int64_t>(b) * tokens : nullptr;
+  uint8_t* om = mask + static_cast<int64_t>(b) * tokens;
+  int32_t* op = positions ? positions + static_cast<int64_t>(b) * tokens : nullptr;
+  const bool forced = force_last != 0;
+  const int t0 = tid * PER;
+  // exclusive prefix of v over the threads; *total the sum
+  const auto prefix = [&](uint32_t v, uint32_t* total) __attribute__((always_inline)) {
+    uint32_t incl = v;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const uint32_t u = __shfl_up(incl, o, kWave);
+      if (lane >= o) incl += u;
+    }
+    __syncthreads();
+    if (lane == 63) cnt[w] = incl;
+    __syncthreads();
+    uint32_t before = 0, sum = 0;
+#pragma unroll
+    for (int q = 0; q < kTopkWaves; ++q) {
+      if (q < w) before += cnt[q];
+      sum += cnt[q];
+    }
+    *total = sum;
+    return before + incl - v;
+  };
+  uint32_t key[PER];
+  uint64_t cand = 0;  // bit j: token t0 + j competes (eligible, and not the forced last)
+  uint32_t n_mine = 0;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int i = min(t0 + j, last);
+    key[j] = order_key(x[i]);
+    const bool ok = t0 + j <= last && (el == nullptr || el[i] != 0);
+    n_mine += ok ? 1u : 0u;
+    if (ok && !(forced && i == last)) cand |= 1ull << j;
+  }
+  uint32_t n_elig;
+  prefix(n_mine, &n_elig);
+  if (n_elig == 0 || (forced && el != nullptr && el[last] == 0)) {  // (the same in every thread)
+    for (int i = tid; i < tokens; i += kTopkThreads) {
+      om[i] = 0;
+      if (op) op[i] = 0;
+    }
+    if (tid == 0) {
+      if (error_flag && !own) atomicExch(error_flag, 1);
+      if (counts) counts[b] = 0;
+    }
+    return;
+  }
+  const double want = ceil(static_cast<double>(tokens) * fraction);
+  const int budget = static_cast<int>(want < 1.0 ? 1.0 : want);
+  const int remaining = min(budget, static_cast<int>(n_elig)) - (forced ? 1 : 0);
+  uint64_t sel = 0;
+  if (remaining > 0) {
+    uint32_t pre = 0, pmask = 0, need = static_cast<uint32_t>(remaining);
+#pragma unroll
+    for (int pass = 0; pass < 3; ++pass) {
+      const int shift = pass == 0 ? 21 : (pass == 1 ? 10 : 0), digits = pass == 2 ? 1024 : kDigits;
+      for (int i = tid; i < kDigits; i += kTopkThreads) hist[i] = 0;
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < PER; ++j)
+        if (((cand >> j) & 1ull) && (key[j] & pmask) == pre) atomicAdd(&hist[(key[j] >> shift) & (digits - 1)], 1u);
+      __syncthreads();
+      // thread t: bins 2047 - 2t and 2046 - 2t, from the top
+      const uint32_t h0 = hist[kDigits - 1 - 2 * tid], h1 = hist[kDigits - 2 - 2 * tid];
+      uint32_t total;
+      const uint32_t above = prefix(h0 + h1, &total);
+      if (above < need && above + h0 >= need) {
+        found[0] = static_cast<uint32_t>(kDigits - 1 - 2 * tid);
+        found[1] = above;
+      } else if (above + h0 < need && above + h0 + h1 >= need) {
+        found[0] = static_cast<uint32_t>(kDigits - 2 - 2 * tid);
+        found[1] = above + h0;
+      }
+      __syncthreads();
+      pre |= found[0] << shift;
+      pmask |= static_cast<uint32_t>(digits - 1) << shift;
+      need -= found[1];
+    }
+    uint64_t eq = 0;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const bool c = (cand >> j) & 1ull;
+      if (c && key[j] > pre) sel |= 1ull << j;
+      if (c && key[j] == pre) eq |= 1ull << j;
+    }
+    uint32_t total;
+    uint32_t rank = prefix(static_cast<uint32_t>(__popcll(eq)), &total);
+#pragma unroll
+    for (int j = 0; j < PER; ++j)
+      if ((eq >> j) & 1ull) {
+        if (rank < need) sel |= 1ull << j;
+        ++rank;
+      }
+  }
+  if (forced && last >= t0 && last < t0 + PER) sel |= 1ull << (last - t0);
+  uint32_t total;
+  uint32_t pos = prefix(static_cast<uint32_t>(__popcll(sel)), &total);
+#pragma unroll
+  for (int j = 0; j < PER; ++j)
+    if (t0 + j < tokens) {
+      const bool s = (sel >> j) & 1ull;
+      om[t0 + j] = s ? 1 : 0;
+      if (s && op) op[pos++] = t0 + j;
+    }
+  if (op)
+    for (int i = static_cast<int>(total) + tid; i < tokens; i += kTopkThreads) op[i] = 0;
+  if (tid == 0 && counts) counts[b] = static_cast<int32_t>(total);
+}
+
+int32_t launch_select_tokens(const float* scores, int32_t batch, int32_t tokens, double fraction,
+                             const uint8_t* eligible, int32_t force_last, uint8_t* mask, int32_t* positions,
+                             int32_t* counts, int32_t* error_flag, int own, hipStream_t st) {
+  const dim3 grid(batch), block(kTopkThreads);
+  // the smallest instantiation that holds the row; more registers than 36 keys a thread spill
+  if (tokens <= 4 * kTopkThreads)
+    hipLaunchKernelGGL(select_tokens_resident_kernel<4>, grid, block, 0, st, scores, tokens, fraction, eligible, force_last,
+                       mask, positions, counts, error_flag, own);
+  else if (tokens <= 8 * kTopkThreads)
+    hipLaunchKernelGGL(select_tokens_resident_kernel<8>, grid, block, 0, st, scores, tokens, fraction, eligible, force_last,
+                       mask, positions, counts, error_flag, own);
+  else if (tokens <= 16 * kTopkThreads)
+    hipLaunchKernelGGL(select_tokens_resident_kernel<16>, grid, block, 0, st, scores, tokens, fraction, eligible,
+                       force_last, mask, positions, counts, error_flag, own);
+  else if (tokens <= kPer * kTopkThreads)
+    hipLaunchKernelGGL(select_tokens_resident_kernel<kPer>, grid, block, 0, st, scores, tokens, fraction, eligible,
+                       force_last, mask, positions, counts, error_flag, own);
+  else
+    hipLaunchKernelGGL(select_tokens_kernel, grid, block, 0, st, scores, tokens, fraction, eligible, force_last, mask,
+                       positions, counts, error_flag, own);
+  FL_LAUNCH_CHECK("fl_select_tokens");
+  return FL_OK;
 }
 
 }  // namespace
@@ -1585,8 +1751,19 @@ extern "C" int32_t fl_select_tokens(const float* scores, int32_t batch, int32_t 
   FL_REQUIRE(batch >= 0 && tokens > 0, "fl_select_tokens: scores must have shape [batch, tokens>0]");
   FL_REQUIRE(fraction > 0.0 && fraction <= 1.0, "fl_select_tokens: fraction must satisfy 0 < fraction <= 1");
   if (batch == 0) return FL_OK;
-  hipLaunchKernelGGL(select_tokens_kernel, dim3(batch), dim3(kTopkThreads), 0, static_cast<hipStream_t>(stream),
-                     scores, tokens, fraction, eligible, force_last, mask, positions, counts, error_flag);
-  FL_LAUNCH_CHECK("fl_select_tokens");
-  return FL_OK;
+  return launch_select_tokens(scores, batch, tokens, fraction, eligible, force_last, mask, positions, counts, error_flag,
+                              0, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int32_t fl_select_tokens_status(const float* scores, int32_t batch, int32_t tokens, double fraction,
+                                           const uint8_t* eligible, int32_t force_last, uint8_t* mask,
+                                           int32_t* positions, int32_t* counts, int32_t* error_flag, void* stream) {
+  using namespace fl;
+  clear_error();
+  FL_REQUIRE(scores && mask && error_flag, "fl_select_tokens_status: null scores/mask/error_flag");
+  FL_REQUIRE(batch > 0 && tokens > 0, "fl_select_tokens_status: scores must have shape [batch>0, tokens>0]");
+  FL_REQUIRE(fraction > 0.0 && fraction <= 1.0, "fl_select_tokens_status: fraction must satisfy 0 < fraction <= 1");
+  FL_REQUIRE(force_last || eligible == nullptr, "fl_select_tokens_status: a mask needs the forced last token");
+  return launch_select_tokens(scores, batch, tokens, fraction, eligible, force_last, mask, positions, counts, error_flag,
+                              1, static_cast<hipStream_t>(stream));
 }

@@ -392,9 +392,9 @@ def gather_rows(src: torch.Tensor, index: torch.Tensor, dim: int) -> torch.Tenso
     dst = torch.empty(shape, dtype=src.dtype, device=src.device)
     o, rows, rb, so, sr = _rows_view(src, dim)
     _, _, _, do, dr = _rows_view(dst, dim)
-    err = torch.zeros(1, dtype=torch.int32, device=src.device)
-    rc = load().fl_gather_rows(src.data_ptr(), so, sr, rows, dst.data_ptr(), do, dr, o, rb, index.data_ptr(),
-                               index.numel(), err.data_ptr(), _stream())
+    err = torch.empty(1, dtype=torch.int32, device=src.device)
+    rc = load().fl_move_rows(0, src.data_ptr(), so, sr, dst.data_ptr(), do, dr, rows, o, rb, index.data_ptr(),
+                             index.numel(), err.data_ptr(), _stream())
     check(rc, "fl_gather_rows")
     return dst, err
 
@@ -408,9 +408,9 @@ def scatter_rows_(dst: torch.Tensor, index: torch.Tensor, src: torch.Tensor, dim
     o2, n, rb2, so, sr = _rows_view(src, dim)
     if o2 != o or rb2 != rb or n != index.numel():
         raise ValueError("src shape does not match dst/index")
-    err = torch.zeros(1, dtype=torch.int32, device=dst.device)
-    rc = load().fl_scatter_rows(src.data_ptr(), so, sr, dst.data_ptr(), do, dr, rows, o, rb, index.data_ptr(),
-                                index.numel(), err.data_ptr(), _stream())
+    err = torch.empty(1, dtype=torch.int32, device=dst.device)
+    rc = load().fl_move_rows(1, src.data_ptr(), so, sr, dst.data_ptr(), do, dr, rows, o, rb, index.data_ptr(),
+                             index.numel(), err.data_ptr(), _stream())
     check(rc, "fl_scatter_rows")
     return dst, err
 
@@ -440,15 +440,18 @@ def select_tokens(scores: torch.Tensor, fraction: float, eligible: torch.Tensor 
     if eligible is not None:
         if eligible.shape != scores.shape:
             raise ValueError("eligible must match scores")
-        el = eligible.to(torch.uint8).contiguous()
+        el = (eligible.view(torch.uint8) if eligible.dtype == torch.bool else eligible.to(torch.uint8)).contiguous()
     mask = torch.empty(b, t, dtype=torch.uint8, device=scores.device)
     pos = torch.empty(b, t, dtype=torch.int32, device=scores.device)
     counts = torch.empty(b, dtype=torch.int32, device=scores.device)
-    err = torch.zeros(1, dtype=torch.int32, device=scores.device)
-    rc = load().fl_select_tokens(scores.data_ptr(), b, t, float(fraction), _p(el), int(bool(force_last_token)),
-                                 mask.data_ptr(), pos.data_ptr(), counts.data_ptr(), err.data_ptr(), _stream())
+    status = b > 0 and (bool(force_last_token) or el is None)  # the kernel writes the flag
+    err = (torch.empty if status else torch.zeros)(1, dtype=torch.int32, device=scores.device)
+    lib = load()
+    call = lib.fl_select_tokens_status if status else lib.fl_select_tokens
+    rc = call(scores.data_ptr(), b, t, float(fraction), _p(el), int(bool(force_last_token)), mask.data_ptr(),
+              pos.data_ptr(), counts.data_ptr(), err.data_ptr(), _stream())
     check(rc, "fl_select_tokens")
-    return mask.bool(), pos, counts, err
+    return mask.view(torch.bool), pos, counts, err
 
 
 # ---------------------------------------------------------------------------- decode-step model ops

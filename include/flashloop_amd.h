@@ -389,6 +389,12 @@ int32_t fl_scatter_rows(const void* src, int64_t src_outer_stride, int64_t src_r
                         int64_t dst_rows, int64_t outer, int64_t row_bytes,
                         const int32_t* index, int64_t n_index, int32_t* error_flag,
                         void* stream);
+/* fl_gather_rows (scatter = 0) or fl_scatter_rows (scatter = 1) with a flag that is written, 0
+ * or 1, not only set on an error; indexed_rows: the rows of the tensor that index addresses. */
+int32_t fl_move_rows(int32_t scatter, const void* src, int64_t src_outer_stride, int64_t src_row_stride,
+                     void* dst, int64_t dst_outer_stride, int64_t dst_row_stride, int64_t indexed_rows,
+                     int64_t outer, int64_t row_bytes, const int32_t* index, int64_t n_index,
+                     int32_t* error_flag, void* stream);
 
 /*
  * J4 -- loop-boundary token score and selection.
@@ -410,6 +416,12 @@ int32_t fl_select_tokens(const float* scores, int32_t batch, int32_t tokens, dou
                          const uint8_t* eligible, int32_t force_last, uint8_t* mask,
                          int32_t* positions, int32_t* counts, int32_t* error_flag,
                          void* stream);
+/* fl_select_tokens with a flag that is written, 0 or 1, not only set on an error (with
+ * force_last, or without an eligibility mask). */
+int32_t fl_select_tokens_status(const float* scores, int32_t batch, int32_t tokens, double fraction,
+                                const uint8_t* eligible, int32_t force_last, uint8_t* mask,
+                                int32_t* positions, int32_t* counts, int32_t* error_flag,
+                                void* stream);
 
 /*
  * Decode-step model ops -- the per-layer work around the readers in one decode step

@@ -1,0 +1,81 @@
+"""Row movement and token selection at the sizes where their kernels change."""
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from flashloop_amd import kernels  # noqa: E402
+from oracle import tokens as OT  # noqa: E402
+
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("outer,rows,width,n", [(1, 1, 2, 1), (3, 700, 6, 300), (16, 300, 128, 257), (2, 5000, 8, 4097),
+                                                (1, 40, 5000, 40)])
+def test_rows_move_and_flag(outer, rows, width, n):
+    """Rows of 4 bytes to 10 KB (4- and 16-byte pieces), workgroups that cross rows, and the flag:
+    written 0 over whatever the memory held, 1 where an index is out of range, whose row stays."""
+    print(f"case: rows outer={outer} rows={rows} width={width} n={n}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(96)
+    src = torch.randint(0, 1 << 15, (outer, rows, width), generator=g, device=DEV).to(torch.int16)
+    pos = torch.randperm(rows, generator=g, device=DEV)[:n].int()
+    got, err = kernels.gather_rows(src, pos, 1)
+    assert torch.equal(got, src.index_select(1, pos.long())) and int(err) == 0
+    new = torch.randint(0, 1 << 15, (outer, pos.numel(), width), generator=g, device=DEV).to(torch.int16)
+    dst, err = kernels.scatter_rows_(src.clone(), pos, new, 1)
+    assert torch.equal(dst, src.index_copy(1, pos.long(), new)) and int(err) == 0
+    for bad in (-1, rows):
+        wrong = pos.clone()
+        wrong[-1] = bad
+        dst, err = kernels.scatter_rows_(src.clone(), wrong, new, 1)
+        assert torch.equal(dst, src.index_copy(1, pos[:-1].long(), new[:, :-1])) and int(err) == 1
+        _, err = kernels.gather_rows(src, wrong, 1)
+        assert int(err) == 1
+
+
+def _scores(kind, b, t, gen):
+    x = torch.randn(b, t, generator=gen, device=DEV)
+    if kind == "tied":
+        x = (x * 3).round() / 3
+    elif kind == "zeros":
+        x = torch.where(x > 0, 0.0, -0.0)
+    return x
+
+
+@pytest.mark.parametrize("kind", ["normal", "tied", "zeros"])
+@pytest.mark.parametrize("b,t", [(1, 1), (3, 5), (2, 4096), (2, 4097), (1, 8193), (1, 16385), (1, 36864), (1, 36865)])
+def test_token_selection_at_instantiation_edges(kind, b, t):
+    """Every instantiation's smallest and largest row, ties, signed zeros, eligibility and the
+    forced last token, against the oracle's selection."""
+    print(f"case: token selection {kind} b={b} t={t}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(97)
+    x = _scores(kind, b, t, gen)
+    el = torch.rand(b, t, generator=gen, device=DEV) < 0.4
+    el[:, -1] = True
+    for fraction, eligible in ((0.25, None), (1.0, None), (0.1, el), (0.9, el)):
+        mask, pos, counts, err = kernels.select_tokens(x, fraction, eligible=eligible)
+        want = OT.select_active_mask(x.cpu().numpy(), fraction, eligible=None if eligible is None else eligible.cpu().numpy())
+        assert np.array_equal(mask.cpu().numpy(), want) and int(err) == 0
+        for i in range(b):
+            on = np.nonzero(want[i])[0]
+            assert int(counts[i]) == len(on)
+            assert np.array_equal(pos[i].cpu().numpy(), np.concatenate([on, np.zeros(t - len(on), on.dtype)]))
+    if b > 1:  # a row whose last token is not eligible is left empty; the others are selected
+        el[1, -1] = False
+        mask, pos, counts, err = kernels.select_tokens(x, 0.25, eligible=el)
+        assert int(err) == 1 and int(counts[1]) == 0 and not bool(mask[1].any()) and not bool(pos[1].any())
+        want = OT.select_active_mask(x[:1].cpu().numpy(), 0.25, eligible=el[:1].cpu().numpy())
+        assert np.array_equal(mask[:1].cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("rows,dim", [(1, 8), (5, 2048), (3, 2056), (7, 100), (2, 16384)])
+def test_hidden_score_widths(rows, dim):
+    print(f"case: hidden score rows={rows} dim={dim}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(98)
+    a, b = (torch.randn(rows, dim, generator=g, device=DEV).bfloat16() for _ in range(2))
+    got = kernels.hidden_delta_score(a, b).double()
+    want = (a.double() - b.double()).norm(dim=-1) / a.double().norm(dim=-1)
+    # two fp32 sums of dim positive terms (halved by the root), a division and two roots
+    assert bool(((got - want).abs() <= (dim + 8) * 2.0 ** -24 * want).all())
