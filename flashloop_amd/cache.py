@@ -51,9 +51,9 @@ class CrossLoopKVLayer:
     residual_length = 64
     group_size = GROUP
 
-    def __init__(self, geometry: LayerGeometry, device, *, _clear: bool = True) -> None:
-        # _clear=False: the buffers are left to fl_cache_prepare and fl_pack_kv_groups, which
-        # between them write every byte (from_prefill)
+    def __init__(self, geometry: LayerGeometry, device, *, _buffers: dict | None = None) -> None:
+        # _buffers: what _fixed_buffers returned, left to fl_cache_prepare and fl_pack_kv_groups,
+        # which between them write every byte (from_prefill)
         g = geometry
         if g.token_capacity % GROUP:
             raise ValueError("token_capacity must be a multiple of 64")
@@ -63,34 +63,24 @@ class CrossLoopKVLayer:
             # the readers read row 0 of a stream in place of an absent row (then mask it)
             raise ValueError("every stream needs a row capacity of at least 1")
         self.geometry = g
-        self.device = torch.device(device)
+        self.device = dev = torch.device(device)
         rows = g.batch * g.heads
-        dev = self.device
-        # one 128-byte line per token and stream: K codes in bytes 0..63, V codes in 64..127
-        new = torch.zeros if _clear else torch.empty
-        self.codes = [new(rows, g.row_capacity[s], 2 * (HEAD_DIM // 2), dtype=torch.uint8, device=dev) for s in range(4)]
-        self.key_codes = [c[..., : HEAD_DIM // 2] for c in self.codes]
-        self.value_codes = [c[..., HEAD_DIM // 2 :] for c in self.codes]
-        self.key_meta = [new(rows, g.token_capacity // GROUP, HEAD_DIM, 2, dtype=torch.float32, device=dev) for _ in range(4)]
-        self.value_meta = [new(rows, g.row_capacity[s], 2, 2, dtype=torch.float32, device=dev) for s in range(4)]
-        # the V metadata of all four streams again, one 64-byte record per logical token
-        # ([half][stream][scale, min]) for the readers of selected tokens
-        self.value_meta_token = new(rows, g.token_capacity, 2, 4, 2, dtype=torch.float32, device=dev)
-        # fp16 copy of the K metadata, streamed by the readers of selected tokens
-        self.key_meta_half = [new(rows, g.token_capacity // GROUP, HEAD_DIM, 2, dtype=torch.float16, device=dev)
-                              for _ in range(4)]
-        self.value_meta_half = [new(rows, g.row_capacity[s], 2, 2, dtype=torch.float16, device=dev) for s in range(4)]
-        self.rank = [new(g.batch, g.token_capacity, dtype=torch.int32, device=dev) for _ in range(2)]
-        if _clear:
+        new = torch.zeros if _buffers is None else torch.empty
+        fixed = _buffers or self._fixed_buffers(g.batch, g.heads, g.token_capacity, g.tail_capacity, dev, new)
+        for name, x in fixed.items():
+            setattr(self, name, x)
+        if _buffers is None:
             for r in self.rank:
                 r.fill_(-1)
-        self.tail_key = [new(rows, g.tail_capacity, HEAD_DIM, dtype=torch.bfloat16, device=dev) for _ in range(4)]
-        self.tail_value = [new(rows, g.tail_capacity, HEAD_DIM, dtype=torch.bfloat16, device=dev) for _ in range(4)]
-        # loop-3/4 activity of tail rows (flashloop/cache.py:_tail_active)
-        self.tail_active = [new(g.batch, g.tail_capacity, dtype=torch.uint8, device=dev) for _ in range(2)]
-        self.packed_tokens = new(g.batch, dtype=torch.int32, device=dev)
-        self.tail_tokens = new(g.batch, dtype=torch.int32, device=dev)
-        self.late_rows = new(2, g.batch, dtype=torch.int32, device=dev)  # rows used in streams 2/3
+        # streams 2/3 hold the rows that loops 3/4 keep; one 128-byte line per token and stream:
+        # K codes in bytes 0..63, V codes in 64..127
+        for s in (2, 3):
+            n = g.row_capacity[s]
+            self.codes.append(new(rows, n, 2 * (HEAD_DIM // 2), dtype=torch.uint8, device=dev))
+            self.value_meta.append(new(rows, n, 2, 2, dtype=torch.float32, device=dev))
+            self.value_meta_half.append(new(rows, n, 2, 2, dtype=torch.float16, device=dev))
+        self.key_codes = [c[..., : HEAD_DIM // 2] for c in self.codes]
+        self.value_codes = [c[..., HEAD_DIM // 2 :] for c in self.codes]
         # host mirrors (no device sync on the decode path)
         self.packed_host = [0] * g.batch
         self.tail_host = [0] * g.batch
@@ -102,6 +92,32 @@ class CrossLoopKVLayer:
         self._late_stale = False
         self._view: FlCacheView | None = None
         self.workspace = kernels.Workspace()
+
+    @staticmethod
+    def _fixed_buffers(batch: int, heads: int, cap: int, tail: int, dev, new) -> dict:
+        """The layer's buffers whose size does not follow from the rows loops 3/4 keep (of the
+        lists per stream, streams 0 and 1), made by ``new`` (``torch.zeros`` or ``torch.empty``)."""
+        rows, groups = batch * heads, cap // GROUP
+        f32, f16, i32, bf16, u8 = torch.float32, torch.float16, torch.int32, torch.bfloat16, torch.uint8
+        return dict(
+            codes=[new(rows, cap, 2 * (HEAD_DIM // 2), dtype=u8, device=dev) for _ in range(2)],
+            key_meta=[new(rows, groups, HEAD_DIM, 2, dtype=f32, device=dev) for _ in range(4)],
+            value_meta=[new(rows, cap, 2, 2, dtype=f32, device=dev) for _ in range(2)],
+            # the V metadata of all four streams again, one 64-byte record per logical token
+            # ([half][stream][scale, min]) for the readers of selected tokens
+            value_meta_token=new(rows, cap, 2, 4, 2, dtype=f32, device=dev),
+            # fp16 copies of the metadata, streamed by the readers
+            key_meta_half=[new(rows, groups, HEAD_DIM, 2, dtype=f16, device=dev) for _ in range(4)],
+            value_meta_half=[new(rows, cap, 2, 2, dtype=f16, device=dev) for _ in range(2)],
+            rank=[new(batch, cap, dtype=i32, device=dev) for _ in range(2)],
+            tail_key=[new(rows, tail, HEAD_DIM, dtype=bf16, device=dev) for _ in range(4)],
+            tail_value=[new(rows, tail, HEAD_DIM, dtype=bf16, device=dev) for _ in range(4)],
+            # loop-3/4 activity of tail rows (flashloop/cache.py:_tail_active)
+            tail_active=[new(batch, tail, dtype=u8, device=dev) for _ in range(2)],
+            packed_tokens=new(batch, dtype=i32, device=dev),
+            tail_tokens=new(batch, dtype=i32, device=dev),
+            late_rows=new(2, batch, dtype=i32, device=dev),  # rows used in streams 2/3
+        )
 
     # ------------------------------------------------------------------ geometry
     @property
@@ -207,23 +223,26 @@ class CrossLoopKVLayer:
             raise ValueError("lengths must give 1..T tokens per sequence")
         dev = keys[0].device
         masks = cls._mask_bytes(mask_loop3, mask_loop4, b, t, dev)
+        tp = [packed_prefix_tokens(x) for x in lengths]
+        tp_max = max(tp)
+        cap = _round_up(max(token_capacity or 0, tp_max, GROUP), GROUP)
+        # the late-row count is under way while the buffers that do not need it are allocated
+        count = cls._start_late_count(masks, tp) if late_counts is None else None
+        fixed = cls._fixed_buffers(b, h, cap, 2 * GROUP, dev, torch.empty)
+        src_k, src_v = [x.contiguous() for x in keys], [x.contiguous() for x in values]
+        group0 = torch.empty(b, dtype=torch.int32, device=dev)
         if late_counts is None:
-            late = cls._late_counts(masks, lengths)
+            late = cls._finish_late_count(count, tp)
         else:
             late = [[int(x) for x in c] for c in late_counts]
             if len(late) != 2 or any(len(c) != b or min(c) < 0 for c in late):
                 raise ValueError("late_counts must give a count per sequence for loops 3 and 4")
-        tp = [packed_prefix_tokens(x) for x in lengths]
-        tp_max = max(tp)
-        cap = _round_up(max(token_capacity or 0, tp_max, GROUP), GROUP)
         growth = cap - min(tp)  # every future decode token is active in every loop
         row_cap = (cap, cap, max(max(late[0]) + growth, 1), max(max(late[1]) + growth, 1))
-        layer = cls(LayerGeometry(b, h, cap, 2 * GROUP, row_cap), dev, _clear=False)
+        layer = cls(LayerGeometry(b, h, cap, 2 * GROUP, row_cap), dev, _buffers=fixed)
         layer.late_rows_host = late
         layer.packed_host = list(tp)
         layer.tail_host = [x - p for x, p in zip(lengths, tp)]
-        src_k, src_v = [x.contiguous() for x in keys], [x.contiguous() for x in values]
-        group0 = torch.empty(b, dtype=torch.int32, device=dev)
         # lengths, loop-3/4 compact rows (rank = running count of active rows), BF16 tails
         # (flashloop/cache.py:806-812) and the unused capacity, then the packed prefix
         kernels.cache_prepare(layer.view(), src_k, src_v, masks, layer.tail_active, tp, layer.tail_host, late,
@@ -252,14 +271,19 @@ class CrossLoopKVLayer:
         return masks
 
     @staticmethod
-    def _late_counts(masks, lengths: Sequence[int]) -> list[list[int]]:
-        tp = [packed_prefix_tokens(x) for x in lengths]
-        if masks[0] is None and masks[1] is None:
+    def _start_late_count(masks, tp: Sequence[int]):
+        """Launch the count of the rows the masks keep (None when they keep every row)."""
+        return None if masks[0] is None and masks[1] is None else kernels.count_active_rows(masks, tp)
+
+    @staticmethod
+    def _finish_late_count(count, tp: Sequence[int]) -> list[list[int]]:
+        if count is None:
             return [list(tp), list(tp)]
-        counts, nested = kernels.count_active_rows(masks, tp)
-        if not nested:
+        got = count.tolist()
+        b = len(tp)
+        if got[2 * b]:
             raise ValueError("Loop-4 overrides must be nested in Loop-3 overrides")
-        return counts
+        return [got[:b], got[b:2 * b]]
 
     @classmethod
     def count_late_rows(cls, mask_loop3: torch.Tensor, mask_loop4: torch.Tensor,
@@ -268,7 +292,8 @@ class CrossLoopKVLayer:
         (``[B, T]`` bool on the device), read back once: ``late_counts`` of ``from_prefill``."""
         b, t = mask_loop3.shape
         masks = cls._mask_bytes(mask_loop3, mask_loop4, b, t, mask_loop3.device)
-        return cls._late_counts(masks, [t] * b if lengths is None else [int(x) for x in lengths])
+        tp = [packed_prefix_tokens(int(x)) for x in ([t] * b if lengths is None else lengths)]
+        return cls._finish_late_count(cls._start_late_count(masks, tp), tp)
 
     # ------------------------------------------------------------------ readers
     def logits_capacity(self) -> int:

@@ -10,7 +10,7 @@
 //
 // All are bound by their launch or by the bytes they write.  As torch ops a build was 91 to 176
 // launches and three host synchronisations (layer of 16 heads, 8192 tokens, masked: 653 us, of
-// which the pack kernel took 83; now 185, one synchronisation) and a rollover ~40 launches (a
+// which the pack kernel took 83; now 152, one synchronisation) and a rollover ~40 launches (a
 // ragged batch of eight over four layers: 1324 us a token before, 1253 now).
 #include <algorithm>
 

@@ -68,10 +68,10 @@ def _ints(values):
     return (C.c_int32 * len(values))(*values)
 
 
-def count_active_rows(masks, packed) -> tuple[list[list[int]], bool]:
+def count_active_rows(masks, packed) -> torch.Tensor:
     """Tokens below each sequence's packed prefix that loops 3/4 keep (``masks``: two u8 [B, T]
-    device tensors or None for every token), and whether the masks are nested
-    (``fl_count_active_rows``).  Reads the counts back (one synchronisation)."""
+    device tensors or None for every token): i32 [2 * B + 1] on the device, loop 3's counts,
+    loop 4's, and whether the masks are not nested (``fl_count_active_rows``)."""
     some = next(m for m in masks if m is not None)
     b, t = some.shape
     for m in masks:
@@ -80,8 +80,7 @@ def count_active_rows(masks, packed) -> tuple[list[list[int]], bool]:
     counts = torch.zeros(2 * b + 1, dtype=torch.int32, device=some.device)
     check(load().fl_count_active_rows(_ptrs(masks), t, b, t, _ints(packed), counts.data_ptr(), _stream()),
           "fl_count_active_rows")
-    got = counts.tolist()
-    return [got[:b], got[b:2 * b]], got[2 * b] == 0
+    return counts
 
 
 def cache_prepare(view, src_keys, src_values, masks, tail_active, packed, tail, late, packed_tokens, tail_tokens,
