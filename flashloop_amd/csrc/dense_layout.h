@@ -66,6 +66,7 @@ struct DenseMergeLds {
 // those waves calls it).  `pieces` loops were read by one launch (dense_pair_kernel: 2):
 // index p*BH + bh merges row bh of piece p, whose units follow those of the earlier
 // pieces.  W: waves of the reader's grid.
+template <bool WIDE>
 __device__ __forceinline__ void dense_merge_row(DenseMergeLds& S, int index, const float* ws0, const float* ws1,
                                                 int W, const fl_cache_view& v, float* out0, float* out1,
                                                 int pieces) {
@@ -87,7 +88,7 @@ __device__ __forceinline__ void dense_merge_row(DenseMergeLds& S, int index, con
   const int gb = rl(v, b);
   vs += static_cast<int64_t>(h) * (kTailUnits + gb) + piece * U;
   const MergeParts P = dense_row_parts(ws, W, BH, bh, vs, gb, chunk_of(pieces * U, W));
-  const float r = merge_softmax(P, S.m);
+  const float r = merge_softmax<WIDE>(P, S.m);
   if (threadIdx.x < kDim) out[static_cast<int64_t>(bh) * kDim + threadIdx.x] = r;
 }
 

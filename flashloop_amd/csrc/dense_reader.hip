@@ -49,7 +49,13 @@ __global__ __launch_bounds__(kMergeThreads) void dense_merge_kernel(const float*
                                                                     fl_cache_view v, float* out0, float* out1,
                                                                     int pieces) {
   __shared__ DenseMergeLds S;
-  dense_merge_row(S, blockIdx.x, ws0, ws1, W, v, out0, out1, pieces);
+  dense_merge_row<false>(S, blockIdx.x, ws0, ws1, W, v, out0, out1, pieces);
+}
+
+__global__ __launch_bounds__(kMergeThreads) void dense_merge_wide_kernel(const float* ws, int W, fl_cache_view v,
+                                                                         float* out) {
+  __shared__ DenseMergeLds S;
+  dense_merge_row<true>(S, blockIdx.x, ws, ws, W, v, out, out, 1);
 }
 
 // Position in the work sequence: row (b, h), group gi of gb, row's first unit vs.
@@ -973,8 +979,15 @@ int32_t dense_launch(const fl_cache_view& v, int32_t loop, const uint16_t* q, co
   FL_LAUNCH_CHECK("fl_decode_attn_dense(reader)");
   if (waves) *waves = a.waves;
   if (!merge) return FL_OK;
-  hipLaunchKernelGGL(dense_merge_kernel, dim3(v.batch * v.heads), dim3(kMergeThreads), 0, st,
-                     static_cast<const float*>(a.ws), static_cast<const float*>(a.ws), a.waves, v, out, out, 1);
+  // long rows of many parts take the wide merge: 16 rows of 70,000 tokens, loops 1 and 2 (128 and
+  // 64 parts) 9.4 -> 6.8 us a merge; at 8192 tokens (66 parts) it loses, 6.0 -> 6.8
+  const int rows = v.batch * v.heads;
+  const bool wide = a.waves / rows > kMergeSplit * kMergeLocal && v.max_packed_tokens >= 32768;
+  const float* p = a.ws;
+  if (wide)
+    hipLaunchKernelGGL(dense_merge_wide_kernel, dim3(rows), dim3(kMergeThreads), 0, st, p, a.waves, v, out);
+  else
+    hipLaunchKernelGGL(dense_merge_kernel, dim3(rows), dim3(kMergeThreads), 0, st, p, p, a.waves, v, out, out, 1);
   FL_LAUNCH_CHECK("fl_decode_attn_dense(merge)");
   return FL_OK;
 }

@@ -139,6 +139,76 @@ __device__ __forceinline__ float dot_bf16_words(uint4 w, const float* q) {
   return d;
 }
 
+// Merge of row bh: slots [f+bh, l+bh] of each partial set (see gather_slot).
+template <bool WIDE>
+__device__ __forceinline__ void gather_merge_row(const float* ws, int waves, int tpr, int nrows, const int32_t* counts,
+                                                 int cap, int tok, float* out, int mode, const float* mass,
+                                                 const float* src, float* src_out) {
+  __shared__ MergeLdsBuf S;
+  __shared__ int live_red[2][kMergeThreads / kWave];
+  const int bh = blockIdx.x, tid = threadIdx.x;
+  // the row's live-tile range [rs, re) and the total, as the reader derived them
+  int64_t rs = static_cast<int64_t>(bh) * tpr, re = rs + tpr, total = static_cast<int64_t>(nrows) * tpr;
+  if (counts != nullptr && nrows <= kLiveRows) {
+    int before = 0, all = 0;
+    for (int r = tid; r < nrows; r += kMergeThreads) {
+      const int n = live_tiles(counts, r, cap, tok);
+      all += n;
+      if (r < bh) before += n;
+    }
+    before = wave_sum_int(before);
+    all = wave_sum_int(all);
+    if ((tid & 63) == 0) {
+      live_red[0][tid >> 6] = before;
+      live_red[1][tid >> 6] = all;
+    }
+    __syncthreads();
+    before = all = 0;
+    for (int w = 0; w < kMergeThreads / kWave; ++w) {
+      before += live_red[0][w];
+      all += live_red[1][w];
+    }
+    rs = before;
+    re = before + live_tiles(counts, bh, cap, tok);
+    total = all;
+  }
+  const int64_t chunk = (total + waves - 1) / waves * kWaves;  // tiles per reader workgroup
+  const int64_t f = rs / chunk, l = (re - 1) / chunk;
+  const int64_t o = static_cast<int64_t>(bh) * kDim + tid;
+  const MergeParts P{ws + (f + bh) * kPartial, static_cast<int>(l - f + 1), nullptr};
+  if (mode == kMergeSum) {
+    const float r = merge_channel_sum<false>(P, nullptr, S.acc);
+    if (tid < kDim) out[o] = r;
+    return;
+  }
+  float res = merge_softmax<WIDE>(P, S);
+  if (mode == kMergeMassDeltaFused) {
+    const MergeParts P2{ws + (static_cast<int64_t>(waves) + nrows + f + bh) * kPartial, static_cast<int>(l - f + 1),
+                        nullptr};
+    const float s = merge_channel_sum<false>(P2, nullptr, S.acc);
+    if (tid < kDim) {
+      src_out[o] = s;
+      res = mass[bh] * (res - s);
+    }
+  } else if (mode == kMergeMassDelta) {
+    if (tid < kDim) res = mass[bh] * (res - src[o]);
+  }
+  if (tid < kDim) out[o] = res;
+}
+
+// (kernels of their own, ahead of the readers, as in dense_reader.hip)
+__global__ __launch_bounds__(kMergeThreads) void gather_merge_kernel(
+    const float* ws, int waves, int tpr, int nrows, const int32_t* counts, int cap, int tok, float* out, int mode,
+    const float* mass, const float* src, float* src_out) {
+  gather_merge_row<false>(ws, waves, tpr, nrows, counts, cap, tok, out, mode, mass, src, src_out);
+}
+
+__global__ __launch_bounds__(kMergeThreads) void gather_merge_wide_kernel(
+    const float* ws, int waves, int tpr, int nrows, const int32_t* counts, int cap, int tok, float* out, int mode,
+    const float* mass, const float* src, float* src_out) {
+  gather_merge_row<true>(ws, waves, tpr, nrows, counts, cap, tok, out, mode, mass, src, src_out);
+}
+
 // ---------------------------------------------------------------------------------
 // Persistent tile readers.  The selection of row bh is cut into tiles of T slots; wave
 // w of the grid owns tiles [w*chunk, min((w+1)*chunk, total)) of the row-major tile
@@ -776,63 +846,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   }
 }
 
-// Merge of row bh: slots [f+bh, l+bh] of each partial set (see gather_slot).
-__global__ __launch_bounds__(kMergeThreads) void gather_merge_kernel(const float* ws, int waves, int tpr, int nrows,
-                                                                     const int32_t* counts, int cap, int tok,
-                                                                     float* out, int mode, const float* mass,
-                                                                     const float* src, float* src_out) {
-  __shared__ MergeLdsBuf S;
-  __shared__ int live_red[2][kMergeThreads / kWave];
-  const int bh = blockIdx.x, tid = threadIdx.x;
-  // the row's live-tile range [rs, re) and the total, as the reader derived them
-  int64_t rs = static_cast<int64_t>(bh) * tpr, re = rs + tpr, total = static_cast<int64_t>(nrows) * tpr;
-  if (counts != nullptr && nrows <= kLiveRows) {
-    int before = 0, all = 0;
-    for (int r = tid; r < nrows; r += kMergeThreads) {
-      const int n = live_tiles(counts, r, cap, tok);
-      all += n;
-      if (r < bh) before += n;
-    }
-    before = wave_sum_int(before);
-    all = wave_sum_int(all);
-    if ((tid & 63) == 0) {
-      live_red[0][tid >> 6] = before;
-      live_red[1][tid >> 6] = all;
-    }
-    __syncthreads();
-    before = all = 0;
-    for (int w = 0; w < kMergeThreads / kWave; ++w) {
-      before += live_red[0][w];
-      all += live_red[1][w];
-    }
-    rs = before;
-    re = before + live_tiles(counts, bh, cap, tok);
-    total = all;
-  }
-  const int64_t chunk = (total + waves - 1) / waves * kWaves;  // tiles per reader workgroup
-  const int64_t f = rs / chunk, l = (re - 1) / chunk;
-  const int64_t o = static_cast<int64_t>(bh) * kDim + tid;
-  const MergeParts P{ws + (f + bh) * kPartial, static_cast<int>(l - f + 1), nullptr};
-  if (mode == kMergeSum) {
-    const float r = merge_channel_sum<false>(P, nullptr, S.acc);
-    if (tid < kDim) out[o] = r;
-    return;
-  }
-  float res = merge_softmax(P, S);
-  if (mode == kMergeMassDeltaFused) {
-    const MergeParts P2{ws + (static_cast<int64_t>(waves) + nrows + f + bh) * kPartial, static_cast<int>(l - f + 1),
-                        nullptr};
-    const float s = merge_channel_sum<false>(P2, nullptr, S.acc);
-    if (tid < kDim) {
-      src_out[o] = s;
-      res = mass[bh] * (res - s);
-    }
-  } else if (mode == kMergeMassDelta) {
-    if (tid < kDim) res = mass[bh] * (res - src[o]);
-  }
-  if (tid < kDim) out[o] = res;
-}
-
 constexpr int32_t kMaxGatherRows = 1 << 24;  // rows per (b, h) and stream that 32-bit line offsets address
 
 int32_t check_gather_args(const fl_cache_view* view, int32_t loop, const int32_t* indices, const uint8_t* valid,
@@ -934,8 +947,15 @@ void launch_gather(GatherArgs& a, int rows, hipStream_t st) {
     default: launch_ns<4, MODE>(a, rows, st); break;
   }
   const int mode = MODE == kSelectedPV ? kMergeSum : (MODE == kSparseDelta ? kMergeMassDelta : kMergeMassDeltaFused);
-  hipLaunchKernelGGL(gather_merge_kernel, dim3(rows), dim3(kMergeThreads), 0, st, static_cast<const float*>(a.ws),
-                     a.waves, a.tpr, rows, a.counts, a.cap, Lay<kLpt>::kTok, a.out, mode, a.mass, a.src, a.src_out);
+  const auto merge = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(rows), dim3(kMergeThreads), 0, st, static_cast<const float*>(a.ws), a.waves, a.tpr,
+                       rows, a.counts, a.cap, Lay<kLpt>::kTok, a.out, mode, a.mass, a.src, a.src_out);
+  };
+  // a row's parts are the workgroups it touches: past 32 the wide merge (33 parts: 7.1 -> 6.4 us)
+  if (a.waves / kWaves / rows + 1 > kMergeSplit * kMergeLocal)
+    merge(gather_merge_wide_kernel);
+  else
+    merge(gather_merge_kernel);
 }
 
 }  // namespace

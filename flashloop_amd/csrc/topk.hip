@@ -931,7 +931,7 @@ __global__ __launch_bounds__(kTopkThreads) void select_merge_kernel(TopkArgs A, 
   // the merge uses the first kMergeThreads threads; the other waves leave (a workgroup
   // barrier waits only for waves that have not ended)
   if (threadIdx.x >= reader::kMergeThreads) return;
-  reader::dense_merge_row(L.m, blockIdx.x - rows, ws, ws, W, v, out, out, 1);
+  reader::dense_merge_row<false>(L.m, blockIdx.x - rows, ws, ws, W, v, out, out, 1);
 }
 
 // ---------------------------------------------------------------------------------

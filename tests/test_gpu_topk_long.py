@@ -8,7 +8,8 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-from flashloop_amd import _lib, kernels  # noqa: E402
+from flashloop_amd import CrossLoopKVLayer, _lib, decode_attention_step, kernels  # noqa: E402
+from flashloop_amd.synthetic import SCALING, loop_chain  # noqa: E402
 
 DEV = "cuda"
 
@@ -63,3 +64,30 @@ def test_long_rows_equal_one_workgroup_per_row(kind, stride, fraction):
         a, b = a.double().cpu().numpy(), b.double().cpu().numpy()
         assert np.array_equal(np.isnan(a), np.isnan(b))
         assert np.all(np.isnan(b) | (np.abs(a - b) <= 2 * cap * 2.0 ** -24 * np.abs(b)))
+
+
+def test_long_row_alone_equals_the_row_in_a_batch():
+    """A long sequence alone merges its many partials on another path (and divides its top-k over
+    workgroups) than as one of a batch: the fp32 sums are grouped differently, nothing else.
+    An output is a mix of V rows with weights that add up to 1, so its sums' sizes are at most
+    max |v|; a partial adds at most 1250 keys in fp32 (40,000 over 32 waves a row), whose
+    roundings average to sqrt(1250) * 2^-24 = 2.1e-6 of that; 4e-6 allows both sides."""
+    print("case: long row alone, t=40000", flush=True)
+    h, t = 16, 40000
+    gen = torch.Generator(device=DEV).manual_seed(99)
+    ks, vs = loop_chain(gen, (1, h, t, 128), device=DEV), loop_chain(gen, (1, h, t, 128), device=DEV)
+    q, kc, vc = ([x for x in loop_chain(gen, (1, h, 1, 128), device=DEV)] for _ in range(3))
+    one = decode_attention_step(CrossLoopKVLayer.from_prefill(ks, vs), q, kc, vc, SCALING)
+    many = decode_attention_step(CrossLoopKVLayer.from_prefill([x.expand(6, -1, -1, -1) for x in ks], [x.expand(6, -1, -1, -1) for x in vs]),
+                                 *([x.expand(6, -1, -1, -1).contiguous() for x in y] for y in (q, kc, vc)), SCALING)
+    size = max(x.float().abs().max().item() for x in vs)
+    for i in (0, 5):
+        same = (one.indices[0] == many.indices[i]).all(-1)  # (a swap at the boundary changes a head's selection)
+        assert int(same.sum()) >= h // 2
+        for name in ("out0", "out1", "selected_output", "delta2", "delta3"):
+            a, b = getattr(one, name)[0], getattr(many, name)[i]
+            if name[:3] != "out":
+                a, b = a[same], b[same]
+            assert (a - b).abs().max().item() <= 4e-6 * size, name
+        # logits are sums of 128 products of sizes up to |q||k| / sqrt(128), about 40
+        assert (one.logits1[0, ..., : t + 1] - many.logits1[i, ..., : t + 1]).abs().max().item() <= 128 * 2.0 ** -24 * 40
