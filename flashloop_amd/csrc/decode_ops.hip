@@ -423,9 +423,9 @@ __global__ __launch_bounds__(kNormThreads) void norm_chain_kernel(NormArgs a) {
 // work, all its weights requested before its first product; its waves split K in steps of 512
 // and their partial tiles meet in LDS.  Eight rows take 8 waves, one wave per chain row; one
 // row takes 4 waves and 4-row tiles (twice the workgroups).  Measured, 2048 wide (q/k/v with
-// RoPE, o_proj, SwiGLU 5632, down, lm_head 49152), us before -> now: 8 rows 46.8 -> 11.3,
-// 12.1 -> 5.7, 75.2 -> 14.2, 15.6 -> 7.9, 287 -> 41 (4.9 TB/s); one row 9.2 -> 7.6, 4.8 -> 5.0,
-// 13.3 -> 11.4, 6.1 -> 6.7, 42.0 -> 36.5 (5.5 TB/s).  One row with 8 waves and 8-row tiles
+// RoPE, o_proj, SwiGLU 5632, down, lm_head 49152), us before -> now: 8 rows 46.8 -> 10.0,
+// 12.1 -> 5.4, 75.2 -> 12.9, 15.6 -> 7.9, 287 -> 40 (5.0 TB/s); one row 9.2 -> 7.7, 4.8 -> 4.9,
+// 13.3 -> 10.8, 6.1 -> 6.9, 42.0 -> 36.5 (5.5 TB/s).  One row with 8 waves and 8-row tiles
 // took 9.1, 5.1, 11.9, 6.9 and 38.4.
 template <int MT>
 struct MmGeom {
@@ -530,9 +530,41 @@ __device__ __forceinline__ void load_unit(const UnitRows<NT>& ur, int K, uint4 (
   }
 }
 
+// What the epilogue of unit u reads besides the dots: cos and sin of the rotary pair, or the
+// addends.  Requested right behind the unit's weights, so that no load follows the last product
+// (8 rows: o_proj 5.7 -> 5.4 us; q/k/v with RoPE 11.3 -> 10.7).
+template <int EPI, int NT>
+struct EpiIn {
+  uint16_t v[EPI == kEpiRope ? 4 : NT];
+};
+
+template <int EPI, int MT, int NT>
+__device__ __forceinline__ void load_epi(const GemvArgs& a, int u, EpiIn<EPI, NT>& e) {
+  constexpr int kTile = MmGeom<MT>::kTile;
+  const int m = threadIdx.x / kTile, i = threadIdx.x % kTile;
+  if (EPI == kEpiRope) {
+    const int per = units_per_matrix<EPI, MT>(a.N), half = a.head_dim / 2;
+    const int mat = u / per, p = (u - mat * per) * kTile + i;
+    if (mat == 2 || m >= min(MT, a.M) || p >= a.N / 2) return;
+    const int64_t o = static_cast<int64_t>(m) * a.head_dim + p % half;
+    e.v[0] = a.cos[o];
+    e.v[1] = a.sin[o];
+    e.v[2] = a.cos[o + half];
+    e.v[3] = a.sin[o + half];
+  } else if (EPI == kEpiAdd) {
+    if (m >= min(MT, a.M)) return;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int n = (NT * u + t) * kTile + i;
+      if (n < a.N) e.v[t] = a.addend[static_cast<int64_t>(m) * a.addend_stride + n];
+    }
+  }
+}
+
 // Output (m, i-th row of each tile) of unit u from the tiles' bf16-rounded dots v[t].
 template <int EPI, int MT, int NT>
-__device__ __forceinline__ void unit_store(const GemvArgs& a, int u, int m, int i, const float* v) {
+__device__ __forceinline__ void unit_store(const GemvArgs& a, int u, int m, int i, const float* v,
+                                           const EpiIn<EPI, NT>& e) {
   constexpr int kTile = MmGeom<MT>::kTile;
   if (EPI == kEpiSwiGlu) {
     const int n = kTile * u + i;
@@ -552,10 +584,8 @@ __device__ __forceinline__ void unit_store(const GemvArgs& a, int u, int m, int 
       y[0] = f32_to_bf16_rne(lo);
       y[half] = f32_to_bf16_rne(hi);
     } else {
-      const uint16_t* cs = a.cos + static_cast<int64_t>(m) * a.head_dim + c;
-      const uint16_t* sn = a.sin + static_cast<int64_t>(m) * a.head_dim + c;
-      y[0] = f32_to_bf16_rne(bf16_round(lo * bf16_to_f32(cs[0])) + bf16_round(-hi * bf16_to_f32(sn[0])));
-      y[half] = f32_to_bf16_rne(bf16_round(hi * bf16_to_f32(cs[half])) + bf16_round(lo * bf16_to_f32(sn[half])));
+      y[0] = f32_to_bf16_rne(bf16_round(lo * bf16_to_f32(e.v[0])) + bf16_round(-hi * bf16_to_f32(e.v[1])));
+      y[half] = f32_to_bf16_rne(bf16_round(hi * bf16_to_f32(e.v[2])) + bf16_round(lo * bf16_to_f32(e.v[3])));
     }
   } else {
 #pragma unroll
@@ -567,7 +597,7 @@ __device__ __forceinline__ void unit_store(const GemvArgs& a, int u, int m, int 
         static_cast<float*>(a.y[0])[o] = v[t];
       else if (EPI == kEpiAdd)
         static_cast<uint16_t*>(a.y[0])[o] =
-            f32_to_bf16_rne(v[t] + bf16_to_f32(a.addend[static_cast<int64_t>(m) * a.addend_stride + n]));
+            f32_to_bf16_rne(v[t] + bf16_to_f32(e.v[t]));
       else
         static_cast<uint16_t*>(a.y[0])[o] = f32_to_bf16_rne(v[t]);
     }
@@ -690,27 +720,40 @@ __device__ __forceinline__ void load_x(const GemvArgs& a, bf16x8_t (&x)[CS]) {
 }
 
 // KCAP: the largest K of the instantiation (a unit's weights are in registers).  MT: x rows
-// (1, or up to 8).  PP: grids of several units per workgroup, two units' weights in flight.
-template <int EPI, int MT, int KCAP, int NT, bool CHAIN, bool PP>
+// (1, or up to 8).  DEPTH: units whose weights are in flight (1: a grid of one unit per workgroup;
+// 2: of several).
+template <int EPI, int MT, int KCAP, int NT, bool CHAIN, int DEPTH>
 __global__ __launch_bounds__(MmGeom<MT>::kThreads, 2) void gemv_mfma_kernel(GemvArgs a, NormArgs c, int units) {
   using G = MmGeom<MT>;
   constexpr int CS = KCAP / kMmStepK;  // steps of a wave over K
   constexpr int kRow = KCAP + 8;       // x row in LDS, elements
+  // one row with RoPE: three short workgroups a CU hide the load, its arithmetic up front costs 0.25 us
+  constexpr bool kAhead = EPI == kEpiAdd || (EPI == kEpiRope && MT > 1);
   __shared__ uint16_t xs[CHAIN ? MT * kRow : 8];
   __shared__ float red[2][G::kParts][NT][MT][G::kTile];  // [unit parity][wave, k-slice][tile][x row][W row]
   __shared__ float nred[2][kNormWaves];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // (buffer descriptors of a wave's row are scalar)
 
-  uint4 w0[NT][CS], w1[PP ? NT : 1][PP ? CS : 1];
+  uint4 w[DEPTH][NT][CS];
+  EpiIn<EPI, NT> e[DEPTH];
   int u = blockIdx.x;
-  const auto load = [&](int unit, auto& w) __attribute__((always_inline)) {
+  const int step = gridDim.x;
+  const auto load = [&](int unit, int d) __attribute__((always_inline)) {
     UnitRows<NT> ur;
-    unit_rows<EPI, MT, NT>(a, min(unit, units - 1), ur);
-    load_unit<MT, NT, CS>(ur, a.K, w);
+    const int K = DEPTH == 1 || unit < units ? a.K : 0;  // (past the last unit: nothing is read)
+    if (DEPTH > 1) unit = min(unit, units - 1);
+    unit_rows<EPI, MT, NT>(a, unit, ur);
+    load_unit<MT, NT, CS>(ur, K, w[d]);
+    // the weights are all requested here (left to itself the compiler loads each before its product
+    // once no loop follows: down 6.9 -> 7.4 us), and ahead of load_epi's index arithmetic
+    __builtin_amdgcn_sched_barrier(0);
+    if (kAhead && wave == 0) load_epi<EPI, MT, NT>(a, unit, e[d]);  // (the threads that store lie in one wave)
   };
+  static_assert(MT * G::kTile <= kWave, "one wave stores");
   const auto load_first = [&]() __attribute__((always_inline)) {
-    load(u, w0);
-    if constexpr (PP) load(u + gridDim.x, w1);
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) load(u + d * step, d);
   };
   bf16x8_t xr[CHAIN ? 1 : CS];
   if constexpr (CHAIN && MT == 1) {
@@ -749,7 +792,7 @@ __global__ __launch_bounds__(MmGeom<MT>::kThreads, 2) void gemv_mfma_kernel(Gemv
 
   const uint16_t* xl = &xs[CHAIN ? (MT == 1 ? 0 : (lane & 7)) * kRow + lane_k0<MT>() : 0];
   int par = 0;
-  const auto compute = [&](const auto& w, int unit) __attribute__((always_inline)) {
+  const auto compute = [&](int d, int unit) __attribute__((always_inline)) {
     f32x4_t acc[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
@@ -762,7 +805,7 @@ __global__ __launch_bounds__(MmGeom<MT>::kThreads, 2) void gemv_mfma_kernel(Gemv
         xv = xr[s];
 #pragma unroll
       for (int t = 0; t < NT; ++t)
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w[t][s]), xv, acc[t], 0, 0, 0);
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w[d][t][s]), xv, acc[t], 0, 0, 0);
     }
     // lane l holds rows 4 (l / 16) ..+3 of column l % 16: the diagonal blocks are kept
     const int row = 4 * (lane >> 4), col = lane & 15;
@@ -782,27 +825,19 @@ __global__ __launch_bounds__(MmGeom<MT>::kThreads, 2) void gemv_mfma_kernel(Gemv
           for (int p = 0; p < G::kParts; ++p) sum += red[par][p][t][m][i];
           v[t] = bf16_round(sum);  // the Linear's bf16 output
         }
-        unit_store<EPI, MT, NT>(a, unit, m, i, v);
+        if constexpr (!kAhead) load_epi<EPI, MT, NT>(a, unit, e[d]);
+        unit_store<EPI, MT, NT>(a, unit, m, i, v, e[d]);
       }
     }
     par ^= 1;  // (a buffer is written again after the next unit's barrier)
   };
-  const int step = gridDim.x;
-  while (true) {
-    compute(w0, u);
-    if constexpr (PP) {
-      if (u + step >= units) break;
-      load(u + 2 * step, w0);
-      compute(w1, u + step);
-      if (u + 2 * step >= units) break;
-      load(u + 3 * step, w1);
-      u += 2 * step;
-    } else {
-      u += step;
-      if (u >= units) break;
-      load(u, w0);
+  for (;; u += DEPTH * step)
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+      compute(d, u + d * step);
+      if (DEPTH == 1 || u + (d + 1) * step >= units) return;
+      load(u + (d + DEPTH) * step, d);
     }
-  }
 }
 
 // ---------------------------------------------------------------------------------
@@ -856,40 +891,41 @@ __global__ __launch_bounds__(kAppendThreads) void append_tail_kernel(AppendArgs 
   if (threadIdx.x == 0) a.tail_tokens[b] = pos + 1;
 }
 
-template <int EPI, int MT, int KCAP, int NT, bool CHAIN, bool PP>
+template <int EPI, int MT, int KCAP, int NT, bool CHAIN, int DEPTH>
 void launch_gemv_mfma(const GemvArgs& a, const NormArgs& c, int workgroups, hipStream_t st) {
   const int per = units_per_matrix<EPI, MT>(a.N);
   const int units = EPI == kEpiRope ? 3 * per : (EPI == kEpiSwiGlu ? per : (per + NT - 1) / NT);
   int grid = units;
-  if (PP) {  // at most `workgroups`, each with the same number of units
+  if (DEPTH > 1) {  // at most `workgroups`, each with the same number of units
     const int rounds = (units + workgroups - 1) / workgroups;
     grid = (units + rounds - 1) / rounds;
   }
-  hipLaunchKernelGGL((gemv_mfma_kernel<EPI, MT, KCAP, NT, CHAIN, PP>), dim3(grid), dim3(MmGeom<MT>::kThreads), 0, st, a, c, units);
+  hipLaunchKernelGGL((gemv_mfma_kernel<EPI, MT, KCAP, NT, CHAIN, DEPTH>), dim3(grid), dim3(MmGeom<MT>::kThreads), 0, st, a, c, units);
 }
 
-// Several units per workgroup (PP) where the prologue or the epilogue of one unit would not
-// hide behind the other workgroups of its CU.  Eight chained rows: the prologue is ~900 VALU
+// Several units per workgroup (DEPTH 2) where the prologue or the epilogue of one unit would not
+// hide behind the other workgroups of its CU.  Eight chained rows: the prologue is ~700 VALU
 // instructions per row, so one workgroup per CU runs it once (SwiGLU 5632 x 2048: 16.8 us with
-// a workgroup per unit, 14.1 with 235 of three units).  One row: only the many units of a
-// head-sized matrix gain (lm_head 49152 x 2048: 37.5 -> 36.3 us; SwiGLU lost, 11.4 -> 13.1).
+// a workgroup per unit, 12.9 with 235 of three units; three units in flight gain nothing there
+// and q/k/v with RoPE, two units each, loses 9.9 -> 10.6).  One row: only the many units of a
+// head-sized matrix gain (lm_head 49152 x 2048: 37.5 -> 36.3 us; SwiGLU lost, 10.8 -> 13.1).
 template <int EPI, int MT, bool CHAIN>
 void launch_gemv_k(const GemvArgs& a, const NormArgs& c, hipStream_t st) {
   constexpr int kPair = EPI == kEpiSwiGlu || EPI == kEpiRope ? 2 : 1;
   if (a.K <= 2048) {
     if constexpr (CHAIN && MT == 8) {
-      return launch_gemv_mfma<EPI, MT, 2048, 2, CHAIN, true>(a, c, 256, st);
+      return launch_gemv_mfma<EPI, MT, 2048, 2, CHAIN, 2>(a, c, 256, st);
     } else {
-      if (a.N >= 16384) return launch_gemv_mfma<EPI, MT, 2048, 2, CHAIN, true>(a, c, 1024, st);
-      launch_gemv_mfma<EPI, MT, 2048, kPair, CHAIN, false>(a, c, 0, st);
+      if (a.N >= 16384) return launch_gemv_mfma<EPI, MT, 2048, 2, CHAIN, 2>(a, c, 1024, st);
+      launch_gemv_mfma<EPI, MT, 2048, kPair, CHAIN, 1>(a, c, 0, st);
     }
   } else if (a.K <= 4096) {
-    launch_gemv_mfma<EPI, MT, 4096, kPair, CHAIN, false>(a, c, 0, st);
+    launch_gemv_mfma<EPI, MT, 4096, kPair, CHAIN, 1>(a, c, 0, st);
   } else if constexpr (!CHAIN) {
     if (a.K <= 6144)
-      launch_gemv_mfma<EPI, MT, 6144, kPair, false, false>(a, c, 0, st);
+      launch_gemv_mfma<EPI, MT, 6144, kPair, false, 1>(a, c, 0, st);
     else
-      launch_gemv_mfma<EPI, MT, kMmMaxK, kPair, false, false>(a, c, 0, st);
+      launch_gemv_mfma<EPI, MT, kMmMaxK, kPair, false, 1>(a, c, 0, st);
   }
 }
 
