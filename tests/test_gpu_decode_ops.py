@@ -192,6 +192,19 @@ def _near(got, want, slack, what, ulps=1.0):
     assert bool((err <= 0).all()), f"{what}: {err.max().item():.3e} beyond the bound"
 
 
+@pytest.mark.parametrize("n", [2060, 4108, 8200])
+def test_gemv_chain_of_several_units(n):
+    """Eight chained rows run on at most 256 workgroups: two, three and five units each, the last
+    workgroups fewer (258, 514 and 1025 SwiGLU units); equal to the chain and the GEMV apart."""
+    print(f"case: gemv chain units n={n}", flush=True)
+    k = 520
+    r, x, wn, mats = _x(8, k, 90), _x(8, k, 91), [_x(1, k, 92 + i)[0] for i in range(2)], [_w(n, k, 94 + i) for i in range(2)]
+    h0, z0 = kernels.norm_chain(r, eps=1e-6, x=x, w_a=wn[0], w_b=wn[1])
+    for epi, ws, extra in ((kernels.EPI_SWIGLU, mats, {}), (kernels.EPI_ADD, mats[:1], dict(addend=_x(8, n, 96)))):
+        h1, got = kernels.gemv_chain(r, ws, eps=1e-6, epilogue=epi, x=x, w_a=wn[0], w_b=wn[1], **extra)
+        assert torch.equal(h1, h0) and torch.equal(got, kernels.gemv(z0, ws, epilogue=epi, **extra))
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 4, 8), (1, 516, 200), (2, 12, 520), (5, 516, 2056), (8, 20, 2048), (8, 16388, 1024),
                                    (1, 16388, 2040), (3, 36, 4104), (8, 260, 6152), (1, 260, 8192), (4, 8, 8200)])
 def test_gemv_at_tile_and_step_edges(m, n, k):
