@@ -1185,11 +1185,11 @@ __global__ __launch_bounds__(kTopkThreads) void split_histogram_kernel(SplitArgs
   if (hist[tid] != 0u) atomicAdd(&s.hist[tid], hist[tid]);
 }
 
-// The boundary bin (all threads): B*, and the number of keys in higher bins.
-__device__ __forceinline__ void split_boundary(const SplitRow& s, uint32_t* cnt, uint32_t* found, int* bstar, int* above) {
+// The bin of the k-th largest key (all threads), and the number of keys in higher bins.
+// h: the count of bin kBins - 1 - tid (a descending scan).
+__device__ __forceinline__ void split_boundary(uint32_t h, int k, uint32_t* cnt, uint32_t* found, int* bstar, int* above) {
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int bin = kBins - 1 - tid;  // descending scan
-  const uint32_t h = s.hist[bin];
+  const int bin = kBins - 1 - tid;
   uint32_t incl = h;
 #pragma unroll
   for (int o = 1; o < kWave; o <<= 1) {
@@ -1201,7 +1201,7 @@ __device__ __forceinline__ void split_boundary(const SplitRow& s, uint32_t* cnt,
   uint32_t before = 0;
   for (int q = 0; q < w; ++q) before += cnt[q];
   const uint32_t up = before + incl - h;
-  if (up < static_cast<uint32_t>(s.k) && up + h >= static_cast<uint32_t>(s.k)) {
+  if (up < static_cast<uint32_t>(k) && up + h >= static_cast<uint32_t>(k)) {
     found[0] = static_cast<uint32_t>(bin);
     found[1] = up;
   }
@@ -1221,7 +1221,7 @@ __global__ __launch_bounds__(kTopkThreads) void split_candidates_kernel(SplitArg
   const SplitScale c = split_scale(s, true);
   if (tid == 0) total = ncand = 0;
   int bstar, above;
-  split_boundary(s, cnt, found, &bstar, &above);  // (its barriers order the counters' reset)
+  split_boundary(s.hist[kBins - 1 - tid], s.k, cnt, found, &bstar, &above);  // (its barriers order the counters' reset)
   const int lane = tid & 63;
   const uint64_t lt_mask = (1ull << lane) - 1ull;
   uint32_t mine = 0;  // the wave's keys above B*
@@ -1255,8 +1255,9 @@ __global__ __launch_bounds__(kTopkThreads) void split_candidates_kernel(SplitArg
 }
 
 __global__ __launch_bounds__(kTopkThreads) void split_compact_kernel(SplitArgs a) {
-  __shared__ uint32_t cnt[kTopkWaves], found[2], kth[2], offset;
-  __shared__ uint32_t ck[kSplitCand], ci[kSplitCand], rk[kSplitCand];
+  __shared__ uint32_t cnt[kTopkWaves], found[2], kth[2], offset, nsub;
+  __shared__ uint64_t cv[kSplitCand];  // key, ~index: the larger is selected first
+  __shared__ uint32_t rk[kSplitCand], sub[kBins];
   __shared__ float red[kTopkWaves];
   const int r = blockIdx.y;
   const SplitRow s = split_row(a, r);
@@ -1275,38 +1276,59 @@ __global__ __launch_bounds__(kTopkThreads) void split_compact_kernel(SplitArgs a
   float x[4];
   slice_scores(s, base, x);
   const SplitScale c = split_scale(s, true);
-  if (tid < static_cast<int>(m)) {
-    ck[tid] = s.cand_key[tid];
-    ci[tid] = s.cand_idx[tid];
-    rk[tid] = 0;
-  }
-  if (tid == 0) offset = 0;
+  static_assert(kSplitCand == kTopkThreads && kBins == kTopkThreads, "one candidate and one bin per thread");
+  const bool mine_c = tid < static_cast<int>(m);
+  const uint32_t my_key = s.cand_key[tid], my_idx = s.cand_idx[tid];  // (past m: not used)
+  sub[tid] = 0;
+  rk[tid] = 0;
+  if (tid == 0) offset = nsub = 0;
   int bstar, above;
-  split_boundary(s, cnt, found, &bstar, &above);
-  const int need = s.k - above;  // keys of B* that are selected, >= 1
-  // the candidates' ranks in (key desc, index asc) order: the m x m comparisons over all waves,
-  // wave w comparing the 64 candidates of block w % nb with part w / nb of the list
-  const int nb = (static_cast<int>(m) + kWave - 1) / kWave, parts = kTopkWaves / nb;
+  split_boundary(s.hist[kBins - 1 - tid], s.k, cnt, found, &bstar, &above);
+  int need = s.k - above;  // keys of B* that are selected, >= 1
+  // B* once more by the next 10 bits, since every slice ranks the candidates and all m * m pairs
+  // of them cost it: only the bin with the last selected key is ranked by pairs (16 rows of
+  // 70,001 keys: 15.9 -> 12.8 us for this launch)
+  int my_sub = 0, sstar = 0;
+  if (c.weighted) {
+    const uint32_t low = static_cast<uint32_t>(max(static_cast<int>(my_key - c.kmin), 0)) - (static_cast<uint32_t>(bstar) << c.shift);
+    my_sub = static_cast<int>(min(low >> (c.shift > 10u ? c.shift - 10u : 0u), kBins - 1u));
+    if (mine_c) atomicAdd(&sub[my_sub], 1u);
+    __syncthreads();
+    int higher;
+    split_boundary(sub[kBins - 1 - tid], need, cnt, found, &sstar, &higher);
+    need -= higher;
+  }
+  const uint64_t my_cv = static_cast<uint64_t>(my_key) << 32 | static_cast<uint32_t>(~my_idx);
+  const bool ranked = mine_c && my_sub == sstar;
+  int at = 0;
+  if (ranked) {
+    at = static_cast<int>(atomicAdd(&nsub, 1u));  // (any order: a rank counts the larger ones)
+    cv[at] = my_cv;
+  }
+  __syncthreads();
+  // ranks in (key desc, index asc) order: the comparisons over all waves, wave w comparing the
+  // 64 candidates of block w % nb with part w / nb of the list
+  const int q = static_cast<int>(nsub), nb = (q + kWave - 1) / kWave, parts = kTopkWaves / nb;
   const int cand = (w % nb) * kWave + lane, part = w / nb;
-  if (part < parts && cand < static_cast<int>(m)) {
-    const int each = (static_cast<int>(m) + parts - 1) / parts;
-    const int u1 = min(static_cast<int>(m), (part + 1) * each);
-    const uint32_t mk = ck[cand], mi = ci[cand];
+  if (part < parts && cand < q) {
+    const int each = (q + parts - 1) / parts, u1 = min(q, (part + 1) * each);
+    const uint64_t v = cv[cand];
     uint32_t rank = 0;
 #pragma unroll 4
-    for (int u = part * each; u < u1; ++u) rank += (ck[u] > mk || (ck[u] == mk && ci[u] < mi)) ? 1u : 0u;
+    for (int u = part * each; u < u1; ++u) rank += cv[u] > v ? 1u : 0u;
     if (rank) atomicAdd(&rk[cand], rank);
   }
   __syncthreads();
-  bool lower = false;  // a selected candidate of an earlier slice
-  if (tid < static_cast<int>(m)) {
-    const int rank = static_cast<int>(rk[tid]);
+  bool lower = mine_c && my_sub > sstar;  // a selected candidate of an earlier slice
+  if (ranked) {
+    const int rank = static_cast<int>(rk[at]);
     if (rank == need - 1) {
-      kth[0] = ck[tid];
-      kth[1] = ci[tid];
+      kth[0] = my_key;
+      kth[1] = my_idx;
     }
-    lower = rank < need && ci[tid] < static_cast<uint32_t>(slice * kSliceKeys);
+    lower = rank < need;
   }
+  lower = lower && my_idx < static_cast<uint32_t>(slice * kSliceKeys);
   uint32_t before = static_cast<uint32_t>(__popcll(ballot64(lower)));
   if (w == 0) {
     uint32_t up = 0;
