@@ -31,7 +31,7 @@ import torch.nn.functional as F
 from . import kernels
 from .cache import CrossLoopKVCache, CrossLoopKVLayer
 from .config import FlashLoopConfig, validate_ouro_model
-from .model import MLP, Attention, OuroConfig, OuroForCausalLM, RMSNorm, apply_rope
+from .model import MLP, Attention, OuroConfig, OuroForCausalLM, RMSNorm, RotaryEmbedding, apply_rope
 
 
 @dataclass(frozen=True)
@@ -130,7 +130,7 @@ class DecodeRunner:
     def _release(self) -> None:
         """Destroy the captured graph and its private memory pool, here and now (never
         inside a capture).  Nothing outside this runner holds a tensor of that pool: the
-        step's logits are copied, inside the graph, into ``out``, an ordinary allocation."""
+        step's logits are written, inside the graph, to ``out``, an ordinary allocation."""
         self.logits = None
         if self.graph is not None:
             self.graph.reset()
@@ -154,7 +154,7 @@ class DecodeRunner:
         dev = token_ids.device
         if not self.use_graphs:
             pos_t = torch.tensor([[int(p)] for p in positions], dtype=torch.long, device=dev)
-            return eng._decode_core(cache, eng.backbone.embed_tokens(token_ids), pos_t)
+            return eng._decode_core(cache, token_ids, pos_t)
         if self.tok is None or self.tok.shape[0] != bsz:
             self._release()
             self.tok = torch.zeros((bsz, 1), dtype=torch.long, device=dev)
@@ -180,7 +180,7 @@ class DecodeRunner:
         side = torch.cuda.Stream()  # default priority
         side.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(side):
-            eng._decode_core(cache, eng.backbone.embed_tokens(self.tok), self.pos)
+            eng._decode_core(cache, self.tok, self.pos)
             for lc in cache.layers:
                 lc.tail_tokens -= 1
         torch.cuda.current_stream().wait_stream(side)
@@ -192,8 +192,9 @@ class DecodeRunner:
         gc.disable()
         try:
             with torch.cuda.graph(graph):
-                self.logits = eng._decode_core(cache, eng.backbone.embed_tokens(self.tok), self.pos)
-                self.out.copy_(self.logits)
+                self.logits = eng._decode_core(cache, self.tok, self.pos, out=self.out)
+                if self.logits is not self.out:
+                    self.out.copy_(self.logits)
         finally:
             if was_enabled:
                 gc.enable()
@@ -458,12 +459,28 @@ class FlashLoopEngine:
         return PrefillOutput(logits=logits, state=self._state)
 
     # ------------------------------------------------------------------ decode
-    def _decode_core(self, cache: CrossLoopKVCache, h: torch.Tensor, pos_t: torch.Tensor) -> torch.Tensor:
+    def _decode_core(self, cache: CrossLoopKVCache, token_ids: torch.Tensor, pos_t: torch.Tensor,
+                     out: torch.Tensor | None = None) -> torch.Tensor:
         """One decode step (see ``_decode_core_fused``); the torch-module form runs when the
-        fused kernels do not apply (``fused_decode`` off, non-bf16 weights, batch > 8)."""
-        if self.fused_decode and h.shape[0] <= 8 and self._fused_weights() is not None:
-            return self._decode_core_fused(cache, h, pos_t)
-        return self._decode_core_modules(cache, h, pos_t)
+        fused kernels do not apply (``fused_decode`` off, non-bf16 weights, batch > 8).  The
+        fused form writes the logits to ``out`` if given."""
+        if self.fused_decode and token_ids.shape[0] <= 8 and self._fused_weights() is not None:
+            return self._decode_core_fused(cache, *self._decode_inputs(token_ids, pos_t), logits_out=out)
+        return self._decode_core_modules(cache, self.backbone.embed_tokens(token_ids), pos_t)
+
+    def _decode_inputs(self, token_ids: torch.Tensor, pos_t: torch.Tensor):
+        """Embedded tokens, cos and sin of a decode step: one launch where the two modules are
+        the plain ones on the device (a replaced or hooked module is called)."""
+        emb, rot = self.backbone.embed_tokens, self.backbone.rotary_emb
+        if (type(emb) is torch.nn.Embedding and type(rot) is RotaryEmbedding
+                and not any(m._forward_hooks or m._forward_pre_hooks or "forward" in vars(m) for m in (emb, rot))
+                and emb.max_norm is None and token_ids.dtype == torch.long
+                and all(t.is_cuda and t.is_contiguous() for t in (token_ids, pos_t, emb.weight, rot.inv_freq))
+                and emb.weight.dtype == torch.bfloat16 and emb.weight.shape[1] % 8 == 0 and emb.weight.data_ptr() % 16 == 0
+                and rot.inv_freq.dtype in (torch.float32, torch.bfloat16)):
+            return kernels.decode_inputs(token_ids, pos_t, emb.weight, rot.inv_freq)
+        h = emb(token_ids)
+        return (h, *rot(h, pos_t))
 
     def _fused_weights(self):
         """Per-layer weight tensors of the fused decode path, or None when a weight is not a
@@ -487,7 +504,8 @@ class FlashLoopEngine:
             self._wcache = (layers, extra) if all(ok(t) for t in extra.values()) else False
         return self._wcache or None
 
-    def _decode_core_fused(self, cache: CrossLoopKVCache, h: torch.Tensor, pos_t: torch.Tensor) -> torch.Tensor:
+    def _decode_core_fused(self, cache: CrossLoopKVCache, h: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
+                           logits_out: torch.Tensor | None = None) -> torch.Tensor:
         """The step of ``_decode_core_modules`` on the fused decode kernels: per layer and
         loop one q/k/v GEMV with RoPE, the cache readers, one o_proj GEMV (+ the loop-2
         projection for loops 3/4), one residual/norm chain, one SwiGLU GEMV, one down GEMV
@@ -501,7 +519,6 @@ class FlashLoopEngine:
         bsz = h.shape[0]
         nl = len(self.layers)
         heads, hd = self.layers[0].self_attn.num_heads, self.layers[0].self_attn.head_dim
-        cos, sin = self.backbone.rotary_emb(h, pos_t)
         rope = (cos.reshape(bsz, hd), sin.reshape(bsz, hd))
         hid = h.reshape(bsz, -1)
         chained = self.fused_chain
@@ -568,7 +585,7 @@ class FlashLoopEngine:
         for li in range(nl):
             cache.layers[li].append_rows(cur_k[li], cur_v[li])
         # the last chain (final norm, no input norm) feeds lm_head
-        return chain_gemv([extra["lm_head"]], epilogue=kernels.EPI_F32)
+        return chain_gemv([extra["lm_head"]], epilogue=kernels.EPI_F32, **({"out": logits_out} if chained else {}))
 
     def _decode_core_modules(self, cache: CrossLoopKVCache, h: torch.Tensor, pos_t: torch.Tensor) -> torch.Tensor:
         """One decode step of ``B`` sequences on the device: every layer and loop, then the

@@ -520,10 +520,11 @@ def norm_chain(r: torch.Tensor, *, x: torch.Tensor | None = None, w_a: torch.Ten
 def gemv_chain(r: torch.Tensor, weights, *, x: torch.Tensor | None = None, w_a: torch.Tensor | None = None,
                w_f: torch.Tensor | None = None, w_b: torch.Tensor | None = None, eps: float, want_h: bool = True,
                epilogue: int = EPI_PLAIN, addend: torch.Tensor | None = None,
-               rope: tuple[torch.Tensor, torch.Tensor] | None = None, head_dim: int = HEAD_DIM):
+               rope: tuple[torch.Tensor, torch.Tensor] | None = None, head_dim: int = HEAD_DIM,
+               out: torch.Tensor | None = None):
     """``norm_chain`` followed by ``gemv`` of its output (z, or h without ``w_b``) in one
     launch (``fl_gemv_bf16_chain``), bit-identical to the two calls.  Returns (h or None,
-    the GEMV output as ``gemv`` returns it)."""
+    the GEMV output as ``gemv`` returns it; ``out`` if given, where it has one tensor)."""
     r2 = _rows2d(r, "r")
     m, d = r2.shape
     x2 = None if x is None else _rows2d(x, "x")
@@ -536,7 +537,13 @@ def gemv_chain(r: torch.Tensor, weights, *, x: torch.Tensor | None = None, w_a: 
     n = ws[0].shape[0]
     dt = torch.float32 if epilogue == EPI_F32 else torch.bfloat16
     nout = 3 if epilogue == EPI_ROPE else 1
-    outs = [torch.empty(m, n, dtype=dt, device=r2.device) for _ in range(nout)]
+    if out is None:
+        outs = [torch.empty(m, n, dtype=dt, device=r2.device) for _ in range(nout)]
+    else:
+        _require(out, dt, "out")
+        if nout != 1 or out.shape != (m, n):
+            raise ValueError(f"out must be one [{m}, {n}] tensor")
+        outs = [out]
     add = None
     if epilogue == EPI_ADD:
         add = addend.reshape(m, n)
@@ -555,6 +562,26 @@ def gemv_chain(r: torch.Tensor, weights, *, x: torch.Tensor | None = None, w_a: 
     )
     check(rc, "fl_gemv_bf16_chain")
     return h, (tuple(outs) if epilogue == EPI_ROPE else outs[0])
+
+
+def decode_inputs(tokens: torch.Tensor, positions: torch.Tensor, table: torch.Tensor, inv_freq: torch.Tensor):
+    """Embedded tokens ``[B, 1, hidden]`` and the rotary ``cos`` / ``sin`` ``[B, 1, head_dim]`` of a
+    decode step (``fl_decode_inputs``): i64 ``tokens`` / ``positions`` [B, 1], a bf16 ``table``
+    [vocab, hidden], f32 or bf16 ``inv_freq`` [head_dim / 2]."""
+    b, (vocab, hidden), hd = tokens.shape[0], table.shape, 2 * inv_freq.numel()
+    for t, nm in ((tokens, "tokens"), (positions, "positions")):
+        _require(t, torch.int64, nm)
+        if t.shape != (b, 1):
+            raise ValueError(f"{nm} must be [B, 1]")
+    _require(table, torch.bfloat16, "table")
+    _require(inv_freq, torch.bfloat16 if inv_freq.dtype == torch.bfloat16 else torch.float32, "inv_freq")
+    h = torch.empty(b, 1, hidden, dtype=torch.bfloat16, device=tokens.device)
+    cos, sin = (torch.empty(b, 1, hd, dtype=torch.bfloat16, device=tokens.device) for _ in range(2))
+    rc = load().fl_decode_inputs(tokens.data_ptr(), positions.data_ptr(), b, table.data_ptr(), vocab, hidden,
+                                 inv_freq.data_ptr(), int(inv_freq.dtype == torch.bfloat16), hd, h.data_ptr(),
+                                 cos.data_ptr(), sin.data_ptr(), _stream())
+    check(rc, "fl_decode_inputs")
+    return h, cos, sin
 
 
 def append_tail(view, keys, values, tail_active, tail_tokens: torch.Tensor) -> None:

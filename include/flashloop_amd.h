@@ -451,6 +451,17 @@ int32_t fl_gemv_bf16(const void* x, int32_t x_is_f32, int64_t x_stride, int32_t 
                      int64_t addend_stride, const uint16_t* rope_cos, const uint16_t* rope_sin,
                      int32_t head_dim, void* stream);
 /*
+ * fl_decode_inputs: what a decode step reads first, per sequence b: h[b] = table[tokens[b]]
+ * (bf16 [vocab, hidden] and [batch, hidden], hidden % 8 == 0, 16-byte aligned) and the rotary
+ * rows cos / sin (bf16 [batch, head_dim], both halves alike) of the fp32 products
+ * positions[b] * inv_freq[i], i < head_dim / 2 (f32, or bf16).  tokens, positions: i64 [batch]
+ * in device memory; a token outside the table gives a row of NaN.
+ */
+int32_t fl_decode_inputs(const int64_t* tokens, const int64_t* positions, int32_t batch,
+                         const uint16_t* table, int64_t vocab, int32_t hidden, const void* inv_freq,
+                         int32_t freq_is_bf16, int32_t head_dim, uint16_t* h, uint16_t* rope_cos,
+                         uint16_t* rope_sin, void* stream);
+/*
  * fl_append_tail: the decode append of one layer (CrossLoopKVLayer.append_decode_token,
  * flashloop/cache.py:1758-1776, device half): for every sequence b, the step's rows
  * keys[r] / values[r] (bf16 [B*H, 128], r = loop 0..3) are written to tail_key[r] /

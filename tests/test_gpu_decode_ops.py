@@ -242,3 +242,21 @@ def test_gemv_rope_at_head_edges(m, heads, hd, k):
         # the dots' own roundings and each product's (2^-8 of its size, twice)
         slack = s + s.roll(hd // 2, dims=-1) + 2.0 ** -7 * (d.abs() + rot.abs())
         _near(got.view(m, heads, hd), want, slack, "rope")
+
+
+@pytest.mark.parametrize("b,d,hd,freq", [(1, 8, 2, torch.float32), (3, 2056, 126, torch.bfloat16), (8, 4096, 1024, torch.float32)])
+def test_decode_inputs(b, d, hd, freq):
+    """Embedding rows exactly; cos and sin of the fp32 angle: 2 ulp of an fp32 function (2^-22 at
+    most), then half a bf16 ulp.  A token outside the table gives a row of NaN."""
+    print(f"case: decode inputs b={b} d={d} hd={hd}", flush=True)
+    table = _x(50, d, 110)
+    tok = torch.tensor([[0], [49], [7], [50], [-1], [3], [1 << 40], [49]][:b], device=DEV)
+    pos = torch.tensor([[8191], [0], [1], [70000], [12345], [2], [64], [1 << 20]][:b], device=DEV)
+    inv = (1.0 / 10000.0 ** (torch.arange(0, hd, 2, device=DEV).float() / hd)).to(freq)
+    h, cos, sin = kernels.decode_inputs(tok, pos, table, inv)
+    ok = ((tok >= 0) & (tok < 50)).flatten()
+    assert torch.equal(h[ok], table[tok[ok]]) and h[~ok].isnan().all()
+    angle = (pos.float() * inv.float()[None]).double().cpu()
+    for got, want in ((cos, angle.cos()), (sin, angle.sin())):
+        want = torch.cat([want, want], -1)
+        assert ((got[:, 0].double().cpu() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -21).all()
