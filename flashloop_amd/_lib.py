@@ -102,6 +102,7 @@ SIGNATURES = {
                                   _I64, _P, _P, _I32, _P]),
     "fl_decode_inputs": (_I32, [_P, _P, _I32, _P, _I64, _I32, _P, _I32, _I32, _P, _P, _P, _P]),
     "fl_append_tail": (_I32, [_VIEW, _PP, _PP, _PP, _P, _P]),
+    "fl_append_tails": (_I32, [_PP, _I32, _PP, _PP, _PP, _PP, _P]),
     "fl_prefill_attention": (_I32, [_P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64, _I32, _I32, _I32, _P,
                                     _F32, _P, _SZ, _P]),
     "fl_prefill_attention_workspace": (_SZ, [_I32, _I32, _I32]),

@@ -428,11 +428,7 @@ class CrossLoopKVLayer:
         """Device half of an append: rows go to each sequence's device tail length, which is
         then incremented -- no host index, so the step can be captured in a HIP graph.
         ``commit_append`` must follow (host mirrors, rollover)."""
-        if len(keys) != 4 or len(values) != 4:
-            raise ValueError("exactly four loop K/V tensors are required")
-        if any(t >= self.geometry.tail_capacity for t in self.tail_host):
-            raise RuntimeError("tail is full; rollover did not run")
-        kernels.append_tail(self.view(), keys, values, self.tail_active, self.tail_tokens)
+        append_layer_rows([self], [keys], [values])
 
     def commit_append(self) -> None:
         """Host half of an append: mirrors follow the device lengths; roll full tails."""
@@ -595,6 +591,22 @@ class CrossLoopKVLayer:
     @property
     def dense_bf16_bytes(self) -> int:
         return 4 * 2 * self.heads * sum(p + t for p, t in zip(self.packed_host, self.tail_host)) * HEAD_DIM * 2
+
+
+def append_layer_rows(layers: Sequence[CrossLoopKVLayer], keys, values) -> None:
+    """``CrossLoopKVLayer.append_rows`` of several layers (``keys[i]`` / ``values[i]``: the four
+    loops' rows of layer i), in one launch where their geometry is the same."""
+    groups: dict[tuple, list] = {}
+    for layer, k, v in zip(layers, keys, values, strict=True):
+        if len(k) != 4 or len(v) != 4:
+            raise ValueError("exactly four loop K/V tensors are required")
+        if any(t >= layer.geometry.tail_capacity for t in layer.tail_host):
+            raise RuntimeError("tail is full; rollover did not run")
+        view = layer.view()
+        groups.setdefault((view.batch, view.heads, view.tail_capacity), []).append(
+            (view, k, v, layer.tail_active, layer.tail_tokens))
+    for members in groups.values():
+        kernels.append_tails(*zip(*members))
 
 
 class CrossLoopKVCache:

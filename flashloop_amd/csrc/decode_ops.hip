@@ -843,52 +843,51 @@ __global__ __launch_bounds__(MmGeom<MT>::kThreads, 2) void gemv_mfma_kernel(Gemv
 // ---------------------------------------------------------------------------------
 // Decode append: the step's K/V rows of the four loops go to each sequence's tail at its
 // device length, the loop-3/4 activity flags of that row are set, and the length is
-// incremented -- one workgroup per sequence, so the increment follows its own copies.
+// incremented -- one workgroup per sequence and layer, so the increment follows its own copies.
+// Bound by its launch, so a step's layers share one (a step of four layers 923 -> 916 us).
 constexpr int kAppendThreads = 256;
+constexpr int kAppendLayers = 16;  // per launch (kernel arguments: 160 bytes a layer)
 
+struct AppendLayer {
+  uint16_t* tail[8];       // tail_key of the four loops, then tail_value
+  const uint16_t* rows[8];  // [B*H, 128] bf16 rows of the step: keys, then values
+  uint8_t* active[2];      // [B, tail_capacity] loop-3/4 tail activity
+  int32_t* tail_tokens;    // the tail lengths, written
+};
 struct AppendArgs {
-  fl_cache_view v;
-  const uint16_t* k[4];  // [B*H, 128] bf16 rows of the step, per loop
-  const uint16_t* val[4];
-  uint8_t* active[2];  // [B, tail_capacity] loop-3/4 tail activity
-  int32_t* tail_tokens;  // the view's tail lengths, written
+  int heads, tail_capacity;
+  AppendLayer layer[kAppendLayers];
 };
 
 __global__ __launch_bounds__(kAppendThreads) void append_tail_kernel(AppendArgs a) {
-  const fl_cache_view& v = a.v;
+  const AppendLayer& l = a.layer[blockIdx.y];
   const int b = blockIdx.x;
-  constexpr int kChunks = kDim / 8;   // 16-byte chunks per row
-  const int per = v.heads * kChunks;  // chunks of one tensor for this sequence
-  // tensor t: loop t & 3, K for t < 4; t is a compile-time index in every use below (a
-  // runtime index into the argument arrays would load each pointer from memory first)
+  constexpr int kChunks = kDim / 8;     // 16-byte chunks per row
+  const int per = a.heads * kChunks;    // chunks of one tensor for this sequence
   auto src_of = [&](int t, int i) __attribute__((always_inline)) {
-    const uint16_t* base = t < 4 ? a.k[t & 3] : a.val[t & 3];
-    const int h = i / kChunks, c = i - h * kChunks;
-    return reinterpret_cast<const uint4*>(base + (static_cast<int64_t>(b) * v.heads + h) * kDim) + c;
+    return reinterpret_cast<const uint4*>(l.rows[t] + static_cast<int64_t>(b) * a.heads * kDim) + i;
   };
   auto dst_of = [&](int t, int i, int pos) __attribute__((always_inline)) {
-    uint16_t* base = static_cast<uint16_t*>(t < 4 ? v.tail_key[t & 3] : v.tail_value[t & 3]);
     const int h = i / kChunks, c = i - h * kChunks;
-    return reinterpret_cast<uint4*>(base + ((static_cast<int64_t>(b) * v.heads + h) * v.tail_capacity + pos) * kDim) +
-           c;
+    return reinterpret_cast<uint4*>(l.tail[t] + ((static_cast<int64_t>(b) * a.heads + h) * a.tail_capacity + pos) * kDim) + c;
   };
   // chunk threadIdx.x of each of the 8 tensors is requested before the first store (the
   // rows do not depend on the tail length, loaded alongside): one memory round trip
-  const int pos = v.tail_tokens[b];
+  const int pos = l.tail_tokens[b];
   const int i0 = threadIdx.x;
   uint4 held[8];
 #pragma unroll
   for (int t = 0; t < 8; ++t) held[t] = i0 < per ? *src_of(t, i0) : make_uint4(0, 0, 0, 0);
-  if (pos < 0 || pos >= v.tail_capacity) return;  // the host rolls over before the tail is full
+  if (pos < 0 || pos >= a.tail_capacity) return;  // the host rolls over before the tail is full
 #pragma unroll
   for (int t = 0; t < 8; ++t)
     if (i0 < per) *dst_of(t, i0, pos) = held[t];
   for (int i = i0 + kAppendThreads; i < per; i += kAppendThreads)  // more than 16 heads
 #pragma unroll
     for (int t = 0; t < 8; ++t) *dst_of(t, i, pos) = *src_of(t, i);
-  if (threadIdx.x < 2) a.active[threadIdx.x][static_cast<int64_t>(b) * v.tail_capacity + pos] = 1;
+  if (threadIdx.x < 2) l.active[threadIdx.x][static_cast<int64_t>(b) * a.tail_capacity + pos] = 1;
   __syncthreads();
-  if (threadIdx.x == 0) a.tail_tokens[b] = pos + 1;
+  if (threadIdx.x == 0) l.tail_tokens[b] = pos + 1;
 }
 
 // ---------------------------------------------------------------------------------
@@ -1144,29 +1143,53 @@ extern "C" int32_t fl_decode_inputs(const int64_t* tokens, const int64_t* positi
   return FL_OK;
 }
 
+extern "C" int32_t fl_append_tails(const fl_cache_view* const* views, int32_t layers, const uint16_t* const* keys,
+                                   const uint16_t* const* values, uint8_t* const* tail_active,
+                                   int32_t* const* tail_tokens, void* stream) {
+  using namespace fl;
+  clear_error();
+  FL_REQUIRE(views && keys && values && tail_active && tail_tokens && layers > 0, "fl_append_tail: null argument");
+  for (int i = 0; i < layers; ++i) {
+    FL_REQUIRE(views[i], "fl_append_tail: null argument");
+    const fl_cache_view& v = *views[i];
+    FL_REQUIRE(v.batch > 0 && v.heads > 0 && v.tail_capacity > 0 && v.tail_tokens, "fl_append_tail: bad view");
+    FL_REQUIRE(v.batch == views[0]->batch && v.heads == views[0]->heads && v.tail_capacity == views[0]->tail_capacity,
+               "fl_append_tails: the layers differ in batch, heads or tail capacity");
+    FL_REQUIRE(tail_tokens[i] == v.tail_tokens, "fl_append_tail: tail_tokens must be the view's length array");
+    for (int r = 4 * i; r < 4 * i + 4; ++r) {
+      FL_REQUIRE(keys[r] && values[r] && v.tail_key[r & 3] && v.tail_value[r & 3], "fl_append_tail: null row or tail");
+      FL_REQUIRE(reinterpret_cast<uintptr_t>(keys[r]) % 16 == 0 && reinterpret_cast<uintptr_t>(values[r]) % 16 == 0,
+                 "fl_append_tail: rows must be 16-byte aligned");
+    }
+    FL_REQUIRE(tail_active[2 * i] && tail_active[2 * i + 1], "fl_append_tail: null tail_active");
+  }
+  for (int i0 = 0; i0 < layers; i0 += kAppendLayers) {
+    const int n = layers - i0 < kAppendLayers ? layers - i0 : kAppendLayers;
+    AppendArgs a{};
+    a.heads = views[0]->heads;
+    a.tail_capacity = views[0]->tail_capacity;
+    for (int j = 0; j < n; ++j) {
+      const int i = i0 + j;
+      AppendLayer& l = a.layer[j];
+      for (int r = 0; r < 4; ++r) {
+        l.tail[r] = static_cast<uint16_t*>(views[i]->tail_key[r]);
+        l.tail[4 + r] = static_cast<uint16_t*>(views[i]->tail_value[r]);
+        l.rows[r] = keys[4 * i + r];
+        l.rows[4 + r] = values[4 * i + r];
+      }
+      l.active[0] = tail_active[2 * i];
+      l.active[1] = tail_active[2 * i + 1];
+      l.tail_tokens = tail_tokens[i];
+    }
+    hipLaunchKernelGGL(append_tail_kernel, dim3(views[0]->batch, n), dim3(kAppendThreads), 0,
+                       static_cast<hipStream_t>(stream), a);
+    FL_LAUNCH_CHECK("fl_append_tail");
+  }
+  return FL_OK;
+}
+
 extern "C" int32_t fl_append_tail(const fl_cache_view* view, const uint16_t* const* keys,
                                   const uint16_t* const* values, uint8_t* const* tail_active,
                                   int32_t* tail_tokens, void* stream) {
-  using namespace fl;
-  clear_error();
-  FL_REQUIRE(view && keys && values && tail_active, "fl_append_tail: null argument");
-  const fl_cache_view& v = *view;
-  FL_REQUIRE(v.batch > 0 && v.heads > 0 && v.tail_capacity > 0 && v.tail_tokens, "fl_append_tail: bad view");
-  FL_REQUIRE(tail_tokens == v.tail_tokens, "fl_append_tail: tail_tokens must be the view's length array");
-  AppendArgs a{};
-  a.v = v;
-  for (int r = 0; r < 4; ++r) {
-    FL_REQUIRE(keys[r] && values[r] && v.tail_key[r] && v.tail_value[r], "fl_append_tail: null row or tail");
-    FL_REQUIRE(reinterpret_cast<uintptr_t>(keys[r]) % 16 == 0 && reinterpret_cast<uintptr_t>(values[r]) % 16 == 0,
-               "fl_append_tail: rows must be 16-byte aligned");
-    a.k[r] = keys[r];
-    a.val[r] = values[r];
-  }
-  FL_REQUIRE(tail_active[0] && tail_active[1], "fl_append_tail: null tail_active");
-  a.active[0] = tail_active[0];
-  a.active[1] = tail_active[1];
-  a.tail_tokens = tail_tokens;
-  hipLaunchKernelGGL(append_tail_kernel, dim3(v.batch), dim3(kAppendThreads), 0, static_cast<hipStream_t>(stream), a);
-  FL_LAUNCH_CHECK("fl_append_tail");
-  return FL_OK;
+  return fl_append_tails(&view, 1, keys, values, tail_active, &tail_tokens, stream);
 }

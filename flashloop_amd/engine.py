@@ -29,7 +29,7 @@ import torch
 import torch.nn.functional as F
 
 from . import kernels
-from .cache import CrossLoopKVCache, CrossLoopKVLayer
+from .cache import CrossLoopKVCache, CrossLoopKVLayer, append_layer_rows
 from .config import FlashLoopConfig, validate_ouro_model
 from .model import MLP, Attention, OuroConfig, OuroForCausalLM, RMSNorm, RotaryEmbedding, apply_rope
 
@@ -582,8 +582,7 @@ class FlashLoopEngine:
                 last = li == nl - 1
                 nxt = None if (last and loop == 3) else layers_w[(li + 1) % nl]["ln1"]
                 pending = dict(x=mo, w_a=w["ln4"], w_f=extra["norm"] if last else None, w_b=nxt)
-        for li in range(nl):
-            cache.layers[li].append_rows(cur_k[li], cur_v[li])
+        append_layer_rows(cache.layers, cur_k, cur_v)
         # the last chain (final norm, no input norm) feeds lm_head
         return chain_gemv([extra["lm_head"]], epilogue=kernels.EPI_F32, **({"out": logits_out} if chained else {}))
 
@@ -640,8 +639,7 @@ class FlashLoopEngine:
                 h = residual + layer.input_layernorm_2(projected)
                 h = h + layer.post_attention_layernorm_2(layer.mlp(layer.post_attention_layernorm(h)))
             h = self.backbone.norm(h)
-        for li in range(nl):
-            cache.layers[li].append_rows(cur_k[li], cur_v[li])
+        append_layer_rows(cache.layers, cur_k, cur_v)
         return self.model.lm_head(h[:, -1]).float()
 
     def _receipt(self, positions: Sequence[int]) -> DecodeReceipt:

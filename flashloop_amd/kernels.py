@@ -585,20 +585,26 @@ def decode_inputs(tokens: torch.Tensor, positions: torch.Tensor, table: torch.Te
 
 
 def append_tail(view, keys, values, tail_active, tail_tokens: torch.Tensor) -> None:
-    """Device half of a decode append (``fl_append_tail``): rows ``keys[r]``/``values[r]``
-    ([B, H, 1, 128] bf16, r = loop) to each sequence's tail at its device length."""
-    rows = view.batch * view.heads
-    ks = [_vec(k, rows, "key") for k in keys]
-    vs = [_vec(v, rows, "value") for v in values]
-    for t in tail_active:
+    """``append_tails`` of one layer."""
+    append_tails([view], [keys], [values], [tail_active], [tail_tokens])
+
+
+def append_tails(views, keys, values, tail_active, tail_tokens) -> None:
+    """Device half of a decode append for several layers of one geometry (``fl_append_tails``):
+    rows ``keys[i][r]`` / ``values[i][r]`` ([B, H, 1, 128] bf16, layer i, loop r) to each
+    sequence's tail at its device length."""
+    rows = views[0].batch * views[0].heads
+    ks = [_vec(k, rows, "key") for layer in keys for k in layer]
+    vs = [_vec(v, rows, "value") for layer in values for v in layer]
+    active = [t for pair in tail_active for t in pair]
+    for t in active:
         _require(t, torch.uint8, "tail_active")
-    _require(tail_tokens, torch.int32, "tail_tokens")
-    rc = load().fl_append_tail(
-        C.byref(view), C.cast(ptr_array([k.data_ptr() for k in ks]), _lib._PP),
-        C.cast(ptr_array([v.data_ptr() for v in vs]), _lib._PP),
-        C.cast(ptr_array([t.data_ptr() for t in tail_active]), _lib._PP), tail_tokens.data_ptr(), _stream(),
-    )
-    check(rc, "fl_append_tail")
+    for t in tail_tokens:
+        _require(t, torch.int32, "tail_tokens")
+    arrays = [C.cast(ptr_array(p), _lib._PP) for p in (
+        [C.addressof(v) for v in views], [k.data_ptr() for k in ks], [v.data_ptr() for v in vs],
+        [t.data_ptr() for t in active], [t.data_ptr() for t in tail_tokens])]
+    check(load().fl_append_tails(arrays[0], len(views), *arrays[1:], _stream()), "fl_append_tails")
 
 
 # ---------------------------------------------------------------------------- prefill ops

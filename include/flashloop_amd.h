@@ -470,10 +470,15 @@ int32_t fl_decode_inputs(const int64_t* tokens, const int64_t* positions, int32_
  * length array, passed writable) -- all on the device, so
  * a captured step replays it.  A sequence whose tail is full is left unchanged (the
  * caller rolls a group out first).
+ * fl_append_tails: the same for several layers with one batch, head count and tail capacity:
+ * keys / values of layer i at 4 i + r, tail_active at 2 i + j; one launch for every 16 layers.
  */
 int32_t fl_append_tail(const fl_cache_view* view, const uint16_t* const* keys,
                        const uint16_t* const* values, uint8_t* const* tail_active,
                        int32_t* tail_tokens, void* stream);
+int32_t fl_append_tails(const fl_cache_view* const* views, int32_t layers, const uint16_t* const* keys,
+                        const uint16_t* const* values, uint8_t* const* tail_active,
+                        int32_t* const* tail_tokens, void* stream);
 int32_t fl_norm_chain(int32_t m, int32_t d, float eps, const uint16_t* x, const uint16_t* r,
                       const uint16_t* w_a, const uint16_t* w_f, const uint16_t* w_b,
                       uint16_t* h_out, uint16_t* z_out, int64_t stride, void* stream);

@@ -7,6 +7,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 from flashloop_amd import CrossLoopKVLayer, packed_prefix_tokens  # noqa: E402
+from flashloop_amd.cache import append_layer_rows  # noqa: E402
 
 DEV = "cuda"
 
@@ -114,3 +115,30 @@ def test_rollover_of_a_ragged_batch_equals_torch():
                 n = layer.tail_host[i]
                 assert torch.equal(after[name][rows, :n], want[:, 64:64 + n] if i in (0, 2) else want[:, :n]), name
     assert layer.late_rows_host == after["late_rows"].tolist()
+
+
+@pytest.mark.parametrize("layers,b,h", [(1, 1, 1), (16, 3, 17), (18, 2, 2)])
+def test_append_of_many_layers_equals_torch(layers, b, h):
+    """One launch per 16 layers, a layer of another geometry in a launch of its own, more chunks
+    than threads (17 heads): rows and flags at each sequence's tail, lengths one up."""
+    print(f"case: append layers={layers} b={b} h={h}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(95)
+    kv = [_kv(g, b, h, 150) for _ in range(2)]
+    lengths = [150, 70, 129][:b]
+    ls = [CrossLoopKVLayer.from_prefill(*kv, lengths=lengths) for _ in range(layers)]
+    ls.append(CrossLoopKVLayer.from_prefill(*([x[:1] for x in y] for y in kv)))
+    rows = [[[torch.randn(x.batch, h, 1, 128, generator=g, device=DEV).to(torch.bfloat16) for _ in range(4)] for x in ls] for _ in range(2)]
+    want = [{k: v.clone() for k, v in x.state_dict()[0].items()} for x in ls]
+    append_layer_rows(ls, *rows)
+    for i, (layer, w) in enumerate(zip(ls, want)):
+        for b_ in range(layer.batch):
+            at = int(w["tail_tokens"][b_])
+            for r in range(4):
+                w[f"tail_key.{r}"][b_ * h:(b_ + 1) * h, at] = rows[0][i][r][b_, :, 0]
+                w[f"tail_value.{r}"][b_ * h:(b_ + 1) * h, at] = rows[1][i][r][b_, :, 0]
+            for s in range(2):
+                w[f"tail_active.{s}"][b_, at] = 1
+            w["tail_tokens"][b_] += 1
+        got = layer.state_dict()[0]
+        assert got.keys() == w.keys()  # (bytes: the tails' unused rows may hold anything)
+        assert [k for k in w if not torch.equal(got[k].contiguous().view(torch.uint8), w[k].contiguous().view(torch.uint8))] == [], i
