@@ -66,16 +66,13 @@ class CrossLoopKVLayer:
         self.device = dev = torch.device(device)
         rows = g.batch * g.heads
         new = torch.zeros if _buffers is None else torch.empty
-        fixed = _buffers or self._fixed_buffers(g.batch, g.heads, g.token_capacity, g.tail_capacity, dev, new)
+        fixed = _buffers or self._fixed_buffers(g.batch, g.heads, g.token_capacity, g.row_capacity[2:], g.tail_capacity, dev, new)
         for name, x in fixed.items():
             setattr(self, name, x)
         if _buffers is None:
             for r in self.rank:
                 r.fill_(-1)
-        # streams 2/3 hold the rows that loops 3/4 keep; one 128-byte line per token and stream:
-        # K codes in bytes 0..63, V codes in 64..127
-        for s in (2, 3):
-            n = g.row_capacity[s]
+        for n in g.row_capacity[len(self.codes):]:  # streams whose size was not known to _fixed_buffers
             self.codes.append(new(rows, n, 2 * (HEAD_DIM // 2), dtype=torch.uint8, device=dev))
             self.value_meta.append(new(rows, n, 2, 2, dtype=torch.float32, device=dev))
             self.value_meta_half.append(new(rows, n, 2, 2, dtype=torch.float16, device=dev))
@@ -94,21 +91,25 @@ class CrossLoopKVLayer:
         self.workspace = kernels.Workspace()
 
     @staticmethod
-    def _fixed_buffers(batch: int, heads: int, cap: int, tail: int, dev, new) -> dict:
-        """The layer's buffers whose size does not follow from the rows loops 3/4 keep (of the
-        lists per stream, streams 0 and 1), made by ``new`` (``torch.zeros`` or ``torch.empty``)."""
+    def _fixed_buffers(batch: int, heads: int, cap: int, late: Sequence[int], tail: int, dev, new) -> dict:
+        """The layer's buffers, made by ``new`` (``torch.zeros`` or ``torch.empty``); of the lists
+        per stream streams 0 and 1, and streams 2/3 (the rows that loops 3/4 keep) if ``late``
+        gives their capacities.  Made stream by stream where they are known: with streams 2/3
+        last the gathers of a ragged batch of 32 took 1.5 us longer each (step 655 -> 659 us)."""
+        row_capacity = (cap, cap, *late)
         rows, groups = batch * heads, cap // GROUP
         f32, f16, i32, bf16, u8 = torch.float32, torch.float16, torch.int32, torch.bfloat16, torch.uint8
         return dict(
-            codes=[new(rows, cap, 2 * (HEAD_DIM // 2), dtype=u8, device=dev) for _ in range(2)],
+            # one 128-byte line per token and stream: K codes in bytes 0..63, V codes in 64..127
+            codes=[new(rows, n, 2 * (HEAD_DIM // 2), dtype=u8, device=dev) for n in row_capacity],
             key_meta=[new(rows, groups, HEAD_DIM, 2, dtype=f32, device=dev) for _ in range(4)],
-            value_meta=[new(rows, cap, 2, 2, dtype=f32, device=dev) for _ in range(2)],
+            value_meta=[new(rows, n, 2, 2, dtype=f32, device=dev) for n in row_capacity],
             # the V metadata of all four streams again, one 64-byte record per logical token
             # ([half][stream][scale, min]) for the readers of selected tokens
             value_meta_token=new(rows, cap, 2, 4, 2, dtype=f32, device=dev),
             # fp16 copies of the metadata, streamed by the readers
             key_meta_half=[new(rows, groups, HEAD_DIM, 2, dtype=f16, device=dev) for _ in range(4)],
-            value_meta_half=[new(rows, cap, 2, 2, dtype=f16, device=dev) for _ in range(2)],
+            value_meta_half=[new(rows, n, 2, 2, dtype=f16, device=dev) for n in row_capacity],
             rank=[new(batch, cap, dtype=i32, device=dev) for _ in range(2)],
             tail_key=[new(rows, tail, HEAD_DIM, dtype=bf16, device=dev) for _ in range(4)],
             tail_value=[new(rows, tail, HEAD_DIM, dtype=bf16, device=dev) for _ in range(4)],
@@ -226,20 +227,25 @@ class CrossLoopKVLayer:
         tp = [packed_prefix_tokens(x) for x in lengths]
         tp_max = max(tp)
         cap = _round_up(max(token_capacity or 0, tp_max, GROUP), GROUP)
-        # the late-row count is under way while the buffers that do not need it are allocated
-        count = cls._start_late_count(masks, tp) if late_counts is None else None
-        fixed = cls._fixed_buffers(b, h, cap, 2 * GROUP, dev, torch.empty)
-        src_k, src_v = [x.contiguous() for x in keys], [x.contiguous() for x in values]
-        group0 = torch.empty(b, dtype=torch.int32, device=dev)
-        if late_counts is None:
-            late = cls._finish_late_count(count, tp)
+        growth = cap - min(tp)  # every future decode token is active in every loop
+        late, count = late_counts, None
+        if late is None:
+            count = cls._start_late_count(masks, tp)
+            late = cls._finish_late_count(None, tp) if count is None else None
         else:
             late = [[int(x) for x in c] for c in late_counts]
             if len(late) != 2 or any(len(c) != b or min(c) < 0 for c in late):
                 raise ValueError("late_counts must give a count per sequence for loops 3 and 4")
-        growth = cap - min(tp)  # every future decode token is active in every loop
-        row_cap = (cap, cap, max(max(late[0]) + growth, 1), max(max(late[1]) + growth, 1))
-        layer = cls(LayerGeometry(b, h, cap, 2 * GROUP, row_cap), dev, _buffers=fixed)
+        # a late-row count on the device is under way while the buffers that do not need it are
+        # allocated
+        late_cap = () if late is None else tuple(max(max(c) + growth, 1) for c in late)
+        fixed = cls._fixed_buffers(b, h, cap, late_cap, 2 * GROUP, dev, torch.empty)
+        src_k, src_v = [x.contiguous() for x in keys], [x.contiguous() for x in values]
+        group0 = torch.empty(b, dtype=torch.int32, device=dev)
+        if late is None:
+            late = cls._finish_late_count(count, tp)
+            late_cap = tuple(max(max(c) + growth, 1) for c in late)
+        layer = cls(LayerGeometry(b, h, cap, 2 * GROUP, (cap, cap, *late_cap)), dev, _buffers=fixed)
         layer.late_rows_host = late
         layer.packed_host = list(tp)
         layer.tail_host = [x - p for x, p in zip(lengths, tp)]
