@@ -272,9 +272,9 @@ class FlashLoopEngine:
                     and getattr(m, "bias", None) is None and w.dtype == torch.bfloat16 and w.is_cuda and w.is_contiguous())
 
         d = hidden.shape[-1]
-        if hidden.dtype != torch.bfloat16 or d % 8 or d > 8192:
+        if hidden.dtype != torch.bfloat16 or d % 8 or d > 8192 or not plain(self.backbone.norm, RMSNorm):
             return None
-        eps = {self.backbone.norm.eps} if plain(self.backbone.norm, RMSNorm) else set()
+        eps = {self.backbone.norm.eps}
         layers = []
         for layer in self.layers:
             a, m = layer.self_attn, layer.mlp

@@ -1,0 +1,56 @@
+"""Which prefill path a model takes: the HIP row kernels for plain modules, the modules themselves
+where one is replaced, hooked or laid out otherwise.  The reference is the dense looped model
+(``dense_forward``), which always calls the modules."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from flashloop_amd.config import FlashLoopConfig  # noqa: E402
+from flashloop_amd.engine import FlashLoopEngine  # noqa: E402
+from flashloop_amd.model import OuroConfig, OuroForCausalLM, RMSNorm  # noqa: E402
+
+TINY = OuroConfig(vocab_size=1024, hidden_size=256, intermediate_size=512, num_hidden_layers=2,
+                  num_attention_heads=2, num_key_value_heads=2)
+ALL_ROWS = FlashLoopConfig(prefill_fraction_loop3=1.0, prefill_fraction_loop4=1.0)
+IDS = torch.randint(0, TINY.vocab_size, (1, 150), generator=torch.Generator().manual_seed(120))
+
+
+def _model():
+    return OuroForCausalLM.random_init(TINY, seed=121, device="cuda")
+
+
+def _rel(got, want):
+    return float((got.double() - want.double()).norm() / want.double().norm())
+
+
+def _like_the_modules(model, what):
+    """Prefill with every row active equals the dense model.  Bound: about ten bf16 roundings
+    (2^-9 each) in each of 2 layers x 4 loops, adding up at random: sqrt(80) * 2^-9 = 1.8e-2."""
+    ids = IDS.cuda()
+    got, want = FlashLoopEngine(model, config=ALL_ROWS).prefill(ids).logits, model.dense_forward(ids)
+    assert _rel(got, want) < 3e-2, f"{what}: {_rel(got, want):.3e} from the modules"
+    return want
+
+
+def test_hooked_final_norm_is_called():
+    print("case: hooked final norm", flush=True)
+    model = _model()
+    calls = []
+    model.model.norm.register_forward_hook(lambda m, a, out: (calls.append(1), out * 3.0)[1])
+    plain = _like_the_modules(_model(), "plain")
+    hooked = _like_the_modules(model, "hooked final norm")
+    assert len(calls) == 8 and _rel(hooked, plain) > 0.1  # (both models, four loops each; the change is well past the bound)
+
+
+def test_final_norm_of_another_class_is_called():
+    """A subclass with its own eps, large enough to matter."""
+    print("case: final norm of another class", flush=True)
+
+    class Other(RMSNorm):
+        pass
+
+    model = _model()
+    model.model.norm = Other(TINY.hidden_size, 4.0).to("cuda", torch.bfloat16)
+    assert _rel(_like_the_modules(model, "another class"), _like_the_modules(_model(), "plain")) > 0.1
