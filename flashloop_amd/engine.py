@@ -34,6 +34,18 @@ from .config import FlashLoopConfig, validate_ouro_model
 from .model import MLP, Attention, OuroConfig, OuroForCausalLM, RMSNorm, RotaryEmbedding, apply_rope
 
 
+_FORWARD = {kind: kind.forward for kind in (torch.nn.Linear, torch.nn.Embedding, RMSNorm, RotaryEmbedding, MLP)}
+
+
+def _is_plain(m: torch.nn.Module, kind: type) -> bool:
+    """Whether calling ``m`` runs the ``forward`` that ``kind`` was defined with and nothing else: no
+    subclass, no ``forward`` replaced on the instance or the class, no hook on it or on every module."""
+    every = torch.nn.modules.module
+    return (type(m) is kind and getattr(m.forward, "__func__", None) is _FORWARD[kind]
+            and not (m._forward_hooks or m._forward_pre_hooks
+                     or every._global_forward_hooks or every._global_forward_pre_hooks))
+
+
 @dataclass(frozen=True)
 class PrefillReceipt:
     """Row accounting of one prefill loop (flashloop/prefill.py:46-58)."""
@@ -264,12 +276,11 @@ class FlashLoopEngine:
 
     def _prefill_weights(self, hidden: torch.Tensor):
         """Per-layer weights of the HIP prefill path and its norm epsilon, or None when a module
-        is not a plain bf16 ``nn.Linear`` / ``RMSNorm`` on the device (a wrapped or hooked
-        module keeps the module path, which calls it)."""
+        is not a plain bf16 ``nn.Linear`` / ``RMSNorm`` on the device (a wrapped, replaced or
+        hooked module keeps the module path, which calls it)."""
         def plain(m, kind) -> bool:
-            w = m.weight
-            return (type(m) is kind and not m._forward_hooks and not m._forward_pre_hooks
-                    and getattr(m, "bias", None) is None and w.dtype == torch.bfloat16 and w.is_cuda and w.is_contiguous())
+            return (_is_plain(m, kind) and getattr(m, "bias", None) is None and m.weight.dtype == torch.bfloat16
+                    and m.weight.is_cuda and m.weight.is_contiguous())
 
         d = hidden.shape[-1]
         if hidden.dtype != torch.bfloat16 or d % 8 or d > 8192 or not plain(self.backbone.norm, RMSNorm):
@@ -281,8 +292,7 @@ class FlashLoopEngine:
             lin = (a.q_proj, a.k_proj, a.v_proj, a.o_proj, m.gate_proj, m.up_proj, m.down_proj)
             norms = (layer.input_layernorm, layer.input_layernorm_2, layer.post_attention_layernorm,
                      layer.post_attention_layernorm_2)
-            if (type(a) is not Attention or type(m) is not MLP or m._forward_hooks or m._forward_pre_hooks
-                    or m.gate_proj.weight.shape[0] % 8
+            if (type(a) is not Attention or not _is_plain(m, MLP) or m.gate_proj.weight.shape[0] % 8
                     or not all(plain(x, torch.nn.Linear) for x in lin) or not all(plain(x, RMSNorm) for x in norms)):
                 return None
             eps.update(x.eps for x in norms)
@@ -472,8 +482,7 @@ class FlashLoopEngine:
         """Embedded tokens, cos and sin of a decode step: one launch where the two modules are
         the plain ones on the device (a replaced or hooked module is called)."""
         emb, rot = self.backbone.embed_tokens, self.backbone.rotary_emb
-        if (type(emb) is torch.nn.Embedding and type(rot) is RotaryEmbedding
-                and not any(m._forward_hooks or m._forward_pre_hooks or "forward" in vars(m) for m in (emb, rot))
+        if (_is_plain(emb, torch.nn.Embedding) and _is_plain(rot, RotaryEmbedding)
                 and emb.max_norm is None and token_ids.dtype == torch.long
                 and all(t.is_cuda and t.is_contiguous() for t in (token_ids, pos_t, emb.weight, rot.inv_freq))
                 and emb.weight.dtype == torch.bfloat16 and emb.weight.shape[1] % 8 == 0 and emb.weight.data_ptr() % 16 == 0

@@ -54,3 +54,54 @@ def test_final_norm_of_another_class_is_called():
     model = _model()
     model.model.norm = Other(TINY.hidden_size, 4.0).to("cuda", torch.bfloat16)
     assert _rel(_like_the_modules(model, "another class"), _like_the_modules(_model(), "plain")) > 0.1
+
+
+REPLACED = ["model.layers.1.self_attn.q_proj", "model.layers.0.self_attn.o_proj", "model.layers.0.mlp.up_proj",
+            "model.layers.1.mlp", "model.layers.0.input_layernorm", "model.layers.1.post_attention_layernorm_2", "model.norm"]
+
+
+@pytest.mark.parametrize("name", REPLACED)
+def test_replaced_forward_is_called(name):
+    """A ``forward`` replaced on the instance, as wrapping and offloading tools do it."""
+    print(f"case: replaced forward {name}", flush=True)
+    model = _model()
+    m = model.get_submodule(name)
+    calls, forward = [], m.forward
+    m.forward = lambda x: (calls.append(1), forward(x) * 2.0)[1]
+    _like_the_modules(model, name)
+    assert len(calls) == 8  # (both models, four loops each)
+
+
+def test_class_forward_and_global_hook_are_called():
+    """A class whose ``forward`` was replaced, and a hook on every module."""
+    print("case: replaced class forward, global hook", flush=True)
+    plain = _like_the_modules(_model(), "plain")
+    forward = RMSNorm.forward
+    RMSNorm.forward = lambda self, x: forward(self, x) * 2.0
+    try:
+        assert _rel(_like_the_modules(_model(), "class forward"), plain) > 0.1
+    finally:
+        RMSNorm.forward = forward
+    hook = torch.nn.modules.module.register_module_forward_hook(
+        lambda m, a, out: out * 2.0 if isinstance(m, RMSNorm) else None)
+    try:
+        assert _rel(_like_the_modules(_model(), "global hook"), plain) > 0.1
+    finally:
+        hook.remove()
+
+
+def test_replaced_embedding_and_rotary_of_a_decode_step_are_called():
+    print("case: replaced embedding and rotary", flush=True)
+    ids = IDS.cuda()
+    for name in ("model.embed_tokens", "model.rotary_emb"):
+        model = _model()
+        eng = FlashLoopEngine(model, use_graphs=False)
+        eng.prefill(ids)
+        m = model.get_submodule(name)
+        calls, forward = [], type(m).forward
+        type(m).forward = lambda self, *a: (calls.append(1), forward(self, *a))[1]
+        try:
+            eng.decode(ids[:, :1])
+        finally:
+            type(m).forward = forward
+        assert len(calls) == 1, name
