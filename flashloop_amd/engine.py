@@ -283,9 +283,10 @@ class FlashLoopEngine:
                     and m.weight.is_cuda and m.weight.is_contiguous())
 
         d = hidden.shape[-1]
-        if hidden.dtype != torch.bfloat16 or d % 8 or d > 8192 or not plain(self.backbone.norm, RMSNorm):
-            return None
-        eps = {self.backbone.norm.eps}
+        final = self.backbone.norm
+        if hidden.dtype != torch.bfloat16 or d % 8 or d > 8192 or not plain(final, RMSNorm) or final.weight.data_ptr() % 16:
+            return None  # (fl_norm_chain loads 16 bytes of up to 8192 values)
+        eps = {final.eps}
         layers = []
         for layer in self.layers:
             a, m = layer.self_attn, layer.mlp
@@ -293,7 +294,8 @@ class FlashLoopEngine:
             norms = (layer.input_layernorm, layer.input_layernorm_2, layer.post_attention_layernorm,
                      layer.post_attention_layernorm_2)
             if (type(a) is not Attention or not _is_plain(m, MLP) or m.gate_proj.weight.shape[0] % 8
-                    or not all(plain(x, torch.nn.Linear) for x in lin) or not all(plain(x, RMSNorm) for x in norms)):
+                    or not all(plain(x, torch.nn.Linear) for x in lin)
+                    or not all(plain(x, RMSNorm) and x.weight.data_ptr() % 16 == 0 for x in norms)):
                 return None
             eps.update(x.eps for x in norms)
             layers.append(tuple(x.weight for x in (*lin, *norms)))

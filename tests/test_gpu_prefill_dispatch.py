@@ -105,3 +105,14 @@ def test_replaced_embedding_and_rotary_of_a_decode_step_are_called():
         finally:
             type(m).forward = forward
         assert len(calls) == 1, name
+
+
+@pytest.mark.parametrize("name", ["model.norm", "model.layers.1.post_attention_layernorm"])
+def test_misaligned_norm_weight(name):
+    """A norm weight that starts two bytes into its storage, which a 16-byte load cannot take."""
+    print(f"case: misaligned {name}", flush=True)
+    model = _model()
+    w = torch.rand(TINY.hidden_size + 1, device="cuda", generator=torch.Generator("cuda").manual_seed(122)).add_(0.5).bfloat16()[1:]
+    assert w.data_ptr() % 16 == 2
+    model.get_submodule(name).weight = torch.nn.Parameter(w)
+    _like_the_modules(model, "misaligned norm weight")
