@@ -274,10 +274,11 @@ class FlashLoopEngine:
         v = attn.v_proj(x).view(bsz, rows, -1, attn.head_dim).transpose(1, 2)
         return q, k, v
 
-    def _prefill_weights(self, hidden: torch.Tensor):
+    def _prefill_weights(self, hidden: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor):
         """Per-layer weights of the HIP prefill path and its norm epsilon, or None when a module
         is not a plain bf16 ``nn.Linear`` / ``RMSNorm`` on the device (a wrapped, replaced or
-        hooked module keeps the module path, which calls it)."""
+        hooked module keeps the module path, which calls it), or when the embedding or the
+        rotary module (called on both paths) gave rows in another layout than the kernels read."""
         def plain(m, kind) -> bool:
             return (_is_plain(m, kind) and getattr(m, "bias", None) is None and m.weight.dtype == torch.bfloat16
                     and m.weight.is_cuda and m.weight.is_contiguous())
@@ -286,6 +287,10 @@ class FlashLoopEngine:
         final = self.backbone.norm
         if hidden.dtype != torch.bfloat16 or d % 8 or d > 8192 or not plain(final, RMSNorm) or final.weight.data_ptr() % 16:
             return None  # (fl_norm_chain loads 16 bytes of up to 8192 values)
+        table = (1, hidden.shape[1], self.layers[0].self_attn.head_dim)
+        if (any(not x.is_contiguous() or x.data_ptr() % 16 for x in (hidden, cos, sin))
+                or any(tuple(x.shape) != table or x.dtype != torch.bfloat16 or not x.is_cuda for x in (cos, sin))):
+            return None
         eps = {final.eps}
         layers = []
         for layer in self.layers:
@@ -328,7 +333,7 @@ class FlashLoopEngine:
 
     def _dense_loop(self, hidden: torch.Tensor, cos, sin):
         """``dense_prefill_loop`` (flashloop/prefill.py:275-304): every row, causal attention."""
-        weights = self._prefill_weights(hidden)
+        weights = self._prefill_weights(hidden, cos, sin)
         if weights is None:
             return self._dense_loop_modules(hidden, cos, sin)
         _, t, d = hidden.shape
@@ -342,7 +347,7 @@ class FlashLoopEngine:
     def _sparse_loop(self, hidden: torch.Tensor, positions: torch.Tensor, prev_keys, prev_values, cos, sin):
         """``sparse_prefill_loop`` (flashloop/prefill.py:122-272): only the active rows are
         recomputed; their K/V replace the previous loop's rows of a composite cache."""
-        weights = self._prefill_weights(hidden)
+        weights = self._prefill_weights(hidden, cos, sin)
         if weights is None:
             return self._sparse_loop_modules(hidden, positions, prev_keys, prev_values, cos, sin)
         keys = [k.clone() for k in prev_keys]

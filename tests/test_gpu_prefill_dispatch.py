@@ -116,3 +116,31 @@ def test_misaligned_norm_weight(name):
     assert w.data_ptr() % 16 == 2
     model.get_submodule(name).weight = torch.nn.Parameter(w)
     _like_the_modules(model, "misaligned norm weight")
+
+
+def test_rotary_tables_of_another_layout():
+    """A rotary module whose tables are not contiguous."""
+    print("case: strided rotary tables", flush=True)
+    model = _model()
+    rot = model.model.rotary_emb
+    forward = rot.forward
+    rot.forward = lambda x, p: torch.stack(forward(x, p), dim=-1).unbind(-1)
+    _like_the_modules(model, "strided rotary tables")
+
+
+def test_embedding_rows_of_another_layout():
+    """An embedding module whose rows are two bytes off, or lie apart."""
+    print("case: embedding rows of another layout", flush=True)
+    for offset, gap in ((1, 0), (0, 8)):
+        model = _model()
+        emb = model.model.embed_tokens
+        forward = emb.forward
+
+        def apart(ids, forward=forward, offset=offset, gap=gap):
+            h = forward(ids)
+            room = h.new_zeros(offset + h.shape[0] * h.shape[1] * (h.shape[2] + gap))[offset:]
+            out = room.view(h.shape[0], h.shape[1], h.shape[2] + gap)[..., : h.shape[2]]
+            return out.copy_(h)
+
+        emb.forward = apart
+        _like_the_modules(model, f"embedding rows offset={offset} gap={gap}")
