@@ -315,8 +315,9 @@ class FlashLoopEngine:
         q, k, v = F.linear(z, wq), F.linear(z, wk), F.linear(z, wv)
         kernels.rope_store(q, k, v, rope, kv[0], kv[1], positions)
         heads = kv[0].shape[0]
+        # (the scale of SDPA, as in the module path: the decode's ``scaling`` attribute has no part in a prefill)
         o = kernels.prefill_attention(q.view(q.shape[0], heads, -1).transpose(0, 1), kv[0], kv[1],
-                                      self.layers[0].self_attn.scaling, positions)
+                                      kv[0].shape[-1] ** -0.5, positions)
         hid, z = kernels.norm_chain(hid, x=F.linear(o, wo), w_a=ln2, w_b=ln3, eps=eps)
         y = F.linear(kernels.swiglu(F.linear(z, gate), F.linear(z, up)), down)
         return kernels.norm_chain(hid, x=y, w_a=ln4, w_f=w_final, w_b=w_next, eps=eps)

@@ -144,3 +144,15 @@ def test_embedding_rows_of_another_layout():
 
         emb.forward = apart
         _like_the_modules(model, f"embedding rows offset={offset} gap={gap}")
+
+
+def test_prefill_attention_scale_is_that_of_the_modules():
+    """The modules' attention divides by sqrt(head_dim), whatever ``scaling`` says."""
+    print("case: scaling attribute", flush=True)
+    model = _model()
+    for layer in model.model.layers:
+        layer.self_attn.scaling *= 16.0
+    with torch.no_grad():
+        for layer in model.model.layers:  # scores that matter
+            layer.self_attn.q_proj.weight.mul_(10.0)
+    _like_the_modules(model, "scaling attribute")
