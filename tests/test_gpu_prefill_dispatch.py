@@ -156,3 +156,35 @@ def test_prefill_attention_scale_is_that_of_the_modules():
         for layer in model.model.layers:  # scores that matter
             layer.self_attn.q_proj.weight.mul_(10.0)
     _like_the_modules(model, "scaling attribute")
+
+
+def test_module_path_equals_the_kernels():
+    """Token-sparse loops over the same rows on both paths (a hook without effect keeps the
+    modules): K/V of every loop and layer, and the logits.  1000 keys: the kernels divide the
+    250 and 100 active rows' keys over several workgroups."""
+    print("case: module path and kernels", flush=True)
+    model = _model()
+    ids = torch.randint(0, TINY.vocab_size, (1, 1000), generator=torch.Generator().manual_seed(123)).cuda()
+    eng = FlashLoopEngine(model)
+    chosen, calls = [], []
+    select = eng._select
+
+    def keep(*args, **kw):
+        chosen.append(select(*args, **kw))
+        return chosen[-1]
+
+    with torch.inference_mode():
+        eng._select = keep
+        a = eng._prefill_loops(ids, all_logits=True)
+        model.model.layers[0].mlp.up_proj.register_forward_hook(lambda m, x, out: calls.append(1))
+        rows = iter(chosen)
+        eng._select = lambda *args, **kw: next(rows)
+        b = eng._prefill_loops(ids, all_logits=True)
+    assert len(calls) == 4 and [r.active_rows for r in a.receipts] == [1000, 1000, 250, 100]
+    assert torch.equal(a.mask3, b.mask3) and torch.equal(a.mask4, b.mask4)
+    # the bound of _like_the_modules
+    assert _rel(a.logits, b.logits) < 3e-2
+    for loop in range(4):
+        for li in range(TINY.num_hidden_layers):
+            for x, y in ((a.keys, b.keys), (a.values, b.values)):
+                assert _rel(x[loop][li], y[loop][li]) < 3e-2, f"loop {loop + 1} layer {li}"
