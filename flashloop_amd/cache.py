@@ -209,7 +209,8 @@ class CrossLoopKVLayer:
         With ``recon=True`` the reconstructed prefixes R_r are returned as
         ``layer.recon_keys/recon_values`` (bf16 ``[B*H, T, 128]``) for audits.
         ``late_counts``: what ``count_late_rows`` returned for these masks and lengths, for a
-        caller that packs several layers with the same masks (rows beyond a count are dropped).
+        caller that packs several layers with the same masks.  Rows beyond a count are dropped;
+        that the masks are nested is checked by ``count_late_rows`` then, not here.
         """
         if len(keys) != 4 or len(values) != 4:
             raise ValueError("exactly four loop K/V tensors are required")

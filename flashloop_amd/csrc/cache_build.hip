@@ -129,7 +129,7 @@ __global__ __launch_bounds__(kBuildThreads) void cache_prepare_kernel(PrepareArg
   const int tid = threadIdx.x;
   if (blk < 2 * a.seqs) {
     const int s = blk / a.seqs, i = blk % a.seqs, b = a.b0 + i;
-    const int n = a.len.packed[i], cap = v.token_capacity, rows = v.row_capacity[2 + s];
+    const int n = a.len.packed[i], cap = v.token_capacity, rows = a.len.late[s][i];  // (a rollover goes on from there)
     const uint8_t* m = a.mask[s] ? a.mask[s] + b * a.mask_stride : nullptr;
     int32_t* out = v.rank[s] + static_cast<int64_t>(b) * cap;
     int run = 0;

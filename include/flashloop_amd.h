@@ -141,7 +141,8 @@ int32_t fl_pack_kv_groups(const fl_cache_view* view, int32_t loops,
  * fl_cache_prepare: fills the parts of a newly allocated layer that fl_pack_kv_groups does not
  * write.  Host arrays: packed, tail [B], late [2, B] (rows kept by streams 2/3).  Writes the
  * device lengths packed_tokens, tail_tokens [B], late_rows [2, B], zeros dst_group0 [B], the
- * rank maps (running count of the active tokens of masks[s] below packed[b]; -1 elsewhere),
+ * rank maps (running count of the active tokens of masks[s] below packed[b]; -1 elsewhere and
+ * from the late[s, b]-th row on),
  * each loop's BF16 tail (source rows packed[b] .. + tail[b], then zeros) with its activity
  * tail_active[s] (u8 [B, tail_capacity]), and zeros in the capacity past the packed prefix
  * and past the kept rows.  Sources as for fl_pack_kv_groups.

@@ -142,3 +142,32 @@ def test_append_of_many_layers_equals_torch(layers, b, h):
         got = layer.state_dict()[0]
         assert got.keys() == w.keys()  # (bytes: the tails' unused rows may hold anything)
         assert [k for k in w if not torch.equal(got[k].contiguous().view(torch.uint8), w[k].contiguous().view(torch.uint8))] == [], i
+
+
+def test_late_rows_beyond_a_given_count_are_dropped():
+    """Counts below the masks': the surplus rows of loops 3/4 are left out (rank -1), so the rows
+    that a rollover adds never share a compact row with them; a count above them leaves rows free."""
+    print("case: late counts that differ from the masks", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(96)
+    b, h, t = 3, 2, 255  # tails of 127 rows
+    ks, vs = _kv(g, b, h, t), _kv(g, b, h, t)
+    m3 = torch.rand(b, t, generator=g, device=DEV) < 0.6
+    m4 = m3 & (torch.rand(b, t, generator=g, device=DEV) < 0.6)
+    true = CrossLoopKVLayer.count_late_rows(m3, m4)
+    given = [[max(0, n - d) for n, d in zip(true[s], (20 + s, 0, -5))] for s in range(2)]
+    layer = CrossLoopKVLayer.from_prefill(ks, vs, mask_loop3=m3, mask_loop4=m4, token_capacity=512, late_counts=given)
+    for s, m in enumerate((m3, m4)):
+        for i in range(b):
+            on = m[i, :128]
+            want = torch.where(on, on.int().cumsum(0) - 1, -1)
+            want = torch.where(want < given[s][i], want, -1).int()
+            assert torch.equal(layer.rank[s][i, :128], want), f"rank map {s} of sequence {i}"
+    assert layer.late_rows.tolist() == given == layer.late_rows_host
+    new = [[torch.randn(b, h, 1, 128, generator=g, device=DEV).to(torch.bfloat16) for _ in range(4)] for _ in range(2)]
+    layer.append_rows(*new)
+    layer.commit_append()
+    assert layer.packed_host == [192] * b
+    for s in range(2):
+        for i in range(b):
+            rows = layer.rank[s][i][layer.rank[s][i] >= 0].tolist()
+            assert len(set(rows)) == len(rows) and max(rows) < int(layer.late_rows[s, i]), f"rank map {s} of sequence {i}"
