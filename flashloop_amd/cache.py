@@ -242,6 +242,8 @@ class CrossLoopKVLayer:
         late_cap = () if late is None else tuple(max(max(c) + growth, 1) for c in late)
         fixed = cls._fixed_buffers(b, h, cap, late_cap, 2 * GROUP, dev, torch.empty)
         src_k, src_v = [x.contiguous() for x in keys], [x.contiguous() for x in values]
+        if not tp_max:  # the tails take any rows (fl_pack_kv_groups refuses misaligned ones)
+            src_k, src_v = ([x.clone() if x.data_ptr() % 16 else x for x in src] for src in (src_k, src_v))
         group0 = torch.empty(b, dtype=torch.int32, device=dev)
         if late is None:
             late = cls._finish_late_count(count, tp)

@@ -171,3 +171,17 @@ def test_late_rows_beyond_a_given_count_are_dropped():
         for i in range(b):
             rows = layer.rank[s][i][layer.rank[s][i] >= 0].tolist()
             assert len(set(rows)) == len(rows) and max(rows) < int(layer.late_rows[s, i]), f"rank map {s} of sequence {i}"
+
+
+@pytest.mark.parametrize("t", [1, 100])
+def test_short_prompts_of_misaligned_rows(t):
+    """Prompts without a packed group, from K/V that start two bytes into their storage."""
+    print(f"case: misaligned short prompt t={t}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(97)
+    shape = (2, 3, t, 128)
+    off = [torch.randn(2 * 3 * t * 128 + 1, generator=g, device=DEV).bfloat16()[1:].view(shape) for _ in range(8)]
+    assert all(x.data_ptr() % 16 == 2 for x in off)
+    layer = CrossLoopKVLayer.from_prefill(off[:4], off[4:])
+    for r in range(4):
+        assert torch.equal(layer.tail_key[r].view(2, 3, -1, 128)[:, :, :t], off[r])
+        assert torch.equal(layer.tail_value[r].view(2, 3, -1, 128)[:, :, :t], off[4 + r])
