@@ -89,7 +89,10 @@ int32_t launch_move(const void* src, int64_t s_outer, int64_t s_row, void* dst, 
 }
 
 // One wave per row.  WIDE: 16-byte loads, four chunks of each row in flight per lane (rows of a
-// multiple of 8 values, 16-byte aligned); 8192 rows of 2048: 17.4 us with 2-byte loads, 12.0.
+// multiple of 8 values, 16-byte aligned); 8192 rows of 2048: 17.4 us with 2-byte loads, 12.0.  From
+// 256 values on, a chunk for half of the lanes: 32768 / 8192 / 100 rows of 512 take 16.3 / 3.8 / 2.8 us
+// with 2-byte loads and 11.3 / 3.6 / 2.3 wide, of 256 9.2 / 3.3 / 2.4 and 8.6 / 3.5 / 2.3, of 128 6.5 / 3.1 /
+// 2.2 and 8.1 / 3.6 / 2.4.
 template <bool WIDE>
 __global__ __launch_bounds__(256) void hidden_delta_score_kernel(const uint16_t* cur, const uint16_t* prev,
                                                                  int64_t rows, int dim, float* score) {
@@ -178,7 +181,7 @@ extern "C" int32_t fl_hidden_delta_score(const uint16_t* cur, const uint16_t* pr
   if (rows == 0) return FL_OK;
   const dim3 grid(static_cast<unsigned>((rows + 3) / 4));
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (dim % 8 == 0 && reinterpret_cast<uintptr_t>(cur) % 16 == 0 && reinterpret_cast<uintptr_t>(prev) % 16 == 0)
+  if (dim % 8 == 0 && dim >= 4 * kWave && reinterpret_cast<uintptr_t>(cur) % 16 == 0 && reinterpret_cast<uintptr_t>(prev) % 16 == 0)
     hipLaunchKernelGGL(hidden_delta_score_kernel<true>, grid, dim3(256), 0, st, cur, prev, rows, dim, score);
   else
     hipLaunchKernelGGL(hidden_delta_score_kernel<false>, grid, dim3(256), 0, st, cur, prev, rows, dim, score);

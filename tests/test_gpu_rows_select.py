@@ -79,3 +79,14 @@ def test_hidden_score_widths(rows, dim):
     want = (a.double() - b.double()).norm(dim=-1) / a.double().norm(dim=-1)
     # two fp32 sums of dim positive terms (halved by the root), a division and two roots
     assert bool(((got - want).abs() <= (dim + 8) * 2.0 ** -24 * want).all())
+
+
+@pytest.mark.parametrize("dim", [1, 64, 248, 256, 264])
+def test_hidden_score_at_the_wide_loads_line(dim):
+    """Rows on both sides of 256 values, against the bound of test_hidden_score_widths."""
+    print(f"case: hidden score line dim={dim}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(99)
+    a, b = (torch.randn(9, dim, generator=g, device=DEV).bfloat16() for _ in range(2))
+    got = kernels.hidden_delta_score(a, b).double()
+    want = (a.double() - b.double()).norm(dim=-1) / a.double().norm(dim=-1)
+    assert bool(((got - want).abs() <= (dim + 8) * 2.0 ** -24 * want).all())
