@@ -1022,6 +1022,13 @@ __device__ __forceinline__ SplitRow split_row(const SplitArgs& a, int r) {
   return s;
 }
 
+// The slice of this workgroup.  Consecutive workgroups go to the 8 XCDs in turn, and to an XCD's CUs, so
+// with a multiple of 8 slices the live ones of short rows would meet on a few of them: there the row
+// turns the slices (64 rows of 20,000 keys, stride 131,072: 113 -> 70 us, of 131,072 keys 137 either way).
+__device__ __forceinline__ int split_slice(const SplitArgs& a) {
+  return static_cast<int>(a.slices % 8 ? blockIdx.x : (blockIdx.x + blockIdx.y) % static_cast<unsigned>(a.slices));
+}
+
 // This thread's four keys of the slice, -inf past n.
 __device__ __forceinline__ void slice_scores(const SplitRow& s, int base, float (&x)[4]) {
   if (base + 4 <= s.n && (reinterpret_cast<uintptr_t>(s.x) & 15u) == 0) {
@@ -1088,7 +1095,7 @@ __device__ __forceinline__ int split_bin(const SplitScale& c, uint32_t key) {
 __global__ __launch_bounds__(kTopkThreads) void split_extremes_kernel(SplitArgs a) {
   __shared__ uint4 red[kTopkWaves];
   const SplitRow s = split_row(a, blockIdx.y);
-  const int slice = blockIdx.x, tid = threadIdx.x, base = slice * kSliceKeys + 4 * tid;
+  const int slice = split_slice(a), tid = threadIdx.x, base = slice * kSliceKeys + 4 * tid;
   if (slice == 0) {
     s.hist[tid] = 0;
     if (tid == 0) s.ncand[0] = 0;
@@ -1169,7 +1176,7 @@ __global__ __launch_bounds__(kTopkThreads) void split_normaliser_kernel(SplitArg
 __global__ __launch_bounds__(kTopkThreads) void split_histogram_kernel(SplitArgs a) {
   __shared__ uint32_t hist[kBins];
   const SplitRow s = split_row(a, blockIdx.y);
-  const int slice = blockIdx.x, tid = threadIdx.x, base = slice * kSliceKeys + 4 * tid;
+  const int slice = split_slice(a), tid = threadIdx.x, base = slice * kSliceKeys + 4 * tid;
   if (slice * kSliceKeys >= s.n) return;
   hist[tid] = 0;
   float x[4];
@@ -1214,7 +1221,7 @@ __global__ __launch_bounds__(kTopkThreads) void split_candidates_kernel(SplitArg
   __shared__ uint32_t cnt[kTopkWaves], found[2], total, ncand, first;
   __shared__ uint32_t ck[kSplitCand], ci[kSplitCand];
   const SplitRow s = split_row(a, blockIdx.y);
-  const int slice = blockIdx.x, tid = threadIdx.x, base = slice * kSliceKeys + 4 * tid;
+  const int slice = split_slice(a), tid = threadIdx.x, base = slice * kSliceKeys + 4 * tid;
   if (slice * kSliceKeys >= s.n) return;
   float x[4];
   slice_scores(s, base, x);
@@ -1261,7 +1268,7 @@ __global__ __launch_bounds__(kTopkThreads) void split_compact_kernel(SplitArgs a
   __shared__ float red[kTopkWaves];
   const int r = blockIdx.y;
   const SplitRow s = split_row(a, r);
-  const int slice = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int slice = split_slice(a), tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int base = slice * kSliceKeys + 4 * tid;
   int32_t* oi = a.indices + static_cast<int64_t>(r) * a.cap;
   uint8_t* ov = a.valid + static_cast<int64_t>(r) * a.cap;
@@ -1386,7 +1393,7 @@ __global__ __launch_bounds__(kTopkThreads) void split_finish_kernel(SplitArgs a)
   __shared__ TopkShared sh;
   const int r = blockIdx.y;
   const SplitRow s = split_row(a, r);
-  const int slice = blockIdx.x, tid = threadIdx.x;
+  const int slice = split_slice(a), tid = threadIdx.x;
   if (s.n > 0 && s.ncand[0] > kSplitCand) {
     if (slice == 0)
       topk_global_row(sh, r, s.n, a.scores, a.stride, a.fraction, a.cap, a.indices, a.valid, a.mass, a.weights, a.counts,
@@ -1729,6 +1736,21 @@ extern "C" size_t fl_decode_topk_workspace(int32_t rows, int64_t scores_stride, 
   using namespace fl;
   if (rows <= 0 || scores_stride <= 0 || select_merge_fits(scores_stride, fraction)) return 0;
   return static_cast<size_t>(rows) * split_words(split_slices(scores_stride)) * sizeof(uint32_t);
+}
+
+// Times in us: a workgroup per row reads its keys seven times, from its XCD's L2 while the rows under
+// way there fit its 4 MiB; the split takes six launches, whose workgroups past the keys cost a third
+// of the others.  Measured (us, one / split): 1 row of 5000 keys 20 / 27, of 8000 28 / 27, of 70,000
+// 178 / 31; 16 rows of 70,000 189 / 42; 64 of 16,000 48 / 46, of 70,000 182 / 89; 128 of 28,000 78 / 88, of
+// 36,900 102 / 91, of 70,000 238 / 151; 256 of 70,000 250 / 272; 300 437 / 323; 512 493 / 523.
+extern "C" int32_t fl_decode_topk_long_pays(int32_t rows, int64_t scores_stride, int64_t keys, double fraction) {
+  using namespace fl;
+  if (rows <= 0 || rows > 65535 || scores_stride <= 0 || select_merge_fits(scores_stride, fraction)) return 0;
+  const double n = static_cast<double>(std::max<int64_t>(1, std::min(keys, scores_stride)));
+  const double slices = split_slices(scores_stride), live = std::ceil(n / kSliceKeys);
+  const bool in_l2 = std::min(rows, 256) * n * sizeof(float) / 8 <= 4.0 * (1 << 20);
+  const double one = 8.5 + (in_l2 ? 2.45e-3 : 3.4e-3) * n * ((rows + 255) / 256);
+  return 27.0 + rows * (0.041 * live + (rows <= 256 ? 0.013 : 0.019) * slices) < one;
 }
 
 extern "C" int32_t fl_decode_topk_long(const float* scores, int64_t scores_stride, int32_t rows, const int32_t* n_keys,

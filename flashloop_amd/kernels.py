@@ -249,9 +249,13 @@ def decode_topk(logits: torch.Tensor, n_keys: torch.Tensor, fraction: float, cap
         if more_keys.numel() != n_keys.numel():
             raise ValueError("more_keys needs the entries of n_keys")
     lib = load()
-    ws_bytes = lib.fl_decode_topk_workspace(rows, logits.stride(0), float(fraction))
-    if ws_bytes and rows <= 65535:  # a row over several workgroups
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    stride = logits.stride(0)
+    # the rows' length as the capacity tells it (to 64 / fraction keys; of the values that a captured step
+    # is made for, so that it and an eager step choose alike).  Either call takes rows of any length.
+    keys = int(min(stride, capacity / fraction)) if fraction > 0 else 0
+    if lib.fl_decode_topk_long_pays(rows, stride, keys, float(fraction)):
+        ws_bytes = lib.fl_decode_topk_workspace(rows, stride, float(fraction))
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)  # a row over several workgroups
         rc = lib.fl_decode_topk_long(logits.data_ptr(), logits.stride(0), rows, n_keys.data_ptr(), _p(more_keys),
                                      int(plus_keys), rows_per_count, float(fraction), capacity, idx.data_ptr(),
                                      valid.data_ptr(), mass.data_ptr(), w.data_ptr(), counts.data_ptr(), _p(nonfinite),

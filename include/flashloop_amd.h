@@ -271,9 +271,12 @@ int32_t fl_decode_topk(const float* scores, int64_t scores_stride, int32_t rows,
  * fl_decode_topk for rows (or selections) beyond the register-resident kernel: the same
  * selection, each row divided over several workgroups.  A row's key count is
  * n_keys[i] + more_keys[i] (nullable) + plus_keys, i = r / rows_per_count.  Workspace
- * (16-byte aligned): fl_decode_topk_workspace bytes, 0 where fl_decode_topk itself is the
- * faster call (logits rows of up to 36864 keys with up to 8192 selected).
+ * (16-byte aligned): fl_decode_topk_workspace bytes, 0 where fl_decode_topk holds a row in registers
+ * (logits rows of up to 36864 keys with up to 8192 selected).
+ * fl_decode_topk_long_pays: 1 where rows of about `keys` keys are selected faster by this call
+ * than by fl_decode_topk (few rows, long and well filled), else 0.
  */
+int32_t fl_decode_topk_long_pays(int32_t rows, int64_t scores_stride, int64_t keys, double fraction);
 size_t fl_decode_topk_workspace(int32_t rows, int64_t scores_stride, double fraction);
 int32_t fl_decode_topk_long(const float* scores, int64_t scores_stride, int32_t rows,
                             const int32_t* n_keys, const int32_t* more_keys, int32_t plus_keys,

@@ -91,3 +91,27 @@ def test_long_row_alone_equals_the_row_in_a_batch():
             assert (a - b).abs().max().item() <= 4e-6 * size, name
         # logits are sums of 128 products of sizes up to |q||k| / sqrt(128), about 40
         assert (one.logits1[0, ..., : t + 1] - many.logits1[i, ..., : t + 1]).abs().max().item() <= 128 * 2.0 ** -24 * 40
+
+
+@pytest.mark.parametrize("rows,stride,n,long", [(16, 70144, 2000, 0), (16, 70144, 70144, 1), (1, 36865, 6000, 0), (1, 36865, 20000, 1),
+                                                (192, 40960, 40960, 0), (9, 131072, 131000, 1), (9, 65536, 30000, 1),
+                                                (256, 36868, 36868, 0)])
+def test_route_by_rows_and_length(rows, stride, n, long):
+    """Short, ordinary and many rows of a wide logits buffer on the call that is faster for them;
+    either way what one workgroup per row selects (numbers of slices that are multiples of 8 among them)."""
+    print(f"case: top-k route rows={rows} stride={stride} n={n}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(98)
+    fraction = 0.1
+    x = _rows("tied", rows, stride, gen)
+    cap = kernels.decode_capacity(n, fraction)
+    lib = _lib.load()
+    assert lib.fl_decode_topk_long_pays(rows, stride, int(min(stride, cap / fraction)), fraction) == long
+    lengths = torch.randint(n // 2, n + 1, (rows,), generator=gen, device=DEV, dtype=torch.int32)
+    lengths[0] = n
+    idx, valid, mass, w, counts = kernels.decode_topk(x, lengths, fraction, cap)
+    want = [torch.empty_like(t) for t in (idx, valid, mass, w, counts)]
+    _lib.check(lib.fl_decode_topk(x.data_ptr(), stride, rows, lengths.data_ptr(), 1, fraction, cap, *(t.data_ptr() for t in want),
+                                  None, torch.cuda.current_stream().cuda_stream), "fl_decode_topk")
+    assert torch.equal(idx, want[0]) and torch.equal(valid, want[1]) and torch.equal(counts, want[4])
+    for got, ref in ((mass, want[2]), (w, want[3])):  # the masses sum in another order (see above)
+        assert bool(((got - ref).abs() <= 2 * cap * 2.0 ** -24 * ref.abs()).all())
