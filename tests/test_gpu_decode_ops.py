@@ -260,3 +260,14 @@ def test_decode_inputs(b, d, hd, freq):
     for got, want in ((cos, angle.cos()), (sin, angle.sin())):
         want = torch.cat([want, want], -1)
         assert ((got[:, 0].double().cpu() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -21).all()
+
+
+@pytest.mark.parametrize("m", [1, 2, 3, 4, 5, 8])
+def test_gemv_of_long_rows(m):
+    """K past the matrix-core form: each number of rows on the instantiation that holds it."""
+    print(f"case: gemv long rows m={m}", flush=True)
+    n, k = 12, 10248
+    x, x32, add, w = _x(m, k, 120), _x(m, k, 121, torch.float32), _x(m, n, 122), _w(n, k, 123)
+    _near(kernels.gemv(x, [w]), *_dots(x, w), "plain")
+    d, s = _dots(x32.bfloat16(), w)
+    _near(kernels.gemv(x32, [w], epilogue=kernels.EPI_ADD, addend=add), d + add.double(), s + 2.0 ** -8 * d.abs(), "add")
