@@ -12,8 +12,9 @@
 // Every rounding to bf16 happens where the torch modules round (Linear output, RMSNorm
 // output, each binary op of rotate-half RoPE, SiLU, the SwiGLU product, residual adds).
 //
-// The GEMVs are memory-bound (bytes = N * K * 2 + M * K * 2); gemv_mfma_kernel runs every K up
-// to 8192, gemv_kernel (VALU dots, one workgroup per 4 rows) the longer ones.
+// The GEMVs are memory-bound (bytes = N * K * 2 + M * K * 2); gemv_mfma_kernel runs K up to 8192
+// (one and two rows: 4096), gemv_flat_kernel (VALU dots, one workgroup per 4 rows) one and two
+// rows up to 8192, gemv_kernel (the same in a loop) the longer ones.
 #include "fl_common.h"
 
 namespace fl {
@@ -252,6 +253,68 @@ __global__ __launch_bounds__(kGemvThreads) void gemv_kernel(GemvArgs a) {
   gemv_finish<MT, EPI>(a, acc, red, mat, n0);
 }
 
+// The GEMV with every chunk a thread owns (S of them per row, K <= S * 2048) requested
+// at once as bounds-checked buffer loads: chunks past K and rows past M read as zero, so
+// no load sits under a branch (the compiler's wait after a branch join drains every
+// outstanding load).  Same accumulation order as gemv_kernel.
+template <int MT, int EPI, bool XF32, int S>
+__global__ __launch_bounds__(kGemvThreads) void gemv_flat_kernel(GemvArgs a) {
+  __shared__ float red[kGemvWaves][MT][kRows];
+  const uint16_t* rp[kRows];
+  int mat, n0;
+  block_rows<EPI>(a, blockIdx.x, rp, &mat, &n0);
+  constexpr int kStep = kGemvThreads;
+  constexpr uint32_t kXb = XF32 ? 4u : 2u;  // bytes per x element
+  const uint32_t q = threadIdx.x;
+  uint4 wv[S][kRows];
+#pragma unroll
+  for (int r = 0; r < kRows; ++r) {
+    const BufRes wr = buf_res(rp[r], static_cast<uint32_t>(a.K) * 2u);
+#pragma unroll
+    for (int s = 0; s < S; ++s) wv[s][r] = buf_load16(wr, 16u * (q + s * kStep));
+  }
+  uint4 xv[MT][S][XF32 ? 2 : 1];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const bool live = m < a.M;
+    const BufRes xr = buf_res(live ? static_cast<const char*>(a.x) + static_cast<int64_t>(m) * a.x_stride * kXb : nullptr,
+                              live ? static_cast<uint32_t>(a.K) * kXb : 0u);
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const uint32_t off = 8u * kXb * (q + s * kStep);
+      xv[m][s][0] = buf_load16(xr, off);
+      if (XF32) xv[m][s][XF32 ? 1 : 0] = buf_load16(xr, off + 16u);
+    }
+  }
+  float acc[MT][kRows];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) acc[m][r] = 0.0f;
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      float x[8];
+      if (XF32) {
+        const uint4 u = xv[m][s][0], v = xv[m][s][XF32 ? 1 : 0];
+        const uint32_t w8[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = bf16_round(__uint_as_float(w8[e]));
+      } else {
+        unpack8(xv[m][s][0], x);
+      }
+#pragma unroll
+      for (int r = 0; r < kRows; ++r) {
+        float f[8];
+        unpack8(wv[s][r], f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[m][r] = fmaf(x[e], f[e], acc[m][r]);
+      }
+    }
+  gemv_finish<MT, EPI>(a, acc, red, mat, n0);
+}
+
 // ---------------------------------------------------------------------------------
 // Residual / RMSNorm chain of one row (one workgroup per row).  Thread t owns the
 // 8-value chunks t, t + 256, ... of the row; every global load (x, r and the three
@@ -425,8 +488,8 @@ __global__ __launch_bounds__(kNormThreads) void norm_chain_kernel(NormArgs a) {
 // row takes 4 waves and 4-row tiles (twice the workgroups).  Measured, 2048 wide (q/k/v with
 // RoPE, o_proj, SwiGLU 5632, down, lm_head 49152), us before -> now: 8 rows 46.8 -> 10.0,
 // 12.1 -> 5.4, 75.2 -> 12.9, 15.6 -> 7.9, 287 -> 40 (5.0 TB/s); one row 9.2 -> 7.7, 4.8 -> 4.9,
-// 13.3 -> 10.8, 6.1 -> 6.9, 42.0 -> 36.5 (5.5 TB/s).  One row with 8 waves and 8-row tiles
-// took 9.1, 5.1, 11.9, 6.9 and 38.4.
+// 13.3 -> 10.8, down stays on the VALU form (6.1, 6.9 here), 42.0 -> 36.5 (5.5 TB/s).  One row with
+// 8 waves and 8-row tiles took 9.1, 5.1, 11.9, 6.9 and 38.4.
 template <int MT>
 struct MmGeom {
   static constexpr int kWaves = MT == 1 ? 4 : 8;
@@ -746,7 +809,7 @@ __global__ __launch_bounds__(MmGeom<MT>::kThreads, 2) void gemv_mfma_kernel(Gemv
     unit_rows<EPI, MT, NT>(a, unit, ur);
     load_unit<MT, NT, CS>(ur, K, w[d]);
     // the weights are all requested here (left to itself the compiler loads each before its product
-    // once no loop follows: down 6.9 -> 7.4 us), and ahead of load_epi's index arithmetic
+    // once no loop follows: K 5632 6.9 -> 7.4 us), and ahead of load_epi's index arithmetic
     __builtin_amdgcn_sched_barrier(0);
     if (kAhead && wave == 0) load_epi<EPI, MT, NT>(a, unit, e[d]);  // (the threads that store lie in one wave)
   };
@@ -941,25 +1004,57 @@ void launch_gemv_mfma(const GemvArgs& a, const NormArgs& c, int workgroups, hipS
   hipLaunchKernelGGL((gemv_mfma_kernel<EPI, MT, KCAP, NT, CHAIN, DEPTH>), dim3(grid), dim3(MmGeom<MT>::kThreads), 0, st, a, c, units);
 }
 
+// The forms give a row the same products in the same order, so a chained call and its GEMV apart
+// may take different ones.  Each reads K in steps of 512 up to its KCAP, so one is there for every
+// 1024 or 2048 of K: one row without a chain, K 1024, lm_head 49152 and SwiGLU 5632 22.1 and 7.3 us
+// on the 2048 form, 18.1 and 6.5 on their own; K 3072 56.2 and 15.8 on the 4096 form, 46.5 and 14.1.
+//
 // Several units per workgroup (DEPTH 2) where the prologue or the epilogue of one unit would not
 // hide behind the other workgroups of its CU.  Eight chained rows: the prologue is ~700 VALU
 // instructions per row, so one workgroup per CU runs it once (SwiGLU 5632 x 2048: 16.8 us with
 // a workgroup per unit, 12.9 with 235 of three units; three units in flight gain nothing there
-// and q/k/v with RoPE, two units each, loses 9.9 -> 10.6).  One row: only the many units of a
-// head-sized matrix gain (lm_head 49152 x 2048: 37.5 -> 36.3 us; SwiGLU lost, 10.8 -> 13.1).
+// and q/k/v with RoPE, two units each, loses 9.9 -> 10.6).  One chained row: only the many units of
+// a head-sized matrix gain (lm_head 49152 x 2048: 37.5 -> 36.3 us, x 3072 67.8 -> 54.2, x 4096 79.4
+// -> 69.9; SwiGLU lost, 10.8 -> 13.1).  Without a chain one or two rows lose by it (lm_head 49152 x
+// 2048 31.3 -> 35.7 and 33.9 -> 36.5 us), three rows and more gain (eight 47.5 -> 38.5).
+//
+// Two tiles a unit where the workgroups are many: a short K of a head-sized matrix (eight rows,
+// lm_head 49152 x 1024 24.9 -> 21.5 us), and f32 rows, whose x loads cost as much as a tile's
+// weights (4096 x 4096 with an addend, one row 9.7 -> 8.6, eight 13.9 -> 11.3; not below one
+// workgroup a CU: two rows, 2048 x 4096 6.1 -> 7.2).
 template <int EPI, int MT, bool CHAIN>
 void launch_gemv_k(const GemvArgs& a, const NormArgs& c, hipStream_t st) {
   constexpr int kPair = EPI == kEpiSwiGlu || EPI == kEpiRope ? 2 : 1;
-  if (a.K <= 2048) {
-    if constexpr (CHAIN && MT == 8) {
-      return launch_gemv_mfma<EPI, MT, 2048, 2, CHAIN, 2>(a, c, 256, st);
+  const bool head = kPair == 1 && a.N >= 16384;
+  if constexpr (CHAIN) {
+    if (a.K <= 2048) {
+      if constexpr (MT == 8) {
+        launch_gemv_mfma<EPI, MT, 2048, 2, true, 2>(a, c, 256, st);
+      } else {
+        if (a.N >= 16384) return launch_gemv_mfma<EPI, MT, 2048, 2, true, 2>(a, c, 1024, st);
+        launch_gemv_mfma<EPI, MT, 2048, kPair, true, 1>(a, c, 0, st);
+      }
     } else {
-      if (a.N >= 16384) return launch_gemv_mfma<EPI, MT, 2048, 2, CHAIN, 2>(a, c, 1024, st);
-      launch_gemv_mfma<EPI, MT, 2048, kPair, CHAIN, 1>(a, c, 0, st);
+      if constexpr (MT == 1 && kPair == 1)
+        if (head) return launch_gemv_mfma<EPI, MT, 4096, 1, true, 2>(a, c, 1024, st);
+      launch_gemv_mfma<EPI, MT, 4096, kPair, true, 1>(a, c, 0, st);
     }
+  } else if (a.K <= 1024) {
+    if constexpr (kPair == 1)
+      if (head) return launch_gemv_mfma<EPI, MT, 1024, 2, false, 1>(a, c, 0, st);
+    launch_gemv_mfma<EPI, MT, 1024, kPair, false, 1>(a, c, 0, st);
+  } else if (a.K <= 2048) {
+    if constexpr (MT == 8)
+      if (a.N >= 16384 && (kPair == 2 || a.M > 2)) return launch_gemv_mfma<EPI, MT, 2048, 2, false, 2>(a, c, 1024, st);
+    launch_gemv_mfma<EPI, MT, 2048, kPair, false, 1>(a, c, 0, st);
+  } else if (a.K <= 3072) {
+    launch_gemv_mfma<EPI, MT, 3072, kPair, false, 1>(a, c, 0, st);
   } else if (a.K <= 4096) {
-    launch_gemv_mfma<EPI, MT, 4096, kPair, CHAIN, 1>(a, c, 0, st);
-  } else if constexpr (!CHAIN) {
+    if constexpr (kPair == 1)
+      if (a.x_f32 && a.N >= 256 * 2 * MmGeom<MT>::kTile)
+        return launch_gemv_mfma<EPI, MT, 4096, 2, false, 1>(a, c, 0, st);
+    launch_gemv_mfma<EPI, MT, 4096, kPair, false, 1>(a, c, 0, st);
+  } else if constexpr (MT > 1) {
     if (a.K <= 6144)
       launch_gemv_mfma<EPI, MT, 6144, kPair, false, 1>(a, c, 0, st);
     else
@@ -967,10 +1062,15 @@ void launch_gemv_k(const GemvArgs& a, const NormArgs& c, hipStream_t st) {
   }
 }
 
+// Workgroups of the kernels of one workgroup per kRows rows.
+template <int EPI>
+int gemv_blocks(int n) {
+  return EPI == kEpiSwiGlu ? n / 2 : (EPI == kEpiRope ? 3 * (n / kRows) : n / kRows);
+}
+
 template <int EPI, bool XF32>
 void launch_gemv_long(const GemvArgs& a, hipStream_t st) {
-  const int blocks = EPI == kEpiSwiGlu ? a.N / 2 : (EPI == kEpiRope ? 3 * (a.N / kRows) : a.N / kRows);
-  const dim3 g(blocks), t(kGemvThreads);
+  const dim3 g(gemv_blocks<EPI>(a.N)), t(kGemvThreads);
   // (no more rows of accumulators than the call has: two rows, K 10240 to 2048, on the eight-row form
   // 12.4 -> 14.4 us, four rows 15.7 -> 17.0)
   if (a.M <= 1)
@@ -983,10 +1083,32 @@ void launch_gemv_long(const GemvArgs& a, hipStream_t st) {
     hipLaunchKernelGGL((gemv_kernel<8, EPI, XF32>), g, t, 0, st, a);
 }
 
-// K up to 8192 (a unit's weights in registers) runs on the matrix cores; longer rows, and
-// heads or x strides so wide that a unit's rows do not fit one buffer, on gemv_kernel.
+// One and two rows of K 4104 to 8192: the matrix cores' 16 k-slices of partial sums and x loads per
+// unit cost more than the rows' own VALU dots.  To 2048, us with them and without: one row K 5632
+// 6.9 -> 6.1, 8192 9.0 -> 8.0, two rows 7.1 -> 6.8 and 9.3 -> 8.6, SwiGLU 5632 x 8192 34.4 -> 31.3
+// and 37.5 -> 31.4; from three rows on they lose (K 5632 8.8 against 7.3).  Up to 4096 one and two
+// rows stay on the matrix cores too, with the bits of the chained call: q/k/v with RoPE and SwiGLU
+// of 2048 are 7.2 and 10.2 us there against 7.0 and 9.8 (the chained call 7.4 and 10.9 against 8.7
+// and 13.1).
+template <int MT, int EPI, bool XF32>
+void launch_gemv_flat(const GemvArgs& a, hipStream_t st) {
+  const dim3 g(gemv_blocks<EPI>(a.N)), t(kGemvThreads);
+  if (a.K <= 6144)
+    hipLaunchKernelGGL((gemv_flat_kernel<MT, EPI, XF32, 3>), g, t, 0, st, a);
+  else
+    hipLaunchKernelGGL((gemv_flat_kernel<MT, EPI, XF32, 4>), g, t, 0, st, a);
+}
+
+// K up to 8192 (a unit's weights in registers) runs on the matrix cores, one and two rows up to
+// 4096, further on gemv_flat_kernel; longer rows, and heads or x strides so wide that a unit's rows
+// do not fit one buffer, on gemv_kernel.
 template <int EPI, bool CHAIN>
 void launch_gemv(const GemvArgs& a, const NormArgs& c, hipStream_t st) {
+  if constexpr (!CHAIN)
+    if (a.M <= 2 && a.K > kChainMaxK && a.K <= kMmMaxK) {
+      if (a.M == 1) return a.x_f32 ? launch_gemv_flat<1, EPI, true>(a, st) : launch_gemv_flat<1, EPI, false>(a, st);
+      return a.x_f32 ? launch_gemv_flat<2, EPI, true>(a, st) : launch_gemv_flat<2, EPI, false>(a, st);
+    }
   const bool wide = (EPI == kEpiRope && (static_cast<int64_t>(a.head_dim) + 16) * a.K * 2 > 0x7FFFFFFF) ||
                     (a.M > 1 && a.x_stride > 0x7FFFFFFF / (4 * kMaxM));
   if (CHAIN || (a.K <= kMmMaxK && !wide)) {

@@ -271,3 +271,25 @@ def test_gemv_of_long_rows(m):
     _near(kernels.gemv(x, [w]), *_dots(x, w), "plain")
     d, s = _dots(x32.bfloat16(), w)
     _near(kernels.gemv(x32, [w], epilogue=kernels.EPI_ADD, addend=add), d + add.double(), s + 2.0 ** -8 * d.abs(), "add")
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 4, 4104), (2, 12, 6144), (2, 516, 6152), (1, 20, 8192),
+                                   (1, 16388, 1024), (2, 16388, 1016), (8, 516, 1024), (2, 16388, 2040), (3, 16388, 1032),
+                                   (1, 516, 3072), (5, 516, 2056), (1, 2052, 4096), (1, 2044, 4096), (8, 4104, 4096)])
+def test_gemv_forms(m, n, k):
+    """Both sides of each line between the forms: one and two rows past K 4096, the steps of K, the
+    head-sized N and the f32 rows of two tiles a unit."""
+    test_gemv_at_tile_and_step_edges(m, n, k)
+
+
+@pytest.mark.parametrize("m", [1, 2, 8])
+@pytest.mark.parametrize("k", [1016, 2048, 3072, 4096])
+def test_gemv_chain_of_a_head(m, k):
+    """A head-sized matrix, where a chained call and the GEMV apart take different forms: equal."""
+    print(f"case: gemv chain head m={m} k={k}", flush=True)
+    n = 16388
+    r, x, wn, w = _x(m, k, 130), _x(m, k, 131), [_x(1, k, 132 + i)[0] for i in range(2)], _w(n, k, 134)
+    h0, z0 = kernels.norm_chain(r, eps=1e-6, x=x, w_a=wn[0], w_b=wn[1])
+    h1, got = kernels.gemv_chain(r, [w], eps=1e-6, epilogue=kernels.EPI_F32, x=x, w_a=wn[0], w_b=wn[1])
+    assert torch.equal(h1, h0) and torch.equal(got, kernels.gemv(z0, [w], epilogue=kernels.EPI_F32))
+    _near(got, *_dots(z0, w), "head", ulps=2.0)  # both sides are rounded: half an ulp, 2^-8 at most, each
