@@ -20,6 +20,7 @@
 // 16 heads, 8192 dense queries: 340-355 us, 775-810 TFLOP/s of the causal half (the SDPA it
 // replaces: 740 us); 2048 of 8192: 490 -> 116 us; 820 of 8192: 940 -> 65 us.
 #include <algorithm>
+#include <cfloat>
 
 #include "fl_common.h"
 
@@ -54,7 +55,7 @@ struct AttnArgs {
   float scale;  // scaling * log2(e)
   int splits;   // key ranges per query block
   float* part_o;   // splits > 1: f32 [splits][n * heads][128], row i * heads + h
-  float* part_ml;  // f32 [splits][n * heads][2]: maximum (base 2) and sum
+  float* part_ml;  // f32 [splits][n * heads][2]: maximum of q.k and sum
 };
 
 __device__ __forceinline__ uint32_t attn_bf16_pair(float lo, float hi) {
@@ -76,6 +77,17 @@ struct AttnLds {
   uint16_t k[2][kKeys * kKRow];
   uint16_t v[2][kKeys * kVRow];
 };
+
+// Base-2 logits past kFar: their products with the scale are no longer exact to a small part of 1, so
+// that exp2(fma(s, scale, -m)) would be off by a power of two, or overflow.  There the differences
+// are taken before the scale.  kNone: the maximum of a query that has seen no key.
+constexpr float kFar = 4096.0f;
+constexpr float kNone = -FLT_MAX;
+__device__ __forceinline__ float scaled_max(float r, float scale) { return fmaxf(r * scale, -FLT_MAX); }
+// 2^(scale (a - b)) of two raw maxima, a <= b; sa, sb: their scaled_max
+__device__ __forceinline__ float exp2_between(float a, float b, float sa, float sb, float scale) {
+  return fast_exp2(fabsf(sa) > kFar || fabsf(sb) > kFar ? (a - b) * scale : sa - sb);
+}
 
 // 4 keys (rows of the tile) of one d per lane: lane i of each 16-lane group passes the
 // address of V[key + i / 4][d + 4 (i % 4)] and receives V[key .. key + 3][d + i].
@@ -157,7 +169,9 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attention_kernel(AttnArgs a) 
   for (int d = 0; d < 4; ++d)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[d][r] = 0.0f;
-  float m = -1e30f, l = 0.0f;  // running maximum (scaled logits, base 2) and this lane's part of the sum
+  // running maximum (of q.k, and scaled to base 2) and this lane's part of the sum
+  float raw = kNone, m = scaled_max(kNone, a.scale), l = 0.0f;
+  bool far = false;  // (wave-uniform) some query's maximum lies past kFar
 
   for (int tile = first; tile < tiles; ++tile) {
     const int buf = (tile - first) & 1;
@@ -186,16 +200,26 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attention_kernel(AttnArgs a) 
       for (int b = 0; b < 2; ++b)
 #pragma unroll
         for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[b][r]);
-      mx = fmaxf(mx, swap_half(mx)) * a.scale;
-      if (__builtin_amdgcn_ballot_w64(mx > m) != 0ull) {
-        const float mn = fmaxf(m, mx);
-        const float alpha = fast_exp2(m - mn);
+      mx = fmaxf(mx, swap_half(mx));
+      if (__builtin_amdgcn_ballot_w64(mx > raw) != 0ull) {
+        const float top = fmaxf(raw, mx), mn = scaled_max(top, a.scale);
+        const float alpha = exp2_between(raw, top, m, mn, a.scale);
+        raw = top;
         m = mn;
         l *= alpha;
+        far = __builtin_amdgcn_ballot_w64(fabsf(m) > kFar && raw > kNone) != 0ull;
 #pragma unroll
         for (int d = 0; d < 4; ++d)
 #pragma unroll
           for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
+      }
+      float off = -m;
+      if (far) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) s[b][r] -= raw;
+        off = 0.0f;
       }
       float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
       bf16x8_t p[4];
@@ -205,8 +229,8 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attention_kernel(AttnArgs a) 
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int r = 8 * (t & 1) + 2 * i;
-          const float p0 = fast_exp2(fmaf(s[t >> 1][r], a.scale, -m));
-          const float p1 = fast_exp2(fmaf(s[t >> 1][r + 1], a.scale, -m));
+          const float p0 = fast_exp2(fmaf(s[t >> 1][r], a.scale, off));
+          const float p1 = fast_exp2(fmaf(s[t >> 1][r + 1], a.scale, off));
           w[i] = attn_bf16_pair(p0, p1);
           sum[i] = add_pair(w[i], sum[i]);
         }
@@ -240,7 +264,7 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attention_kernel(AttnArgs a) 
         for (int g = 0; g < 4; ++g)
           *reinterpret_cast<float4*>(op + 32 * d + 8 * g) =
               make_float4(o[d][4 * g], o[d][4 * g + 1], o[d][4 * g + 2], o[d][4 * g + 3]);
-      if (h == 0) *reinterpret_cast<float2*>(a.part_ml + 2 * row) = make_float2(m, l);
+      if (h == 0) *reinterpret_cast<float2*>(a.part_ml + 2 * row) = make_float2(raw, l);
     }
     return;
   }
@@ -265,14 +289,15 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(AttnArgs a) {
   const int64_t row = static_cast<int64_t>(blockIdx.x) * 8 + (threadIdx.x >> 5);
   if (row >= rows) return;
   const int c = (threadIdx.x & 31) * 4;
-  float M = -1e30f;
+  float M = kNone;
   for (int s = 0; s < a.splits; ++s) M = fmaxf(M, a.part_ml[2 * (s * rows + row)]);
+  const float sm = scaled_max(M, a.scale);
   float l = 0.0f;
   float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   for (int s = 0; s < a.splits; ++s) {
     const float2 ml = *reinterpret_cast<const float2*>(a.part_ml + 2 * (s * rows + row));
     const float4 p = *reinterpret_cast<const float4*>(a.part_o + (s * rows + row) * kDim + c);
-    const float w = fast_exp2(ml.x - M);
+    const float w = exp2_between(ml.x, M, scaled_max(ml.x, a.scale), sm, a.scale);
     l = fmaf(w, ml.y, l);
     o.x = fmaf(w, p.x, o.x);
     o.y = fmaf(w, p.y, o.y);

@@ -41,6 +41,38 @@ def test_prefill_attention(h, n, t):
         assert bool((err <= 0).all()), f"{err.max().item():.3e} beyond the bound"
 
 
+def _want(q, k, v, at):
+    """Attention of queries [H, n, 128] at positions ``at`` in float64, and the same of |v|."""
+    s = torch.bmm(q.double(), k.double().transpose(1, 2).contiguous()) * 128 ** -0.5
+    w = s.masked_fill(torch.arange(k.shape[1], device=DEV)[None, None] > at[None, :, None], -torch.inf).softmax(-1)
+    rows = lambda x: torch.bmm(w, x).transpose(0, 1).reshape(q.shape[1], -1)
+    return rows(v.double()), rows(v.double().abs())
+
+
+def _within(got, want, size, what):
+    """The bound of test_prefill_attention."""
+    err = (got.double() - want).abs() - (2.0 ** -8 * size + 2.0 ** -8 * want.abs() + 1e-6)
+    assert bool((err <= 0).all()), f"{what}: {err.max().item():.3e} beyond the bound"
+
+
+@pytest.mark.parametrize("n,t", [(150, 150), (40, 1000)])
+def test_prefill_attention_of_large_scores(n, t):
+    """Scores whose base-2 image is past the last fraction of an fp32 value, of both signs: equal
+    ones, and ones that differ from key to key."""
+    g = torch.Generator(device=DEV).manual_seed(84)
+    v = _r(g, 2, t, 128)
+    pos = None if n == t else torch.randperm(t, generator=g, device=DEV)[:n].sort().values.int()
+    at = torch.arange(n, device=DEV) if pos is None else pos.long()
+    for size in (3e2, 3e3, 3e4, 1e7, 1e10, 1e20, 1e31, 1e34):
+        for sign in (1.0, -1.0):
+            for spread in (0.0, 0.3):
+                print(f"case: prefill attention scores n={n} t={t} {sign * size:.0e} {spread}", flush=True)
+                a = (size / 128 ** 0.5) ** 0.5
+                q = torch.full((2, n, 128), a, device=DEV).bfloat16()
+                k = (sign * a * (1.0 + spread * torch.rand(2, t, 1, generator=g, device=DEV))).expand(2, t, 128).bfloat16()
+                _within(kernels.prefill_attention(q, k, v, 128 ** -0.5, pos), *_want(q, k, v, at), f"{sign * size:.0e}")
+
+
 @pytest.mark.parametrize("ranges", [0, 1, 2, 5])
 def test_prefill_attention_with_less_workspace(ranges):
     """A workspace of fewer key ranges than asked for (or none) divides the keys less."""
