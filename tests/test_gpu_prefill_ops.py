@@ -73,6 +73,61 @@ def test_prefill_attention_of_large_scores(n, t):
                 _within(kernels.prefill_attention(q, k, v, 128 ** -0.5, pos), *_want(q, k, v, at), f"{sign * size:.0e}")
 
 
+@pytest.mark.parametrize("n,t", [(70, 70), (40, 1000)])
+def test_prefill_attention_of_strided_rows(n, t):
+    """K and V in any head and row stride: token-major rows, and rows 136 apart."""
+    print(f"case: prefill attention strides n={n} t={t}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(85)
+    pos = None if n == t else torch.randperm(t, generator=g, device=DEV)[:n].sort().values.int()
+    at = torch.arange(n, device=DEV) if pos is None else pos.long()
+    q, k, v = _r(g, 3, n, 136)[..., :128], _r(g, t, 3, 128).transpose(0, 1), _r(g, 3, t, 136)[..., :128]
+    _within(kernels.prefill_attention(q, k, v, 128 ** -0.5, pos), *_want(q, k, v, at), "strides")
+
+
+@pytest.mark.parametrize("n,t", [(200, 200), (40, 1000)])
+def test_prefill_attention_of_non_finite_rows(n, t):
+    """A NaN in a K row reaches the queries that see it and no other; scores of -inf weigh nothing;
+    a query whose scores are all -inf, or NaN, gives NaN alone."""
+    print(f"case: prefill attention non-finite n={n} t={t}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(86)
+    pos = None if n == t else torch.randperm(t, generator=g, device=DEV)[:n].sort().values.int()
+    at = torch.arange(n, device=DEV) if pos is None else pos.long()
+    q, k, v = _r(g, 2, n, 128).abs(), _r(g, 2, t, 128), _r(g, 2, t, 128)
+    scale, hole = 128 ** -0.5, t // 2 + 1
+    bad = k.clone()
+    bad[0, hole, 5] = torch.nan
+    got = kernels.prefill_attention(q, bad, v, scale, pos).view(n, 2, 128)
+    sees = at >= hole
+    assert sees.any() and not sees.all()
+    assert got[sees, 0].isnan().all() and not got[~sees].isnan().any() and not got[:, 1].isnan().any()
+    want, size = (x.view(n, 2, 128) for x in _want(q, k, v, at))
+    _within(got[~sees], want[~sees], size[~sees], "before a NaN")
+    _within(got[:, 1], want[:, 1], size[:, 1], "another head")
+    low = k.clone()
+    low[:, 1::3] = -torch.inf
+    _within(kernels.prefill_attention(q, low, v, scale, pos), *_want(q, low, v, at), "-inf")
+    odd = q.clone()
+    odd[0, 3], odd[1, n - 1, 0] = -torch.inf, torch.nan
+    got = kernels.prefill_attention(odd, k.abs(), v, scale, pos).view(n, 2, 128)
+    want, size = (x.view(n, 2, 128) for x in _want(odd, k.abs(), v, at))
+    assert got[3, 0].isnan().all() and got[n - 1, 1].isnan().all() and int(got.isnan().sum()) == 2 * 128
+    ok = ~got.isnan()
+    _within(got[ok], want[ok], size[ok], "other queries")
+
+
+@pytest.mark.parametrize("h,n,t", [(2, 8200, 8200), (1, 3300, 33000)])
+def test_prefill_attention_of_long_prompts(h, n, t):
+    """Many query blocks and key tiles; 64 of the queries against float64."""
+    print(f"case: prefill attention long h={h} n={n} t={t}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(87)
+    q, k, v = _r(g, n, h, 128).transpose(0, 1), _r(g, h, t, 128), _r(g, h, t, 128)
+    pos = None if n == t else torch.randperm(t, generator=g, device=DEV)[:n].sort().values.int()
+    at = torch.arange(n, device=DEV) if pos is None else pos.long()
+    some = torch.cat((torch.randperm(n, generator=g, device=DEV)[:62], torch.tensor([0, n - 1], device=DEV)))
+    got = kernels.prefill_attention(q, k, v, 128 ** -0.5, pos)
+    _within(got[some], *_want(q[:, some], k, v, at[some]), "long")
+
+
 @pytest.mark.parametrize("ranges", [0, 1, 2, 5])
 def test_prefill_attention_with_less_workspace(ranges):
     """A workspace of fewer key ranges than asked for (or none) divides the keys less."""
@@ -84,8 +139,8 @@ def test_prefill_attention_with_less_workspace(ranges):
     lib = _lib.load()
     one = n * h * 130 * 4
     assert lib.fl_prefill_attention_workspace(h, n, t) >= 6 * one
-    ws = torch.empty(max(1, ranges * one), dtype=torch.uint8, device=DEV)
-    guard = torch.full((64,), 7, dtype=torch.uint8, device=DEV)
+    room = torch.full((ranges * one + 64,), 7, dtype=torch.uint8, device=DEV)
+    ws, guard = room, room[ranges * one:]
     out = torch.empty(n, h * 128, dtype=torch.bfloat16, device=DEV)
     _lib.check(lib.fl_prefill_attention(
         q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0), k.stride(1), v.data_ptr(), v.stride(0),
