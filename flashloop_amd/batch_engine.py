@@ -151,7 +151,8 @@ class FlashLoopBatchEngine:
     @torch.inference_mode()
     def decode(self, token_ids: torch.Tensor) -> BatchDecodeOutput:
         """One step for every sequence: ``token_ids`` ``[B, 1]``.  With graphs on, the
-        returned logits live in the graph's output buffer until the next step."""
+        returned logits live in the graph's output buffer until the next step.  A token
+        outside the vocabulary gives its sequence NaN logits and rows (``FlashLoopEngine.decode``)."""
         st = self.state
         bsz = len(st.positions)
         if tuple(token_ids.shape) != (bsz, 1):

@@ -5,8 +5,8 @@ Mirrors ``FlashLoopEngine`` (flashloop/engine.py:112-607): ``from_pretrained``,
 on this build's HIP kernels:
 
 * token-sparse prefill loops 3/4 -- row scores (``fl_hidden_delta_score``), nested global
-  top-k selection with the forced last token (``fl_select_tokens``) and row gather /
-  scatter of hidden states and K/V (``fl_gather_rows`` / ``fl_scatter_rows``);
+  top-k selection with the forced last token (``fl_select_tokens_status``) and row gather /
+  scatter of hidden states and K/V (``fl_move_rows``; the K/V rows by ``fl_rope_store``);
 * the int4 anchor + residual cross-loop KV cache (``fl_pack_kv_groups``);
 * decode loops 1-2 dense over the packed cache (``fl_decode_attn_dense``), loop-2 key
   selection (``fl_decode_topk``), loops 3-4 cached-mass sparse attention
@@ -678,7 +678,9 @@ class FlashLoopEngine:
         """``FlashLoopEngine.decode`` (flashloop/engine.py:373-570).  With ``use_graphs`` the
         step replays a captured HIP graph (recaptured when the selection capacity changes
         its shapes); the returned logits then live in the runner's output buffer and are
-        overwritten by the next step."""
+        overwritten by the next step.  The fused step does not refuse a token outside the
+        vocabulary (that would need a synchronisation): its logits are NaN, and so are the
+        rows it appends."""
         state = self.state
         if token_ids.shape != (1, 1):
             raise ValueError("decode requires exactly one token at batch size one")

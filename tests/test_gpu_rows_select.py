@@ -6,7 +6,7 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-from flashloop_amd import kernels  # noqa: E402
+from flashloop_amd import _lib, kernels  # noqa: E402
 from oracle import tokens as OT  # noqa: E402
 
 DEV = "cuda"
@@ -33,6 +33,53 @@ def test_rows_move_and_flag(outer, rows, width, n):
         assert torch.equal(dst, src.index_copy(1, pos[:-1].long(), new[:, :-1])) and int(err) == 1
         _, err = kernels.gather_rows(src, wrong, 1)
         assert int(err) == 1
+
+
+@pytest.mark.parametrize("width,gap", [(2, 0), (6, 2), (128, 0), (200, 8), (4, 4)])
+def test_row_calls_that_only_set_the_flag(width, gap):
+    """fl_gather_rows and fl_scatter_rows through the C API, rows apart in 4- and 16-byte pieces:
+    a flag of the caller's is set by an index out of range and otherwise left as it was; none may
+    be given; no index moves nothing."""
+    print(f"case: row calls width={width} gap={gap}", flush=True)
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device=DEV).manual_seed(98)
+    outer, rows, n, pitch = 3, 500, 131, width + gap
+    rand = lambda *shape: torch.randint(0, 1 << 15, shape, generator=g, device=DEV).to(torch.int16)
+    full, new = rand(outer, rows, pitch), rand(outer, n, pitch)
+    pos = torch.randperm(rows, generator=g, device=DEV)[:n].int()
+    wrong = pos.clone()
+    wrong[7], wrong[100] = rows, -1
+    ok = torch.ones(n, dtype=torch.bool, device=DEV)
+    ok[7] = ok[100] = False
+
+    def gather(index, count, flag):
+        dst = new.clone()
+        _lib.check(lib.fl_gather_rows(full.data_ptr(), rows * pitch * 2, pitch * 2, rows, dst.data_ptr(), n * pitch * 2, pitch * 2,
+                                      outer, width * 2, index.data_ptr(), count, None if flag is None else flag.data_ptr(), stream),
+                   "fl_gather_rows")
+        return dst
+
+    def scatter(index, count, flag):
+        dst = full.clone()
+        _lib.check(lib.fl_scatter_rows(new.data_ptr(), n * pitch * 2, pitch * 2, dst.data_ptr(), rows * pitch * 2, pitch * 2, rows,
+                                       outer, width * 2, index.data_ptr(), count, None if flag is None else flag.data_ptr(), stream),
+                   "fl_scatter_rows")
+        return dst
+
+    for index, moved in ((pos, torch.ones_like(ok)), (wrong, ok)):
+        at = index[moved].long()
+        got = new.clone()
+        got[:, moved, :width] = full[:, at, :width]
+        put = full.clone()
+        put[:, at, :width] = new[:, moved, :width]
+        for held in (0, 5, None):
+            flag = None if held is None else torch.full((1,), held, dtype=torch.int32, device=DEV)
+            for call, want in ((gather, got), (scatter, put)):
+                assert torch.equal(call(index, n, flag), want)
+                if flag is not None:
+                    assert int(flag) == (held if bool(moved.all()) else 1)
+    flag = torch.full((1,), 5, dtype=torch.int32, device=DEV)
+    assert torch.equal(gather(wrong, 0, flag), new) and torch.equal(scatter(wrong, 0, flag), full) and int(flag) == 5
 
 
 def _scores(kind, b, t, gen):
