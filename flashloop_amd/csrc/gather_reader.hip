@@ -951,8 +951,12 @@ void launch_gather(GatherArgs& a, int rows, hipStream_t st) {
     hipLaunchKernelGGL(kernel, dim3(rows), dim3(kMergeThreads), 0, st, static_cast<const float*>(a.ws), a.waves, a.tpr,
                        rows, a.counts, a.cap, Lay<kLpt>::kTok, a.out, mode, a.mass, a.src, a.src_out);
   };
-  // a row's parts are the workgroups it touches: past 32 the wide merge (33 parts: 7.1 -> 6.4 us)
-  if (a.waves / kWaves / rows + 1 > kMergeSplit * kMergeLocal)
+  // A row's parts are the workgroups that its tiles touch, as gather_merge_row counts them; past 32 the
+  // wide merge.  Loop-4 reader and merge, us without it and with it: 8 rows of 9000 tokens (31 parts)
+  // 14.6 / 14.7, of 12,000 (39) 18.0 / 16.4, of 40,000 (64) 24.8 / 21.5; 16 rows of 12,000 (20 parts on
+  // 512 workgroups) 19.3 / 19.8, of 16,000 (27) 20.0 / 20.7, of 40,000 (33) 30.5 / 29.7
+  const int64_t chunk = (static_cast<int64_t>(rows) * a.tpr + a.waves - 1) / a.waves * kWaves;
+  if ((a.tpr + chunk - 1) / chunk + 1 > kMergeSplit * kMergeLocal)
     merge(gather_merge_wide_kernel);
   else
     merge(gather_merge_kernel);

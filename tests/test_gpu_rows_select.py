@@ -137,3 +137,39 @@ def test_hidden_score_at_the_wide_loads_line(dim):
     got = kernels.hidden_delta_score(a, b).double()
     want = (a.double() - b.double()).norm(dim=-1) / a.double().norm(dim=-1)
     assert bool(((got - want).abs() <= (dim + 8) * 2.0 ** -24 * want).all())
+
+
+@pytest.mark.parametrize("heads,tokens", [(16, 12000), (16, 20000), (8, 9000), (8, 12000)])
+def test_sparse_merges_on_both_sides_of_the_wide_line(heads, tokens):
+    """20, 33, 31 and 39 parts a row: each head alone (31 parts or more) gives the same loop-3 and
+    loop-4 deltas and source sum.  Bound: fp32 sums over k selected keys of weights that add up to
+    1, k * 2^-24 of the largest value each way, for the two sums of a delta."""
+    print(f"case: sparse merges heads={heads} tokens={tokens}", flush=True)
+    from flashloop_amd.cache import CrossLoopKVLayer
+    g = torch.Generator(device=DEV).manual_seed(99)
+    rand = lambda *shape: torch.randn(shape, generator=g, device=DEV).to(torch.bfloat16)
+    ks, vs = [rand(1, heads, tokens, 128) for _ in range(4)], [rand(1, heads, tokens, 128) for _ in range(4)]
+    q, k, v, v1 = (rand(1, heads, 1, 128) for _ in range(4))
+
+    def deltas(rows, chosen):
+        lc = CrossLoopKVLayer.from_prefill([x[:, rows] for x in ks], [x[:, rows] for x in vs])
+        at = lambda x: x[:, rows].contiguous()
+        if chosen is None:
+            _, _, chosen = lc.dense_source_attention_select(1, query=q, current_key=k, current_value=v1, scaling=0.088,
+                                                            fraction=0.1)
+        else:
+            idx, valid, mass, w, cnt = chosen
+            chosen = (at(idx), at(valid), at(mass), at(w), cnt.view(1, -1)[:, rows].flatten().contiguous())
+        idx, valid, mass, w, cnt = chosen
+        common = dict(query=at(q), current_key=at(k), current_value=at(v), indices=idx, valid=valid, global_mass=mass,
+                      scaling=0.088, counts=cnt)
+        d3, so = lc.cached_mass_sparse_attention_delta_with_source(2, source_weights=w, source_current_value=at(v1), **common)
+        d4 = lc.cached_mass_sparse_attention_delta(3, source_selected_output=so, **common)
+        return chosen, (d3, so, d4)
+
+    chosen, together = deltas(slice(0, heads), None)
+    bound = 4 * int(chosen[4].max()) * 2.0 ** -24 * max(float(x.abs().max()) for x in vs)
+    for h in range(0, heads, 5):
+        _, alone = deltas(slice(h, h + 1), chosen)
+        for a, b in zip(together, alone):
+            assert float((a.view(heads, 128)[h] - b.view(128)).abs().max()) <= bound
