@@ -16,9 +16,10 @@
 // no longer exactly 1 in bf16: error against 64 bits 2.05e-3 instead of 2.00e-3 at 2048 keys.)
 //
 // Bound by the matrix cores, the softmax's VALU work (quarter-rate exp) and the LDS reads at
-// about the same rate each, so two workgroups share a CU (202 VGPRs, 76 KB of LDS).  Measured,
-// 16 heads, 8192 dense queries: 340-355 us, 775-810 TFLOP/s of the causal half (the SDPA it
-// replaces: 740 us); 2048 of 8192: 490 -> 116 us; 820 of 8192: 940 -> 65 us.
+// about the same rate each, so two workgroups share a CU (76 KB of LDS).  Measured, 16 heads, 8192
+// dense queries: 338-370 us back to back (745-815 TFLOP/s of the causal half), 380 among the other
+// kernels of a prompt (725); the SDPA it replaces: 725-740 us.  2048 of 8192: 118 us, 2000 937 -> 133;
+// 820 of 8192: 940 -> 72 us.
 #include <algorithm>
 #include <cfloat>
 
@@ -63,8 +64,10 @@ __device__ __forceinline__ uint32_t attn_bf16_pair(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2_t));
 }
 
-// acc + both values of a packed bf16 pair (v_dot2_f32_bf16 with ones): the sum of the
-// probabilities as the second product sees them, in half the instructions
+// acc + both values of a packed bf16 pair (v_dot2_f32_bf16 with ones): the fp32 sum of the
+// probabilities as the second product sees them, so that their roundings cancel in the quotient.
+// The sum of the unrounded ones is 1-3% faster and errs more: against 64 bits 2.00e-3 instead of
+// 1.99e-3 at 2048 dense queries, 2.03e-3 and 2.02e-3 at 8192 (the SDPA: 2.03e-3 and 2.08e-3).
 __device__ __forceinline__ float add_pair(uint32_t w, float acc) {
   const bf16x2_t one = {static_cast<__bf16>(1.0f), static_cast<__bf16>(1.0f)};
   return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, w), one, acc, false);

@@ -980,7 +980,10 @@ int32_t dense_launch(const fl_cache_view& v, int32_t loop, const uint16_t* q, co
   if (waves) *waves = a.waves;
   if (!merge) return FL_OK;
   // long rows of many parts take the wide merge: 16 rows of 70,000 tokens, loops 1 and 2 (128 and
-  // 64 parts) 9.4 -> 6.8 us a merge; at 8192 tokens (66 parts) it loses, 6.0 -> 6.8
+  // 64 parts) 9.4 -> 6.8 us a merge; at 8192 tokens (66 parts) a merge alone loses, 6.0 -> 6.8.  Reader
+  // and merge, us without it and with it: at the line (16 rows of 32,700 tokens) loop 1 24.1 / 24.0,
+  // loop 2 34.1 / 34.8; past it, at 34,000, 27.5 / 25.7 and 37.6 / 35.4, at 40,000 30.2 / 27.3 and
+  // 38.7 / 40.0; below it the sign goes by length and loop (16,000: 20.1 / 17.3 and 23.2 / 26.2)
   const int rows = v.batch * v.heads;
   const bool wide = a.waves / rows > kMergeSplit * kMergeLocal && v.max_packed_tokens >= 32768;
   const float* p = a.ws;

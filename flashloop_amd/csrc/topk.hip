@@ -1679,7 +1679,8 @@ int32_t launch_select_merge(const fl_cache_view& v, const float* ws, int W, floa
   const int rows = v.batch * v.heads;
   const int per = static_cast<int>((logits_stride + kTopkThreads - 1) / kTopkThreads);
   const dim3 grid(2 * rows), block(kTopkThreads);
-  // rows of up to 4096 keys: 9.7 -> 8.6 us at 16 rows of 2049 (8 and 16 keys a thread gained nothing)
+  // rows of up to 4096 keys: 9.7 -> 8.6 us at 16 rows of 2049, with their read 16.6 -> 15.8 (8 and 16
+  // keys a thread gained nothing)
   if (per <= 4)
     hipLaunchKernelGGL(select_merge_kernel<4>, grid, block, 0, st, A, v, ws, W, out);
   else if (per <= 12)
