@@ -7,6 +7,8 @@
 //
 // fl_hidden_delta_score is _hidden_delta_score (flashloop/engine.py:78-81), one wave
 // per row.
+#include <algorithm>
+
 #include "fl_common.h"
 
 namespace fl {
@@ -39,7 +41,7 @@ __global__ __launch_bounds__(256) void move_rows_kernel(const uint8_t* src, int6
   }
   const int64_t item = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   if (item >= items) return;
-  const int64_t i = item <= 0xFFFFFFFFll ? static_cast<uint32_t>(item) / row_vecs : item / row_vecs;
+  const int64_t i = static_cast<uint32_t>(item) / row_vecs;
   const int64_t e = item - i * row_vecs;
   const int64_t o = blockIdx.y;
   const int32_t t = index[i];
@@ -71,19 +73,28 @@ int32_t launch_move(const void* src, int64_t s_outer, int64_t s_row, void* dst, 
   const bool empty = outer == 0 || n_index == 0 || row_bytes == 0;
   if (empty && !OWN) return FL_OK;
   const int64_t vecs = empty ? 1 : (vec16 ? row_bytes / 16 : row_bytes / 4);
-  const int64_t items = empty ? 0 : vecs * n_index;
-  const int64_t blocks = empty ? 1 : (items + 255) / 256;
-  FL_REQUIRE(vecs <= 0xFFFFFFFFll && blocks <= 0x7FFFFFFFll, std::string(who) + ": rows too large");
-  const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(empty ? 1 : outer));
+  constexpr int64_t kMaxItems = 0xFFFFFFFFll / 256 * 256;  // threads of a launch
+  FL_REQUIRE(vecs <= kMaxItems, std::string(who) + ": rows too large");
   hipStream_t st = static_cast<hipStream_t>(stream);
   const uint8_t* s = static_cast<const uint8_t*>(src);
   uint8_t* d = static_cast<uint8_t*>(dst);
-  if (vec16)
-    hipLaunchKernelGGL((move_rows_kernel<uint4, SCATTER, OWN>), grid, dim3(256), 0, st, s, s_outer, s_row, d, d_outer,
-                       d_row, rows, static_cast<uint32_t>(vecs), items, index, n_index, err);
-  else
-    hipLaunchKernelGGL((move_rows_kernel<uint32_t, SCATTER, OWN>), grid, dim3(256), 0, st, s, s_outer, s_row, d, d_outer,
-                       d_row, rows, static_cast<uint32_t>(vecs), items, index, n_index, err);
+  // one launch up to 2^32 pieces of an outer index; of several, the first writes the flag for all
+  const int64_t step = empty ? 1 : kMaxItems / vecs;
+  int64_t i0 = 0;
+  do {
+    const int64_t items = empty ? 0 : vecs * std::min(step, n_index - i0);
+    const dim3 grid(static_cast<unsigned>(std::max<int64_t>(1, (items + 255) / 256)), static_cast<unsigned>(empty ? 1 : outer));
+    const auto go = [&](auto kernel, int32_t* flag) {
+      hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, s + (SCATTER ? i0 * s_row : 0), s_outer, s_row,
+                         d + (SCATTER ? 0 : i0 * d_row), d_outer, d_row, rows, static_cast<uint32_t>(vecs), items, index + i0,
+                         n_index - i0, flag);
+    };
+    if (OWN && i0 > 0)
+      vec16 ? go(move_rows_kernel<uint4, SCATTER, false>, nullptr) : go(move_rows_kernel<uint32_t, SCATTER, false>, nullptr);
+    else
+      vec16 ? go(move_rows_kernel<uint4, SCATTER, OWN>, err) : go(move_rows_kernel<uint32_t, SCATTER, OWN>, err);
+    i0 += step;
+  } while (!empty && i0 < n_index);
   FL_LAUNCH_CHECK(who);
   return FL_OK;
 }

@@ -82,6 +82,27 @@ def test_row_calls_that_only_set_the_flag(width, gap):
     assert torch.equal(gather(wrong, 0, flag), new) and torch.equal(scatter(wrong, 0, flag), full) and int(flag) == 5
 
 
+def test_rows_past_a_launch():
+    """More than 2^32 pieces of 4 bytes (17 GB): the rows of both launches, and the flag, which an
+    index of the second one sets."""
+    print("case: rows past a launch", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(94)
+    width, rows = 2 * 1025, 1000
+    n = 2 ** 32 // 1025 + 3000
+    src = torch.randint(0, 1 << 15, (1, rows, width), generator=g, device=DEV).to(torch.int16)
+    pos = torch.randint(0, rows, (n,), generator=g, device=DEV).int()
+    got, err = kernels.gather_rows(src, pos, 1)
+    assert int(err) == 0
+    some = torch.cat((torch.arange(5, device=DEV), torch.arange(n - 6000, n, device=DEV)))
+    assert torch.equal(got[0, some], src[0, pos[some].long()])
+    back = torch.zeros_like(src)
+    pos.fill_(-1)  # (no two alike: the last 1000 rows go to places of their own)
+    pos[-rows:] = torch.randperm(rows, generator=g, device=DEV).int()
+    pos[0] = rows
+    _, err = kernels.scatter_rows_(back, pos, got, 1)
+    assert int(err) == 1 and torch.equal(back[0, pos[-rows:].long()], got[0, -rows:])
+
+
 def _scores(kind, b, t, gen):
     x = torch.randn(b, t, generator=gen, device=DEV)
     if kind == "tied":
