@@ -360,7 +360,7 @@ extern "C" int32_t fl_prefill_attention(const uint16_t* q, int64_t q_head_stride
     FL_REQUIRE(reinterpret_cast<uintptr_t>(p) % 16 == 0, "fl_prefill_attention: every tensor must be 16-byte aligned");
   if (queries == 0) return FL_OK;
   const int64_t blocks = (static_cast<int64_t>(queries) + kQueries - 1) / kQueries;
-  FL_REQUIRE(blocks * heads <= 0x7FFFFFFF / 16, "fl_prefill_attention: grid too large");
+  FL_REQUIRE(blocks * heads <= 0xFFFFFFFFll / kAttnThreads, "fl_prefill_attention: grid too large");
   AttnArgs a{q, k, v, out, positions, q_head_stride, q_row_stride, k_head_stride, k_row_stride,
              v_head_stride, v_row_stride, out_head_stride, out_row_stride, queries, keys, heads,
              scaling * kLog2e, attention_splits(heads, queries, keys), nullptr, nullptr};

@@ -21,7 +21,7 @@ namespace {
 
 constexpr int kBuildThreads = 512;
 constexpr int kBuildWaves = kBuildThreads / kWave;
-constexpr int kMaxSeqs = 64;      // sequences of one launch (their lengths travel as arguments)
+constexpr int kMaxSeqs = 64;      // most sequences of one launch (their lengths travel as arguments)
 constexpr int kScanPer = 16;      // tokens per thread and scan step
 constexpr int kClearBytes = 32768;  // per workgroup
 constexpr int kRegions = 21;
@@ -367,23 +367,34 @@ extern "C" int32_t fl_cache_prepare(const fl_cache_view* view, const uint16_t* c
       FL_REQUIRE(late[s * v.batch + b] >= 0 && late[s * v.batch + b] <= v.row_capacity[2 + s],
                  "fl_cache_prepare: late rows exceed the row capacity");
   }
-  for (int b0 = 0; b0 < v.batch; b0 += kMaxSeqs) {
+  // workgroups of a launch over sequences b0 .. b0 + seqs - 1
+  const auto plan = [&](int b0, int seqs) {
+    int64_t unused = 0;  // the most bytes a (b,h) row of a region has to clear
+    for (int i = 0; i < seqs; ++i)
+      for (const Region& r : a.region) {
+        const int used = r.kind == 0 ? packed[b0 + i]
+                                     : (r.kind == 1 ? packed[b0 + i] / kGroup : late[(r.kind - 2) * v.batch + b0 + i]);
+        unused = std::max(unused, r.row - static_cast<int64_t>(used) * r.unit);
+      }
+    const int64_t rows = static_cast<int64_t>(seqs) * v.heads;
+    a.clear_chunks = static_cast<int>(std::max<int64_t>(1, (unused + kClearBytes - 1) / kClearBytes));
+    return 3 * seqs + 8 * rows + (unused > 0 ? kRegions * rows * a.clear_chunks : 0);
+  };
+  constexpr int64_t kMaxBlocks = 0xFFFFFFFFll / kBuildThreads;  // 2^32 threads of a launch, past which it wraps
+  for (int b0 = 0; b0 < v.batch; b0 += a.seqs) {
     a.b0 = b0;
     a.seqs = std::min(kMaxSeqs, v.batch - b0);
-    int64_t unused = 0;  // the most bytes a (b,h) row of a region has to clear
+    int64_t blocks = plan(b0, a.seqs);
+    while (blocks > kMaxBlocks && a.seqs > 1) {
+      a.seqs = (a.seqs + 1) / 2;
+      blocks = plan(b0, a.seqs);
+    }
+    FL_REQUIRE(blocks <= kMaxBlocks, "fl_cache_prepare: grid too large");
     for (int i = 0; i < a.seqs; ++i) {
       a.len.packed[i] = packed[b0 + i];
       a.len.tail[i] = tail[b0 + i];
       for (int s = 0; s < 2; ++s) a.len.late[s][i] = late[s * v.batch + b0 + i];
-      for (const Region& r : a.region) {
-        const int used = r.kind == 0 ? packed[b0 + i] : (r.kind == 1 ? packed[b0 + i] / kGroup : a.len.late[r.kind - 2][i]);
-        unused = std::max(unused, r.row - static_cast<int64_t>(used) * r.unit);
-      }
     }
-    const int64_t rows = static_cast<int64_t>(a.seqs) * v.heads;
-    a.clear_chunks = static_cast<int>(std::max<int64_t>(1, (unused + kClearBytes - 1) / kClearBytes));
-    const int64_t blocks = 3 * a.seqs + 8 * rows + (unused > 0 ? kRegions * rows * a.clear_chunks : 0);
-    FL_REQUIRE(blocks <= 0x7FFFFFFF, "fl_cache_prepare: grid too large");
     hipLaunchKernelGGL(cache_prepare_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kBuildThreads), 0,
                        static_cast<hipStream_t>(stream), a);
     FL_LAUNCH_CHECK("fl_cache_prepare");

@@ -145,7 +145,7 @@ extern "C" int32_t fl_rope_store(const uint16_t* q, const uint16_t* k, const uin
     FL_REQUIRE(aligned16(p), "fl_rope_store: every tensor must be 16-byte aligned");
   if (n == 0) return FL_OK;
   const int64_t blocks = (static_cast<int64_t>(n) * heads * 8 + 255) / 256;
-  FL_REQUIRE(blocks <= 0x7FFFFFFF, "fl_rope_store: grid too large");
+  FL_REQUIRE(blocks <= 0xFFFFFFFFll / 256, "fl_rope_store: grid too large");
   const RopeStoreArgs a{{q, k, v}, row_stride, q_out, {k_dst, v_dst}, dst_head_stride, rope_cos, rope_sin, positions,
                         n, heads, rows};
   hipLaunchKernelGGL(rope_store_kernel, dim3(static_cast<unsigned>(blocks), 3), dim3(256), 0,
@@ -162,7 +162,7 @@ extern "C" int32_t fl_swiglu(const uint16_t* gate, const uint16_t* up, uint16_t*
   FL_REQUIRE(aligned16(gate) && aligned16(up) && aligned16(out), "fl_swiglu: every tensor must be 16-byte aligned");
   if (count == 0) return FL_OK;
   const int64_t blocks = (count / 8 + 255) / 256;
-  FL_REQUIRE(blocks <= 0x7FFFFFFF, "fl_swiglu: grid too large");
+  FL_REQUIRE(blocks <= 0xFFFFFFFFll / 256, "fl_swiglu: grid too large");
   hipLaunchKernelGGL(swiglu_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, static_cast<hipStream_t>(stream),
                      gate, up, out, count / 8);
   FL_LAUNCH_CHECK("fl_swiglu");

@@ -185,3 +185,31 @@ def test_short_prompts_of_misaligned_rows(t):
     for r in range(4):
         assert torch.equal(layer.tail_key[r].view(2, 3, -1, 128)[:, :, :t], off[r])
         assert torch.equal(layer.tail_value[r].view(2, 3, -1, 128)[:, :, :t], off[4 + r])
+
+
+def test_capacity_past_a_launch_is_cleared():
+    """64 sequences of 16 heads with room for 131,072 tokens (103 GB): the clears are more than a
+    launch's 2^32 threads."""
+    print("case: capacity past a launch", flush=True)
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 180 << 30:
+        pytest.skip("needs 180 GB of free device memory")
+    g = torch.Generator(device=DEV).manual_seed(95)
+    b, h, t = 64, 16, 130
+    ks = _kv(g, b, h, t)
+    junk = [torch.full((n << 30,), 0xA5, dtype=torch.uint8, device=DEV) for n in [16] * 4 + [8] + [2] * 14]
+    del junk  # (freed memory is not zero)
+    layer = CrossLoopKVLayer.from_prefill(ks, ks, token_capacity=131072)
+    assert layer.packed_tokens.tolist() == [64] * b and layer.tail_tokens.tolist() == [t - 64] * b
+    for s in range(4):
+        for x in (layer.codes[s][:, 64:], layer.value_meta[s][:, 64:], layer.value_meta_half[s][:, 64:], layer.key_meta[s][:, 1:],
+                  layer.key_meta_half[s][:, 1:]):
+            for row in x.reshape(x.shape[0], -1).split(64):  # (a copy of a sixteenth at a time)
+                assert not bool(row.view(torch.int64).any())
+    assert not bool(layer.value_meta_token[:, 64:].any())
+    for r in layer.rank:
+        assert torch.equal(r[:, :64], torch.arange(64, device=DEV, dtype=torch.int32).expand(b, 64)) and bool((r[:, 64:] == -1).all())
+    for got, want in zip((*layer.tail_key, *layer.tail_value), (*ks, *ks)):
+        assert torch.equal(got[:, : t - 64], want.view(b * h, t, 128)[:, 64:]) and not bool(got[:, t - 64:].any())
+    del layer, got, r, x, row
+    torch.cuda.empty_cache()
