@@ -37,13 +37,23 @@ from .model import MLP, Attention, OuroConfig, OuroForCausalLM, RMSNorm, RotaryE
 _FORWARD = {kind: kind.forward for kind in (torch.nn.Linear, torch.nn.Embedding, RMSNorm, RotaryEmbedding, MLP)}
 
 
+def _calls_are_plain() -> bool:
+    """Whether these classes still have the ``forward`` they were defined with, and no hook is on
+    every module."""
+    every = torch.nn.modules.module
+    return (not (every._global_forward_hooks or every._global_forward_pre_hooks)
+            and all(kind.forward is f for kind, f in _FORWARD.items()))
+
+
+def _is_bare(m: torch.nn.Module, kind: type) -> bool:
+    """Whether ``m`` is of ``kind`` itself, with no ``forward`` replaced on the instance and no hook."""
+    return type(m) is kind and "forward" not in m.__dict__ and not (m._forward_hooks or m._forward_pre_hooks)
+
+
 def _is_plain(m: torch.nn.Module, kind: type) -> bool:
     """Whether calling ``m`` runs the ``forward`` that ``kind`` was defined with and nothing else: no
     subclass, no ``forward`` replaced on the instance or the class, no hook on it or on every module."""
-    every = torch.nn.modules.module
-    return (type(m) is kind and getattr(m.forward, "__func__", None) is _FORWARD[kind]
-            and not (m._forward_hooks or m._forward_pre_hooks
-                     or every._global_forward_hooks or every._global_forward_pre_hooks))
+    return _is_bare(m, kind) and _calls_are_plain()
 
 
 @dataclass(frozen=True)
@@ -279,14 +289,28 @@ class FlashLoopEngine:
         is not a plain bf16 ``nn.Linear`` / ``RMSNorm`` on the device (a wrapped, replaced or
         hooked module keeps the module path, which calls it), or when the embedding or the
         rotary module (called on both paths) gave rows in another layout than the kernels read."""
-        def plain(m, kind) -> bool:
-            return (_is_plain(m, kind) and getattr(m, "bias", None) is None and m.weight.dtype == torch.bfloat16
-                    and m.weight.is_cuda and m.weight.is_contiguous())
+        # (host time that the GPU waits for after each loop boundary's read-back: what holds for every
+        # module is looked at once, and children and weights are taken from the modules' own tables)
+        if not _calls_are_plain():
+            return None
+
+        def weight(m, kind):
+            """The weight that calling ``m`` multiplies by, if ``m`` is plain and has no bias."""
+            if not _is_bare(m, kind):
+                return None
+            w = m._parameters.get("weight")
+            ok = (w is not None and w.dtype == torch.bfloat16 and w.is_cuda and w.is_contiguous()
+                  and m._parameters.get("bias") is None and "bias" not in m.__dict__)
+            return w if ok else None
+
+        def norm(m):
+            w = weight(m, RMSNorm)
+            return w if w is not None and w.data_ptr() % 16 == 0 else None  # (fl_norm_chain loads 16 bytes)
 
         d = hidden.shape[-1]
         final = self.backbone.norm
-        if hidden.dtype != torch.bfloat16 or d % 8 or d > 8192 or not plain(final, RMSNorm) or final.weight.data_ptr() % 16:
-            return None  # (fl_norm_chain loads 16 bytes of up to 8192 values)
+        if hidden.dtype != torch.bfloat16 or d % 8 or d > 8192 or norm(final) is None:  # (... of up to 8192 values)
+            return None
         table = (1, hidden.shape[1], self.layers[0].self_attn.head_dim)
         if (any(not x.is_contiguous() or x.data_ptr() % 16 for x in (hidden, cos, sin))
                 or any(tuple(x.shape) != table or x.dtype != torch.bfloat16 or not x.is_cuda for x in (cos, sin))):
@@ -295,15 +319,17 @@ class FlashLoopEngine:
         layers = []
         for layer in self.layers:
             a, m = layer.self_attn, layer.mlp
-            lin = (a.q_proj, a.k_proj, a.v_proj, a.o_proj, m.gate_proj, m.up_proj, m.down_proj)
+            if type(a) is not Attention or not _is_bare(m, MLP):
+                return None
             norms = (layer.input_layernorm, layer.input_layernorm_2, layer.post_attention_layernorm,
                      layer.post_attention_layernorm_2)
-            if (type(a) is not Attention or not _is_plain(m, MLP) or m.gate_proj.weight.shape[0] % 8
-                    or not all(plain(x, torch.nn.Linear) for x in lin)
-                    or not all(plain(x, RMSNorm) and x.weight.data_ptr() % 16 == 0 for x in norms)):
+            w = (*(weight(a._modules.get(n), torch.nn.Linear) for n in ("q_proj", "k_proj", "v_proj", "o_proj")),
+                 *(weight(m._modules.get(n), torch.nn.Linear) for n in ("gate_proj", "up_proj", "down_proj")),
+                 *(norm(x) for x in norms))
+            if any(x is None for x in w) or w[4].shape[0] % 8:
                 return None
             eps.update(x.eps for x in norms)
-            layers.append(tuple(x.weight for x in (*lin, *norms)))
+            layers.append(w)
         return (layers, float(eps.pop())) if len(eps) == 1 else None
 
     def _layer_rows(self, weights, hid, z, rope, kv, positions, eps, w_next, w_final):
